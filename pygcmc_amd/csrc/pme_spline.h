@@ -7,19 +7,33 @@
 
 namespace gcmc_spline {
 
-// weights of the 4 grid points f, f-1, f-2, f-3 of scaled coordinate u in [0, K)
-__device__ inline void spline4(float u, int K, int &f, float w[4])
+// weights at fractional offset t in [0, 1) of the 4 grid points f, f-1, f-2, f-3
+__device__ inline void weights4(float t, float w[4])
 {
-    const float fl = floorf(u);
-    f = (int)fl;
-    const float t = u - fl;  // [0, 1)
     const float t2 = t * t, t3 = t2 * t;
     const float s = 1.0f - t;
     w[0] = t3 * (1.0f / 6.0f);                                         // M4(t)
     w[1] = (-3.0f * t3 + 3.0f * t2 + 3.0f * t + 1.0f) * (1.0f / 6.0f);  // M4(t+1)
     w[2] = (3.0f * t3 - 6.0f * t2 + 4.0f) * (1.0f / 6.0f);              // M4(t+2)
     w[3] = s * s * s * (1.0f / 6.0f);                                   // M4(t+3)
-    f = ((f % K) + K) % K;
+}
+
+// grid point f = floor(u) and offset t = u - f of a scaled coordinate u in
+// [0, K) (scaled() below; a NaN gives point 0): no integer remainder, which
+// costs more than the weights
+__device__ inline int base4(float u, float &t)
+{
+    const float fl = floorf(u);
+    t = u - fl;
+    return fl > 0.0f ? (int)fl : 0;
+}
+
+// weights of the 4 grid points f, f-1, f-2, f-3 of scaled coordinate u in [0, K)
+__device__ inline void spline4(float u, int, int &f, float w[4])
+{
+    float t;
+    f = base4(u, t);
+    weights4(t, w);
 }
 
 // scaled coordinate K * frac(x / L) in [0, K)

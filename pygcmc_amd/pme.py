@@ -73,7 +73,7 @@ class PME:
     def solve(self):
         """Reciprocal energy of the charge grid (kJ/mol, float64 GPU tensor);
         also prepares the potential for gather."""
-        e = torch.zeros(1, dtype=torch.float64, device='cuda')
+        e = torch.empty(1, dtype=torch.float64, device='cuda')
         _engine._check(_lib().gcmc_pme_solve(self._h, ctypes.c_void_p(e.data_ptr()), _stream()))
         return e
 

@@ -87,3 +87,61 @@ def test_pme_slab_config_grid():
     ref = ewald.recip_energy(xyz, q, L, 0.34, kmax=(60, 60, 48))
     assert abs(e - ref) <= 1e-3 * abs(ref)
     p.close()
+
+
+def _spme64(xyzq, K, L, beta):
+    """Potential of smooth PME at the charges themselves, in FP64."""
+    K = np.array(K)
+    u = np.mod(xyzq[:, :3].astype(np.float64) / L, 1.0) * K
+    f = np.floor(u).astype(np.int64) % K
+    t = u - np.floor(u)
+    w = np.stack([t ** 3 / 6, (-3 * t ** 3 + 3 * t ** 2 + 3 * t + 1) / 6, (3 * t ** 3 - 6 * t ** 2 + 4) / 6,
+                  (1 - t) ** 3 / 6])
+    pts = [(tuple((f[:, d] - j[d]) % K[d] for d in range(3)), w[j[0], :, 0] * w[j[1], :, 1] * w[j[2], :, 2])
+           for j in np.ndindex(4, 4, 4)]
+    Q = np.zeros(K)
+    for k, v in pts:
+        np.add.at(Q, k, v * xyzq[:, 3])
+    B, m = [], []
+    for d in range(3):
+        i = np.arange(K[d])
+        z = sum(a * np.exp(2j * np.pi * i * n / K[d]) for n, a in enumerate((1 / 6, 2 / 3, 1 / 6)))
+        B.append(1.0 / np.abs(z) ** 2)
+        m.append(np.where(i <= K[d] // 2, i, i - K[d]) / L[d])
+    m2 = m[0][:, None, None] ** 2 + m[1][None, :, None] ** 2 + m[2][None, None, :] ** 2
+    m2[0, 0, 0] = 1.0
+    G = 1388.431112 / (np.pi * np.prod(L)) * np.exp(-np.pi ** 2 * m2 / beta ** 2) / m2
+    G *= B[0][:, None, None] * B[1][None, :, None] * B[2][None, None, :]
+    G[0, 0, 0] = 0.0
+    phi = np.fft.ifftn(G * np.fft.fftn(Q)).real * Q.size
+    return sum(phi[k] * v for k, v in pts)
+
+
+@pytest.mark.parametrize('K', [(4, 5, 4), (8, 8, 16), (9, 17, 18), (10, 25, 34), (31, 33, 50)])
+@pytest.mark.parametrize('n', [16383, 16384, 40001])
+def test_pme_spread_of_many_charges(K, n):
+    """Charges sorted by grid tile (one call) give the same charge grid, bit
+    for bit, as added a few at a time, and the FP64 potential: tiles cut by
+    the box, last tiles of one or two points, an axis of one tile, more charges
+    than are sorted at once, zero charges, positions outside the box.
+    Tolerance: FP32 weights, transforms and sums of n charges, 2e-5 of the
+    largest potential."""
+    rng = np.random.default_rng(n + K[0])
+    L = np.array([0.9 * k for k in K])
+    a = np.concatenate([(rng.random((n, 3)) * 3.0 - 1.0) * L, rng.normal(0, 0.3, (n, 1))], 1).astype(np.float32)
+    a[:, 3] -= a[:, 3].mean()
+    a[::97, 3] = 0.0
+    t = torch.tensor(a, device='cuda')
+    out = []
+    for step in (n, 5000):
+        p = PME(K, L, 0.34)
+        p.clear()
+        for i in range(0, n, step):
+            p.spread(t[i:i + step])
+        e = p.solve()
+        out.append((p.gather(t[:, :3].contiguous()).cpu().numpy(), float(e.item())))
+        p.close()
+    (phi, e), (phi1, e1) = out
+    assert np.array_equal(phi.view(np.uint32), phi1.view(np.uint32)) and e == e1
+    ref = _spme64(a, K, np.float32(L).astype(np.float64), float(np.float32(0.34)))
+    assert np.abs(phi - ref).max() <= 2e-5 * np.abs(ref).max()
