@@ -14,13 +14,13 @@
 // and the parameters the pair table was built from, the energy equals the
 // engine's trial energy.
 //
-// One workgroup per pose: the candidate scan is eval_energy's (cell list,
-// exact FP32 group test); the pair pass keeps per-fragment-atom gradient
-// sums in registers (one lane per environment atom, fragment atoms
-// unrolled), adds environment-type terms once per environment atom to LDS
-// accumulators, and writes, per pose, dE/dx [nf][3] and the per-type
-// derivatives [3][Y] (dq, eps, rmin).  FP32 arithmetic and accumulation;
-// the energy keeps the engine's compensated sum.
+// One wave per pose (four share one when there are few): the candidate scan is
+// the energy path's; the pair pass keeps per-fragment-atom gradient sums in
+// registers (one lane per environment atom, fragment atoms unrolled, ordered by
+// type so that a table entry and 1/sigma serve all atoms of a type), adds
+// environment-type terms once per environment atom to LDS accumulators, and
+// writes, per pose, dE/dx [nf][3] and the per-type derivatives [3][Y] (dq, eps,
+// rmin).  FP32 arithmetic; gradients accumulate in FP32, the energy in FP64.
 #pragma once
 
 #include "engine_kernels.h"
@@ -34,26 +34,30 @@ struct AdjLds {
     float4 *tab;    // [X*Y] (100 sigma^2 hi, 4 epsilon, 100 sigma^2 lo, 0) from the per-type parameters
     float *dq;      // [Y]
     float *inv2e;   // [Y] 1 / (2 |eps|), 0 where eps = 0
-    float *gq, *ge, *gr;  // [Y] per-type derivative sums of this pose
-    float *red;     // [6*MAXF] per-fragment-atom sums
+    float *gq, *ge, *gr;  // [Y] per-type derivative sums of this wave's pose
+    float *red;     // [6*MAXF] per-fragment-atom sums of a shared pose
 };
 
-__host__ __device__ inline int adj_lds_bytes(int X, int Y)
+// the tables, then per wave the type sums and the per-atom sums
+__host__ __device__ inline int adj_wave_bytes(int Y) { return (12 * Y + 4 * 6 * MAXF + 15) & ~15; }
+__host__ __device__ inline int adj_lds_bytes(int X, int Y, int nw)
 {
     auto up = [](int x) { return (x + 15) & ~15; };
-    return up(16 * X * Y) + 5 * up(4 * Y) + up(4 * 6 * MAXF);
+    return up(16 * X * Y) + 2 * up(4 * Y) + nw * adj_wave_bytes(Y);
 }
 
-__device__ inline AdjLds adj_carve(char *b, int X, int Y)
+// own: the wave whose sums these are (the team's first for a shared pose)
+__device__ inline AdjLds adj_carve(char *b, int X, int Y, int own)
 {
     auto up = [](int x) { return (x + 15) & ~15; };
     AdjLds A;
     A.tab = (float4 *)b; b += up(16 * X * Y);
     A.dq = (float *)b; b += up(4 * Y);
     A.inv2e = (float *)b; b += up(4 * Y);
-    A.gq = (float *)b; b += up(4 * Y);
-    A.ge = (float *)b; b += up(4 * Y);
-    A.gr = (float *)b; b += up(4 * Y);
+    b += own * adj_wave_bytes(Y);
+    A.gq = (float *)b; b += 4 * Y;
+    A.ge = (float *)b; b += 4 * Y;
+    A.gr = (float *)b; b += 4 * Y;
     A.red = (float *)b;
     return A;
 }
@@ -61,27 +65,56 @@ __device__ inline AdjLds adj_carve(char *b, int X, int Y)
 template <int NF>
 struct AdjPass {
     AdjLds A;
-    float gx[NF], gy[NF], gz[NF], sr[NF], se[NF], sq[NF];
+    int spi, nf;
+    double acc;
+    float gx[NF], gy[NF], gz[NF], sr[NF], se[NF], sq[NF];   // in the order of Species::slot
 
-    template <int NT, bool STAGED>
-    __device__ __attribute__((always_inline)) int run(CRep &C, const Lds &L, int n, int nf, float &acc,
-                                                      float &cmp, double &acc64)
+    __device__ __forceinline__ void run(CRep &C, const Lds &L, const WaveLds &W, int g, int At)
     {
-        const int At = wg_scan<NT>(L.incn, n, L.misc);
+        const int lane = threadIdx.x & 63;
+        CSpecies &F = species_of(C, spi);
+        const auto atom = gbl(C.atom);
+        const auto atype = gbl(C.atype);
+        const float4 *fs = (const float4 *)W.fragd;
         const float Lx = C.L[0], Ly = C.L[1], Lz = C.L[2];
         const float ix = C.invL[0], iy = C.invL[1], iz = C.invL[2];
-        for (int t = threadIdx.x; t < At; t += NT) {
-            const int g = bsearch_le(L.incn, n, t);
-            const int a = L.incs[g] + (t - L.incn[g]);
-            const float4 at = C.atom[a];
-            const int ty = C.atype[a];
+        const bool mapped = At <= WL_ATOMS;
+        int carry = 0;
+        float4 an;
+        int tn;
+        auto fetch = [&](int base) {
+            const int t = base + lane, tq = min(t, At - 1);
+            int slot;
+            if (mapped) {
+                slot = max(wave_scan_max(W.amap[t]), carry);
+                carry = __builtin_amdgcn_readlane(slot, 63);
+            } else {
+                slot = bsearch_off(W.goff, g, tq);
+            }
+            const int a = W.gdel[slot] + tq;
+            an = atom[a];
+            tn = atype[a];
+        };
+        fetch(0);
+        for (int base = 0; base < At; base += 64) {
+            const float4 at = an;
+            const int ty = tn;
+            if (base + 64 < At) fetch(base + 64);
+            if (base + lane >= At) continue;
             const float qa = at.w + A.dq[ty];
-            float tr = 0.f, te = 0.f, tq = 0.f;
+            float tr = 0.f, te = 0.f, tq = 0.f, isg = 0.f;
+            float4 pp = make_float4(0.f, 0.f, 0.f, 0.f);
+            int row = -1;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
                 if (f < nf) {
-                    const float4 fr = L.frag[f];
-                    const float4 pp = A.tab[L.frow[f] + ty];
+                    if (F.srow[f] != row) {
+                        row = F.srow[f];
+                        pp = A.tab[row + ty];
+                        // 1/sigma_pair = 10/sqrt(pp.x), nm^-1
+                        isg = pp.x > 0.0f ? 10.0f * __builtin_amdgcn_rsqf(pp.x) : 0.0f;
+                    }
+                    const float4 fr = fs[f];
                     float ex, ey, ez;
                     float dx = two_diff(at.x, fr.x, ex);
                     float dy = two_diff(at.y, fr.y, ey);
@@ -102,21 +135,15 @@ struct AdjPass {
                     const float s12 = s6 * s6;
                     const float lj = pp.y * (s12 - s6);
                     const float el = (fr.w * qa) * ir;
-                    const float term = lj + el;
-                    const float s = acc + term;
-                    const float bp = s - acc;
-                    const float err = (acc - (s - bp)) + (term - bp);
-                    acc = s;
-                    cmp += err;
+                    acc += (double)(lj + el);
                     // dE/d(r^2); with d = x_a - x_f, dE/dx_f = -2 dE/d(r^2) d
                     const float dr2 = (pp.y * fmaf(-6.0f, s12, 3.0f * s6) - 0.5f * el) * ir2;
                     const float gs = -2.0f * dr2;
                     gx[f] = fmaf(gs, dx + ex, gx[f]);
                     gy[f] = fmaf(gs, dy + ey, gy[f]);
                     gz[f] = fmaf(gs, dz + ez, gz[f]);
-                    // dE/dsigma_pair = 4 eps (12 s^12 - 6 s^6) / sigma_pair, 1/sigma = 10/sqrt(pp.x);
+                    // dE/dsigma_pair = 4 eps (12 s^12 - 6 s^6) / sigma_pair;
                     // dsigma_pair/drmin = 2^(5/6)/20 on each side
-                    const float isg = pp.x > 0.0f ? 10.0f * __builtin_amdgcn_rsqf(pp.x) : 0.0f;
                     const float ds = pp.y * fmaf(12.0f, s12, -6.0f * s6) * isg * (0.5f * SIGMA_PER_RMINHALF);
                     sr[f] += ds;
                     tr += ds;
@@ -132,33 +159,53 @@ struct AdjPass {
             atomicAdd(&A.ge[ty], te * A.inv2e[ty]);
             atomicAdd(&A.gq[ty], tq);
         }
-        __syncthreads();
-        return At;
     }
 };
 
+// sum over the wave, in every lane
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_add_f(float x)
+{
+    return x + __int_as_float(dpp_i<CTRL, ROWS>(0, __float_as_int(x)));
+}
+__device__ __forceinline__ float wave_sum_f(float x)
+{
+    x = dpp_add_f<DPP_SHR1, 0xf>(x);
+    x = dpp_add_f<DPP_SHR2, 0xf>(x);
+    x = dpp_add_f<DPP_SHR4, 0xf>(x);
+    x = dpp_add_f<DPP_SHR8, 0xf>(x);
+    x = dpp_add_f<DPP_BC15, 0xa>(x);
+    x = dpp_add_f<DPP_BC31, 0xc>(x);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
 // poses [npose][nf][3], centres [npose][3]; outputs E [npose] (FP64),
-// dEdx [npose][nf][3], partial [npose][3][Y] (dq, eps, rmin)
-template <int NT, int NF>
-__global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi, const float *centres,
+// dEdx [npose][nf][3], partial [npose][3][Y] (dq, eps, rmin).  PARTS waves share
+// a pose; every workgroup builds the pair table once and takes poses in turn.
+template <int NT, int NF, int PARTS>
+__global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi, int npose, const float *centres,
                                                const float *poses, const float *eps_kcal,
                                                const float *rmin_half, const float *dq, double *E,
                                                float *dEdx, float *partial, LdsLayout lay, int adj_off)
 {
     extern __shared__ __align__(16) char smem[];
+    constexpr int NW = NT / 64, PER = NW / PARTS;
     const Lds L = carve(smem, lay);
     CRep &C = rep_of(reps, r);
     const int X = C.X, Y = C.Y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform_i(tid >> 6), part = wave % PARTS;
+    const WaveLds W = wave_lds(L, wave);
     AdjPass<NF> P;
-    P.A = adj_carve(smem + adj_off, X, Y);
+    P.A = adj_carve(smem + adj_off, X, Y, wave - part);
     CSpecies &F = species_of(C, spi);
-    const int nf = F.nf, i = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int nf = F.nf;
+    P.spi = spi;
+    P.nf = nf;
     for (int t = tid; t < Y; t += NT) {
         const float ek = fabsf(eps_kcal[t]);
         P.A.inv2e[t] = ek > 0.0f ? 0.5f / ek : 0.0f;
         P.A.dq[t] = dq ? dq[t] : 0.0f;
     }
-    for (int q = tid; q < 6 * MAXF; q += NT) P.A.red[q] = 0.0f;
     load_species_table(C, L);
     // pair entries in FP64, rounded once to FP32 (as a host-built table is)
     for (int q = tid; q < X * Y; q += NT) {
@@ -169,62 +216,74 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         const float hi = (float)s2;
         P.A.tab[q] = make_float4(hi, (float)(4.0 * sqrt(ee)), (float)(s2 - (double)hi), 0.0f);
     }
-    if (tid < nf) {
-        const float *p = poses + ((size_t)i * nf + tid) * 3;
-        const float kq = dq ? KCOUL_F * (F.tmpl[tid].w + dq[F.ttype[tid]]) : F.kq[tid];
-        L.frag[tid] = make_float4(p[0], p[1], p[2], kq);
-        L.frow[tid] = F.trow[tid];
-    }
     __syncthreads();
-    for (int t = tid; t < Y; t += NT) {
-        P.A.gq[t] = 0.0f;
-        P.A.ge[t] = 0.0f;
-        P.A.gr[t] = 0.0f;
-    }
+    for (int i0 = blockIdx.x * PER; i0 < npose; i0 += gridDim.x * PER) {
+        const int i = i0 + wave / PARTS, q = min(i, npose - 1);
+        if (PARTS == 1 && i >= npose) break;
+        const float c[3] = {uniform_f(centres[3 * (size_t)q]), uniform_f(centres[3 * (size_t)q + 1]),
+                            uniform_f(centres[3 * (size_t)q + 2])};
+        if (lane < nf) {
+            const float *p = poses + ((size_t)q * nf + lane) * 3;
+            const float kq = dq ? KCOUL_F * (F.tmpl[lane].w + dq[F.ttype[lane]]) : F.kq[lane];
+            ((float4 *)W.fragd)[F.slot[lane]] = make_float4(p[0], p[1], p[2], kq);
+        }
+        if (part == 0)
+            for (int t = lane; t < 3 * Y + 6 * MAXF; t += 64) P.A.gq[t] = 0.0f;
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        P.gx[f] = P.gy[f] = P.gz[f] = 0.0f;
-        P.sr[f] = P.se[f] = P.sq[f] = 0.0f;
-    }
-    __syncthreads();
-    double e;
-    int n, na;
-    uint32_t h;
-    eval_energy_pass<NT, false>(C, centres[3 * i], centres[3 * i + 1], centres[3 * i + 2], nf, -1, L, P, &e, &n, &h,
-                                &na, nullptr);
+        for (int f = 0; f < NF; ++f) {
+            P.gx[f] = P.gy[f] = P.gz[f] = 0.0f;
+            P.sr[f] = P.se[f] = P.sq[f] = 0.0f;
+        }
+        P.acc = 0.0;
+        if (PARTS > 1) __syncthreads();
+        wave_sync();
+        ScanSums o{};
+        scan_groups(C, L, W, c, c, 1, -1, part, PARTS, P, o);
+        // lane f of the first wave: the sums of the atom in place f
+        float s[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        if (f < nf) {
-            float v[6] = {P.gx[f], P.gy[f], P.gz[f], P.sr[f], P.se[f], P.sq[f]};
+        for (int f = 0; f < NF; ++f) {
+            if (f < nf) {
+                const float v[6] = {P.gx[f], P.gy[f], P.gz[f], P.sr[f], P.se[f], P.sq[f]};
 #pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                float x = v[k];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-                if (lane == 0) atomicAdd(&P.A.red[6 * f + k], x);
+                for (int k = 0; k < 6; ++k) {
+                    const float x = wave_sum_f(v[k]);
+                    if (lane == f) s[k] = x;
+                }
             }
         }
+        PoseSums ps{};
+        ps.e[0] = lane_d(wave_scan_add(P.acc), 63);
+        if (PARTS > 1) {
+            if (lane < nf)
+                for (int k = 0; k < 6; ++k) atomicAdd(&P.A.red[6 * lane + k], s[k]);
+            team_sum<NT>(L, ps);
+            if (lane < nf)
+                for (int k = 0; k < 6; ++k) s[k] = P.A.red[6 * lane + k];
+        }
+        wave_sync();
+        if (part == 0 && i < npose) {
+            // the place's atom (Species::slot is the other way round)
+            if (lane < nf) {
+                int a = 0;
+                for (int b = 0; b < nf; ++b) a = F.slot[b] == lane ? b : a;
+                const int tf = F.ttype[a];
+                float *o = dEdx + ((size_t)i * nf + a) * 3;
+                o[0] = s[0];
+                o[1] = s[1];
+                o[2] = s[2];
+                atomicAdd(&P.A.gr[tf], s[3]);
+                atomicAdd(&P.A.ge[tf], s[4] * P.A.inv2e[tf]);
+                atomicAdd(&P.A.gq[tf], s[5] * KCOUL_F);
+            }
+            wave_sync();
+            float *pp = partial + (size_t)i * 3 * Y;
+            for (int t = lane; t < 3 * Y; t += 64) pp[t] = P.A.gq[t];
+            if (lane == 0) E[i] = ps.e[0];
+        }
+        wave_sync();
+        if (PARTS > 1) __syncthreads();
     }
-    __syncthreads();
-    if (tid < nf) {
-        const int tf = F.ttype[tid];
-        const float *rd = P.A.red + 6 * tid;
-        float *o = dEdx + ((size_t)i * nf + tid) * 3;
-        o[0] = rd[0];
-        o[1] = rd[1];
-        o[2] = rd[2];
-        atomicAdd(&P.A.gr[tf], rd[3]);
-        atomicAdd(&P.A.ge[tf], rd[4] * P.A.inv2e[tf]);
-        atomicAdd(&P.A.gq[tf], rd[5] * KCOUL_F);
-    }
-    __syncthreads();
-    float *pp = partial + (size_t)i * 3 * Y;
-    for (int t = tid; t < Y; t += NT) {
-        pp[t] = P.A.gq[t];
-        pp[Y + t] = P.A.ge[t];
-        pp[2 * Y + t] = P.A.gr[t];
-    }
-    if (tid == 0) E[i] = e;
 }
 
 // tmp[c][j] = sum over poses p of chunk c of w[p] partial[p][j] (FP64);

@@ -221,7 +221,7 @@ constexpr float STENCIL_EPS = 0.05f;  // A of slack over FP32 rounding of the gr
 
 void cell_geometry(const float cryst[3], float cell_size, int nc[3], float inv_h[3])
 {
-    const float h = cell_size > 0 ? cell_size : 5.0f;
+    const float h = cell_size > 0 ? cell_size : 6.5f;
     for (int i = 0; i < 3; ++i) {
         nc[i] = std::max(1, (int)std::floor(cryst[i] / h));
         nc[i] = std::min(nc[i], 255);
@@ -229,30 +229,40 @@ void cell_geometry(const float cryst[3], float cell_size, int nc[3], float inv_h
     }
 }
 
+// Reach of the stencil along axis i: r cells of edge h each way, when a centre
+// may lie up to ext past its home cell; `full`: it wraps onto itself, every
+// cell of the axis is listed once.
+bool stencil_reach(float L, int nc, float rc, float ext, int *r)
+{
+    *r = (int)std::floor((rc + STENCIL_EPS + ext) / ((double)L / nc)) + 1;
+    return 2 * *r + 1 >= nc;
+}
+
 // Trial-specific pruning of the stencil (stencil_cell_near): cell edges, the
 // axes whose stencil offsets are the minimum-image ones (the stencil does not
 // wrap onto itself there) and the squared reach rc + slack.
-void stencil_prune(const float L[3], const int nc[3], float rc, float h[3], int *prune, float *r2)
+void stencil_prune(const float L[3], const int nc[3], float rc, float ext, float h[3], int *prune, float *r2)
 {
     *prune = 0;
     for (int i = 0; i < 3; ++i) {
+        int r;
         h[i] = L[i] / (float)nc[i];
-        const int r = (int)std::floor((rc + STENCIL_EPS) / ((double)L[i] / nc[i])) + 1;
-        if (2 * r + 1 < nc[i]) *prune |= 1 << i;
+        if (!stencil_reach(L[i], nc[i], rc, ext, &r)) *prune |= 1 << i;
     }
     *r2 = (rc + STENCIL_EPS) * (rc + STENCIL_EPS);
 }
 
-// cell stencil: offsets whose cell box lies within rc + eps of the centre cell
-std::vector<int> make_stencil(const float L[3], const int nc[3], float rc, float eps)
+// cell stencil: offsets whose cell box lies within rc + slack of the centre's
+// cell, extended by ext towards positive offsets
+std::vector<int> make_stencil(const float L[3], const int nc[3], float rc, float ext)
 {
     int lo[3], hi[3];
     bool full[3];
     double h[3];
     for (int i = 0; i < 3; ++i) {
         h[i] = (double)L[i] / nc[i];
-        int r = (int)std::floor((rc + eps) / h[i]) + 1;
-        full[i] = (2 * r + 1 >= nc[i]);
+        int r;
+        full[i] = stencil_reach(L[i], nc[i], rc, ext, &r);
         if (full[i]) {
             lo[i] = -((nc[i] - 1) / 2);
             hi[i] = lo[i] + nc[i] - 1;
@@ -261,23 +271,31 @@ std::vector<int> make_stencil(const float L[3], const int nc[3], float rc, float
             hi[i] = r;
         }
     }
-    const double lim = (double)(rc + eps) * (rc + eps);
+    const double lim = (double)(rc + STENCIL_EPS) * (rc + STENCIL_EPS);
+    // gap between the home cell [0, h + ext] and the cell at offset n
+    auto gap = [&](int n, double hh) {
+        return std::max(0.0, n > 0 ? (n - 1) * hh - ext : (n < 0 ? (-n - 1) * hh : 0.0));
+    };
     std::vector<int> out;
     for (int a = lo[0]; a <= hi[0]; ++a)
         for (int b = lo[1]; b <= hi[1]; ++b)
             for (int c = lo[2]; c <= hi[2]; ++c) {
-                int d[3] = {a, b, c};
+                const int d[3] = {a, b, c};
                 double s = 0;
                 for (int i = 0; i < 3; ++i) {
-                    int n = std::abs(d[i]);
-                    if (full[i]) n = std::min(n, nc[i] - n);
-                    double g = std::max(0, n - 1) * h[i];
+                    double g = gap(d[i], h[i]);
+                    if (full[i]) g = std::min(g, gap(d[i] > 0 ? d[i] - nc[i] : d[i] + nc[i], h[i]));
                     s += g * g;
                 }
                 if (s <= lim) out.push_back((a + 128) | ((b + 128) << 8) | ((c + 128) << 16));
             }
     return out;
 }
+
+// Translations of at most this much (grid_dx, A) evaluate the old and the new
+// pose in one scan of a stencil wide enough for both centres; the wider ones
+// scan twice (the union of two distant neighbourhoods would be scanned for each).
+constexpr float WIDE_DX = 2.0f;
 
 template <class T>
 hipError_t put(T **dst, DevBuf &b, const T *src, size_t n)
@@ -307,6 +325,8 @@ int upload_rep(gcmc_engine *E, HostRep &H)
         R.L[i] = I.cryst[i];
         R.start[i] = I.startxyz[i];
         R.invL[i] = 1.0f / I.cryst[i];
+        R.Ld[i] = (double)R.L[i];
+        R.invLd[i] = (double)R.invL[i];
         R.ax[i].L = I.cryst[i];
         R.ax[i].t[0] = shift_threshold(I.cryst[i], 1);
         R.ax[i].t[1] = shift_threshold(I.cryst[i], 2);
@@ -381,13 +401,21 @@ int upload_rep(gcmc_engine *E, HostRep &H)
         atype[a] = A.type;
     }
     std::vector<float4> pair((size_t)R.X * R.Y);
+    const bool fp64_terms = R.coul64 && !(H.ew_beta > 0.0f);
     for (size_t i = 0; i < pair.size(); ++i) {
         // 100 sigma^2 as an unevaluated FP32 sum hi + lo (exact to ~2^-48);
         // 4 eps is exact in FP32
         const double sg = H.ff[2 * i], ep = H.ff[2 * i + 1];
         const double s2 = sg * sg * 100.0;
-        const float hi = (float)s2;
-        pair[i] = make_float4(hi, (float)(4.0 * ep), (float)(s2 - (double)hi), 0.0f);
+        const float hi = (float)s2, lo = (float)(s2 - (double)hi), e4 = (float)(4.0 * ep);
+        pair[i] = make_float4(hi, e4, lo, 0.0f);
+        if (fp64_terms) {
+            // 4 eps (S^6 r^-12 - S^3 r^-6) = (A r^-6 - B) r^-6
+            const double S = (double)hi + (double)lo, S3 = S * S * S;
+            const double AB[2] = {(double)e4 * S3 * S3, (double)e4 * S3};
+            static_assert(sizeof(AB) == sizeof(float4), "pair table entry");
+            std::memcpy(&pair[i], AB, sizeof(AB));
+        }
     }
     std::vector<Species> sp(T);
     for (int s = 0; s < T; ++s) {
@@ -410,6 +438,16 @@ int upload_rep(gcmc_engine *E, HostRep &H)
             S.ttype[a] = A.type;
             if (A.type < 0 || A.type >= R.X)
                 return fail(GCMC_E_ARG, "fragment atom type outside the pair table rows");
+        }
+        // atoms ordered by type, stably
+        int order[MAXF];
+        for (int a = 0; a < S.nf; ++a) order[a] = a;
+        std::stable_sort(order, order + S.nf, [&](int a, int b) { return S.ttype[a] < S.ttype[b]; });
+        for (int i = 0; i < S.nf; ++i) {
+            S.slot[order[i]] = i;
+            S.srow[i] = S.trow[order[i]];
+            if (i == 0 || S.ttype[order[i]] != S.ttype[order[i - 1]]) S.run_row[S.nrun++] = S.trow[order[i]];
+            S.run_end[S.nrun - 1] = i + 1;
         }
     }
     // Rep::nowrap.  An environment atom of an included group lies within
@@ -510,14 +548,20 @@ int upload_rep(gcmc_engine *E, HostRep &H)
             mrec[pos] = make_float4(r.position[0], r.position[1], r.position[2], w);
         }
     }
-    std::vector<int> st = make_stencil(R.L, R.nc, R.rc, STENCIL_EPS);
+    std::vector<int> st = make_stencil(R.L, R.nc, R.rc, 0.0f);
     R.nst = (int)st.size();
     // Per trial, a stencil cell whose box lies farther than rc + slack from
     // the trial centre holds no group that passes the group test: skipped.
     // Along an axis whose stencil offsets are the minimum-image ones (it does
     // not wrap onto itself) the box distance is measured from the centre's
     // position in its cell; other axes count no distance.
-    stencil_prune(R.L, R.nc, R.rc, R.cell_h, &R.prune, &R.prune_r2);
+    stencil_prune(R.L, R.nc, R.rc, 0.0f, R.cell_h, &R.prune, &R.prune_r2);
+    if (R.dx <= WIDE_DX) {
+        const std::vector<int> wide = make_stencil(R.L, R.nc, R.rc, R.dx);
+        R.nst_wide = (int)wide.size();
+        st.insert(st.end(), wide.begin(), wide.end());
+        stencil_prune(R.L, R.nc, R.rc, R.dx, R.cell_h, &R.prune_wide, &R.prune_r2);
+    }
 
     DevBuf &B = H.buf;
     HIPX(put((float **)&R.grid, B, H.grid.data(), H.grid.size()));
@@ -539,6 +583,7 @@ int upload_rep(gcmc_engine *E, HostRep &H)
             break;
         }
         if (P.rep.X == R.X && P.rep.Y == R.Y && P.pair.size() == pair.size() &&
+            (P.ew_beta > 0.0f) == (H.ew_beta > 0.0f) &&
             std::memcmp(P.pair.data(), pair.data(), pair.size() * sizeof(float4)) == 0) {
             R.tab = P.rep.tab;
             break;
@@ -603,48 +648,30 @@ int upload_rep(gcmc_engine *E, HostRep &H)
 int compute_layout(gcmc_engine *E)
 {
     // the pair table held in LDS: X x Y entries of the largest table
-    int nst = 1, xy = 1;
-    for (HostRep *H : E->reps) {
-        nst = std::max(nst, H->rep.nst);
-        xy = std::max(xy, H->rep.X * H->rep.Y);
-    }
+    int xy = 1;
+    for (HostRep *H : E->reps) xy = std::max(xy, H->rep.X * H->rep.Y);
     const int pair_bytes = 16 * xy;
     E->staged = E->tune.pair_lds >= 0 && pair_bytes <= 16384;
     auto up = [](int x) { return (x + 15) & ~15; };
     LdsLayout &l = E->lay;
-    l.inc_cap = INC_CAP;
+    const int nw = E->nt / 64;
     int o = 0;
-    l.smob = o; o = up(o + 4 * (nst + 2));
-    l.sfst = o; o = up(o + 4 * (nst + 2));
-    l.sfix = o; o = up(o + 4 * (nst + 2));
-    l.soff = o; o = up(o + 4 * (nst + 2));
-    l.incs = o; o = up(o + 4 * (l.inc_cap + 1));
-    l.incn = o; o = up(o + 4 * (l.inc_cap + 1));
-    l.map_cap = 4096;
-    l.cand = o; o = up(o + 2 * l.map_cap);
-    l.amap = o; o = up(o + 2 * l.map_cap);
-    l.frag = o; o = up(o + 16 * MAXF);
-    l.frow = o; o = up(o + 4 * MAXF);
-    o = (o + 31) & ~31;
-    l.fragd = o; o = up(o + 32 * MAXF);
-    if (E->staged) {
-        l.pair = o;
-        o = up(o + pair_bytes);
-    } else {
-        l.pair = -1;
-    }
+    l.wave = o; o = (o + nw * WL_BYTES);
     const int eval_end = o;
-    // accept and prep phases reuse the evaluation region
+    // accept and prep phases reuse the waves' scratch
     int a = 0;
     l.members = a; a = up(a + 4 * E->maxk);
     l.w = a; a = up(a + 8 * E->maxk);
     l.val = a; a = up(a + 8 * E->maxk);
     l.accl = a; a = up(a + 8 * E->maxk);
-    l.rsel = a; a = up(a + 8 * E->maxk);
-    l.racc = a; a = up(a + 8 * E->maxk);
-    l.ea = a; a = up(a + 8 * E->maxk);
+    const int mw = (E->maxk + 31) / 32;
+    l.gmask = a; a = up(a + 4 * SEL_GROUPS * mw);
+    l.goff = a; a = up(a + 2 * SEL_GROUPS * mw);
+    l.gstart = a; a = up(a + 4 * (SEL_GROUPS + 1));
+    l.gmin = a; a = up(a + 8 * 64);
+    l.drop = a; a = up(a + 4 * mw);
     // adjacency rows of a move staged in LDS for its accept phase, when they fit
-    const int adj_bytes = 4 * E->maxk * ((E->maxk + 31) / 32);
+    const int adj_bytes = 4 * E->maxk * mw;
     if (a + adj_bytes + 4096 <= 49152) {
         l.adjl = a;
         a = up(a + adj_bytes);
@@ -653,21 +680,33 @@ int compute_layout(gcmc_engine *E)
     }
     l.J = 0;  // prep runs after accept in the same workgroup
     o = std::max(eval_end, a);
+    // the tables stay in LDS through accept and prep
+    if (E->staged) {
+        l.pair = o;
+        o = up(o + pair_bytes);
+    } else {
+        l.pair = -1;
+    }
+    l.team = o; o = up(o + nw * TEAM_BYTES);
     l.spt = o; o = up(o + 16 * MAXT);
     l.misc = o; o = up(o + 4 * MISC_INTS);
-    l.dred = o; o = up(o + 8 * MAXWAVE);
     l.total = o;
-    if (l.total > 65536)
-        return fail(GCMC_E_ARG, "LDS layout exceeds 64 KiB (stencil or confBias too large; raise cell_size)");
+    // 64 KiB for the accept phase (confBias), all of a CU's for the waves' scratch
+    if (a + 16 * MAXT + 4 * MISC_INTS > 65536 || l.total > 163840)
+        return fail(GCMC_E_ARG, "LDS layout exceeds 64 KiB (confBias too large)");
     return 0;
 }
 
-template <int NT, bool S, bool EW>
+template <int NT, bool S, int TM>
 void launch_plain_step(gcmc_engine *E, int r)
 {
+    constexpr bool EW = TM == T_EWALD;
     const size_t lds = E->lay.total;
-    hipLaunchKernelGGL((k_eval_plain<NT, S, EW>), dim3(2 * E->reps[r]->maxk), dim3(NT), lds, E->stream, E->d_rep,
-                       E->d_state, r, E->lay);
+    // workgroups for the most items a move can have, by its teams or its waves
+    const int few = std::min(E->reps[r]->maxk, COOP_TRIALS);
+    const int wgs = std::max((few + NT / 64 / COOP - 1) / (NT / 64 / COOP), (E->reps[r]->maxk + NT / 64 - 1) / (NT / 64));
+    hipLaunchKernelGGL((k_eval_plain<NT, S, TM>), dim3(wgs), dim3(NT), lds, E->stream, E->d_rep, E->d_state, r,
+                       E->lay);
     hipLaunchKernelGGL((k_accept_plain<NT, S, EW>), dim3(1), dim3(NT), lds, E->stream, E->d_rep, E->d_state, r,
                        E->lay);
 }
@@ -681,18 +720,18 @@ void launch_batched(gcmc_engine *E, int nsteps)
                        nsteps, E->d_sched);
     hipLaunchKernelGGL((k_start<NT, S>), dim3(R), dim3(NT), lds, E->stream, E->d_rep, E->d_state, E->d_sched,
                        E->lay, 0, 1);
+    const auto kernel = E->tune.fp32_coulomb ? k_batched<NT, S, T_FP32> : k_batched<NT, S, T_FP64>;
     if (E->resident <= 0) {
         // workgroups beyond the resident ones would only start once the
         // others have exited: launch no more than fit
         int occ = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_batched<NT, S>, NT, lds) != hipSuccess || occ < 1)
-            occ = 1;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, NT, lds) != hipSuccess || occ < 1) occ = 1;
         E->resident = occ * std::max(E->ncu, 1);
     }
     const int nwg = std::min(E->nwg, E->resident);
     if (E->timed_kernel) (void)hipEventRecord(E->evk0, E->stream);
-    hipLaunchKernelGGL((k_batched<NT, S>), dim3(nwg), dim3(NT), lds, E->stream, E->d_rep, E->d_state, R,
-                       E->d_sched, E->lay, E->spin_limit, E->xm, std::min(std::max(E->tune.claim_affinity, 0), 254));
+    hipLaunchKernelGGL(kernel, dim3(nwg), dim3(NT), lds, E->stream, E->d_rep, E->d_state, R, E->d_sched, E->lay,
+                       E->spin_limit, E->xm, std::min(std::max(E->tune.claim_affinity, 0), 254));
     if (E->timed_kernel) (void)hipEventRecord(E->evk1, E->stream);
 }
 
@@ -710,8 +749,9 @@ void launch_plain(gcmc_engine *E, int nsteps)
         const int n = std::min(nsteps, std::max(rem, 0));
         HostRep &H = *E->reps[r];
         for (int s = 0; s < n; ++s) {
-            if (H.pme) launch_plain_step<NT, S, true>(E, r);
-            else launch_plain_step<NT, S, false>(E, r);
+            if (H.pme) launch_plain_step<NT, S, T_EWALD>(E, r);
+            else if (E->tune.fp32_coulomb) launch_plain_step<NT, S, T_FP32>(E, r);
+            else launch_plain_step<NT, S, T_FP64>(E, r);
             if (H.pme) {
                 // charges moved by the step enter the PME grid; new potential
                 gcmc_internal::pme_spread_counted(H.pme, H.rep.pme_cap, H.rep.pme_ndelta, H.rep.pme_delta,
@@ -744,7 +784,7 @@ void launch_ewald_moves(gcmc_engine *E, int nmoves)
     for (int m = 0; m < nmoves; ++m)
         for (int r = 0; r < (int)E->reps.size(); ++r) {
             HostRep &H = *E->reps[r];
-            launch_plain_step<NT, S, true>(E, r);
+            launch_plain_step<NT, S, T_EWALD>(E, r);
             gcmc_internal::pme_spread_counted(H.pme, H.rep.pme_cap, H.rep.pme_ndelta, H.rep.pme_delta,
                                               H.rep.pme_ndelta, E->stream);
             gcmc_pme_solve(H.pme, nullptr, E->stream);
@@ -775,17 +815,29 @@ template <int NT, bool S>
 struct RunEwaldMoves {
     static void run(gcmc_engine *E, int n) { launch_ewald_moves<NT, S>(E, n); }
 };
+// Poses from which one wave each fills the GPU; fewer are shared by four waves.
+constexpr int POSE_WAVES = 4096;
+constexpr int ADJ_WAVES = 2048;   // the same for gradients
+
 template <int NT, bool S>
 struct RunPoses {
+    template <int TM>
+    static void launch(gcmc_engine *E, int npose, int r, int species, const float *dc, const float *dp, const int *dx,
+                       double *de, int *dn, uint32_t *dh)
+    {
+        // every workgroup stages the tables: no more of them than run at once
+        const bool few = npose < POSE_WAVES;
+        const int per = NT / 64 / (few ? COOP : 1), most = std::max(E->ncu, 1) * (1024 / NT);
+        hipLaunchKernelGGL((few ? k_eval_poses<NT, S, TM, COOP> : k_eval_poses<NT, S, TM, 1>),
+                           dim3(std::min((npose + per - 1) / per, most)), dim3(NT), E->lay.total, E->stream, E->d_rep, r,
+                           species, npose, dc, dp, dx, de, dn, dh, E->lay);
+    }
     static void run(gcmc_engine *E, int npose, int r, int species, const float *dc, const float *dp, const int *dx,
                     double *de, int *dn, uint32_t *dh)
     {
-        if (E->reps[r]->pme)
-            hipLaunchKernelGGL((k_eval_poses<NT, S, true>), dim3(npose), dim3(NT), E->lay.total, E->stream, E->d_rep,
-                               r, species, dc, dp, dx, de, dn, dh, E->lay);
-        else
-            hipLaunchKernelGGL((k_eval_poses<NT, S, false>), dim3(npose), dim3(NT), E->lay.total, E->stream,
-                               E->d_rep, r, species, dc, dp, dx, de, dn, dh, E->lay);
+        if (E->reps[r]->pme) launch<T_EWALD>(E, npose, r, species, dc, dp, dx, de, dn, dh);
+        else if (E->tune.fp32_coulomb) launch<T_FP32>(E, npose, r, species, dc, dp, dx, de, dn, dh);
+        else launch<T_FP64>(E, npose, r, species, dc, dp, dx, de, dn, dh);
     }
 };
 
@@ -1689,13 +1741,24 @@ int gcmc_engine_adjoint(gcmc_engine *E, int r, int species, int npose, const flo
     if (H.pme) return fail(GCMC_E_ARG, "the adjoint covers plain Coulomb, not Ewald electrostatics");
     const int nf = H.frag[species].num_atoms;
     const int X = H.rep.X, Y = H.rep.Y;
-    const int adj_off = (E->lay.total + 15) & ~15;
-    const int lds = adj_off + adj_lds_bytes(X, Y);
+    // four waves' scratch, the tables of the layout's end, and the adjoint's own
+    constexpr int NT = 256;
+    LdsLayout l{};
+    l.pair = -1;
+    l.adjl = -1;
+    l.team = NT / 64 * WL_BYTES;
+    l.spt = l.team + NT / 64 * TEAM_BYTES;
+    const int adj_off = l.spt + 16 * MAXT;
+    const int lds = l.total = adj_off + adj_lds_bytes(X, Y, NT / 64);
     if (lds > 65536) return fail(GCMC_E_ARG, "adjoint LDS layout exceeds 64 KiB (too many atom types)");
     hipStream_t s = (hipStream_t)stream;
-#define ADJ_LAUNCH(NFV)                                                                                         \
-    hipLaunchKernelGGL((k_adjoint<256, NFV>), dim3(npose), dim3(256), lds, s, E->d_rep, r, species, centres, poses, \
-                       eps_kcal, rmin_half, dq, energy, dEdx, partial, E->lay, adj_off)
+    // one wave per pose when they fill the GPU, else four; no more workgroups
+    // than run at once (each builds the pair table)
+    const bool few = npose < ADJ_WAVES;
+    const int per = few ? 1 : NT / 64, wgs = std::min((npose + per - 1) / per, std::max(E->ncu, 1) * 4);
+#define ADJ_LAUNCH(NFV)                                                                                            \
+    hipLaunchKernelGGL((few ? k_adjoint<NT, NFV, COOP> : k_adjoint<NT, NFV, 1>), dim3(wgs), dim3(NT), lds, s, E->d_rep, \
+                       r, species, npose, centres, poses, eps_kcal, rmin_half, dq, energy, dEdx, partial, l, adj_off)
     if (nf <= 4) ADJ_LAUNCH(4);
     else if (nf <= 8) ADJ_LAUNCH(8);
     else if (nf <= 12) ADJ_LAUNCH(12);
@@ -1851,10 +1914,10 @@ int gcmc_host_stencil_covers(int n, const float *centres, const float *groups, c
         st[i] = startxyz[i];
     }
     cell_geometry(L, cell_size, nc, inv_h);
-    const std::vector<int> sten = make_stencil(L, nc, cutoff, STENCIL_EPS);
+    const std::vector<int> sten = make_stencil(L, nc, cutoff, 0.0f);
     float h[3], r2;
     int prune;
-    stencil_prune(L, nc, cutoff, h, &prune, &r2);
+    stencil_prune(L, nc, cutoff, 0.0f, h, &prune, &r2);
     for (int q = 0; q < n; ++q) {
         const int cc = cell_index(L, st, inv_h, nc, centres[3 * q], centres[3 * q + 1], centres[3 * q + 2]);
         const int cg = cell_index(L, st, inv_h, nc, groups[3 * q], groups[3 * q + 1], groups[3 * q + 2]);
@@ -1862,10 +1925,11 @@ int gcmc_host_stencil_covers(int n, const float *centres, const float *groups, c
         const int ci[3] = {c0, c1, c2};
         float u[3];
         cell_offset(L, st, h, ci, centres[3 * q], centres[3 * q + 1], centres[3 * q + 2], u);
+        float base[3], hp[3];
+        stencil_base(u, h, prune, base, hp);
         out[q] = 0;
         for (int code : sten) {
-            const int d[3] = {(code & 255) - 128, ((code >> 8) & 255) - 128, ((code >> 16) & 255) - 128};
-            if (!stencil_cell_near(u, d, h, prune, r2)) continue;     // the kernel skips this cell
+            if (!stencil_cell_near(code, base, hp, r2)) continue;     // the kernel skips this cell
             int i0 = c0 + (code & 255) - 128, i1 = c1 + ((code >> 8) & 255) - 128, i2 = c2 + ((code >> 16) & 255) - 128;
             i0 = ((i0 % nc[0]) + nc[0]) % nc[0];
             i1 = ((i1 % nc[1]) + nc[1]) % nc[1];

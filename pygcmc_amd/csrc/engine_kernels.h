@@ -5,8 +5,9 @@
 // threads (NT = 256, 512 or 1024, a tuning choice):
 //   prep    decode moveArray[step]; pick slots (partial Fisher-Yates);
 //           trial centres                      (gcmc_move_*.h host side)
-//   item    one trial evaluation: build the pose, scan the cell list,
-//           group test, pair energies          (Gmove_*, calcEnergy)
+//   item    one trial: build its pose (or old and new pose), scan the cell
+//           list, group test, pair energies    (Gmove_*, calcEnergy), by one
+//           wave, or by four in moves of few trials
 //   accept  grouping of trials, selection, Metropolis in FP64, commit
 //           (move_add/del/trn/rot host logic, Gupdate*)
 // The plain form launches item and accept kernels per move; the batched form
@@ -51,14 +52,42 @@ using CSpecies = const __attribute__((address_space(4))) Species;
 using CRep = const Rep;
 using CSpecies = const Species;
 #endif
+// The same Rep behind an address the compiler cannot relate to C: fields read
+// through it are loaded where they are used (scalar loads), instead of all at
+// once ahead of the loops, which spilled a hundred scalars into vector registers.
+__device__ __forceinline__ CRep &fresh(CRep &C)
+{
+    CRep *p = &C;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(p));
+#endif
+    return *p;
+}
+// The lane index, and a wave-uniform value, as the compiler's own for this use:
+// addresses built from them are not kept in registers through the whole kernel.
+__device__ __forceinline__ int fresh_lane()
+{
+    int l = threadIdx.x & 63;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(l));
+#endif
+    return l;
+}
+__device__ __forceinline__ int fresh_uniform(int x)
+{
+    x = __builtin_amdgcn_readfirstlane(x);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(x));
+#endif
+    return x;
+}
 __device__ __forceinline__ CRep &rep_of(const Rep *reps, int r) { return ((CRep *)reps)[r]; }
 __device__ __forceinline__ CSpecies &species_of(CRep &C, int s) { return ((CSpecies *)C.sp)[s]; }
 
 // scratch ints of a workgroup (Lds::misc)
 enum Misc : int {
-    M_SCAN = 0,      // [0, NW]   scan partials, total at NW
-    M_NIN = 40,      // [40, 56)  per-wave included count
-    M_HASH = 56,     // [56, 72)  per-wave set hash
+    M_GN = 78,       // groups in the batch (select_groups)
+    M_NEXT = 79,     // next of the claimed trials (eval_items)
     M_ACC = 80,      // accept: decision / count of accepted
     M_NG = 81,       //         groups
     M_N = 82,        //         species count after the move
@@ -72,55 +101,69 @@ enum Misc : int {
 };
 
 struct Lds {
-    int *smob, *sfst, *sfix, *soff, *incs, *incn;
-    float4 *frag;
-    int *frow;
-    double4 *fragd;   // fragment pose minus the trial centre (x, y, z), K q (w), FP64
+    char *wave;       // per-wave scratch of evaluations (WaveLds)
+    void *team;       // sums of the waves that share a trial
     float4 *pair;
     int4 *spt;
     int *misc;
-    double *dred;
     int *members;
     double *w, *val;
     int2 *accl;
     uint32_t *adjl;   // adjacency rows staged for the accept phase (null: read C.adj)
-    double *rsel, *racc, *ea;  // accept: selection / acceptance draw per group, exp term per trial
+    // accept, a batch of groups: member masks, first place of each mask's members
+    // and of each group in `members`, lowest values (order_key)
+    uint32_t *gmask, *drop;
+    uint16_t *goff;
+    int *gstart;
+    unsigned long long *gmin;
     int *J;
-    int inc_cap;
-    uint16_t *cand, *amap;  // index maps expanded by wg_scan (valid when the total <= map_cap)
-    int map_cap;
 };
 
 __device__ inline Lds carve(char *b, const LdsLayout &l)
 {
     Lds s;
-    s.smob = (int *)(b + l.smob);
-    s.sfst = (int *)(b + l.sfst);
-    s.sfix = (int *)(b + l.sfix);
-    s.soff = (int *)(b + l.soff);
-    s.incs = (int *)(b + l.incs);
-    s.incn = (int *)(b + l.incn);
-    s.frag = (float4 *)(b + l.frag);
-    s.frow = (int *)(b + l.frow);
-    s.fragd = (double4 *)(b + l.fragd);
+    s.wave = b + l.wave;
+    s.team = b + l.team;
     s.pair = (float4 *)(b + (l.pair >= 0 ? l.pair : 0));
     s.spt = (int4 *)(b + l.spt);
     s.misc = (int *)(b + l.misc);
-    s.dred = (double *)(b + l.dred);
     s.members = (int *)(b + l.members);
     s.w = (double *)(b + l.w);
     s.val = (double *)(b + l.val);
     s.accl = (int2 *)(b + l.accl);
     s.adjl = l.adjl >= 0 ? (uint32_t *)(b + l.adjl) : nullptr;
-    s.rsel = (double *)(b + l.rsel);
-    s.racc = (double *)(b + l.racc);
-    s.ea = (double *)(b + l.ea);
+    s.gmask = (uint32_t *)(b + l.gmask);
+    s.drop = (uint32_t *)(b + l.drop);
+    s.goff = (uint16_t *)(b + l.goff);
+    s.gstart = (int *)(b + l.gstart);
+    s.gmin = (unsigned long long *)(b + l.gmin);
     s.J = (int *)(b + l.J);
-    s.inc_cap = l.inc_cap;
-    s.cand = (uint16_t *)(b + l.cand);
-    s.amap = (uint16_t *)(b + l.amap);
-    s.map_cap = l.map_cap;
     return s;
+}
+
+// A wave's scratch: the cells it scans, the batch of included groups (offset of
+// its first atom in the batch << 2 | flags; atom index minus that offset), the
+// batch's atom -> group marks, candidate -> cell marks, and up to two poses.
+struct WaveLds {
+    uint32_t *list;
+    int *goff, *gdel;
+    uint8_t *amap, *head;
+    float4 *frag;      // [2][MAXF] (x, y, z, K q), atom order
+    double4 *fragd;    // [2][MAXF] ordered by type: relative to the centre, K q (or float4, absolute)
+};
+
+__device__ __forceinline__ WaveLds wave_lds(const Lds &L, int wave)
+{
+    char *b = L.wave + wave * WL_BYTES;
+    WaveLds w;
+    w.fragd = (double4 *)b; b += 2 * MAXF * 32;
+    w.frag = (float4 *)b; b += 2 * MAXF * 16;
+    w.amap = (uint8_t *)b; b += WL_ATOMS;
+    w.list = (uint32_t *)b; b += 4 * WL_CELLS;
+    w.goff = (int *)b; b += 4 * WL_GROUPS;
+    w.gdel = (int *)b; b += 4 * WL_GROUPS;
+    w.head = (uint8_t *)b;
+    return w;
 }
 
 __device__ inline void wave_sync()
@@ -228,78 +271,17 @@ __device__ inline double permute_d(int dst, double v)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// exclusive scan of a[0..n) in LDS, a[n] = total; returns total
-template <int NT>
-// When map is given and the total is at most cap, also writes map[j] = i for
-// every j in [a'[i], a'[i+1]) (a' the scanned array): the entry each item
-// belongs to, so a thread finds it with one read instead of a binary search.
-__device__ inline int wg_scan(int *a, int n, int *misc, uint16_t *map = nullptr, int cap = 0)
-{
-    constexpr int NW = NT / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int per = (n + NT - 1) / NT;
-    const int b = tid * per;
-    const int e = min(n, b + per);
-    int sum = 0;
-    for (int i = b; i < e; ++i) sum += a[i];
-    const int x = wave_scan_add(sum);
-    if (lane == 63) misc[M_SCAN + wave] = x;
-    __syncthreads();
-    if (tid == 0) {
-        int t = 0;
-        for (int w = 0; w < NW; ++w) {
-            int v = misc[M_SCAN + w];
-            misc[M_SCAN + w] = t;
-            t += v;
-        }
-        misc[M_SCAN + NW] = t;
-    }
-    __syncthreads();
-    int base = misc[M_SCAN + wave] + x - sum;
-    const int total = misc[M_SCAN + NW];
-    const bool expand = map != nullptr && total <= cap;
-    for (int i = b; i < e; ++i) {
-        int v = a[i];
-        a[i] = base;
-        if (expand)
-            for (int j = 0; j < v; ++j) map[base + j] = (uint16_t)i;
-        base += v;
-    }
-    if (tid == 0) a[n] = total;
-    __syncthreads();
-    return total;
-}
-
-// largest e in [0, n) with a[e] <= m (a[0] = 0 <= m < a[n])
-__device__ inline int bsearch_le(const int *a, int n, int m)
+// largest e in [0, n) with a[e] >> 2 <= m (a[0] >> 2 = 0 <= m): the group an atom
+// of a batch that is too large for its atom map belongs to
+__device__ inline int bsearch_off(const int *a, int n, int m)
 {
     int lo = 0, hi = n - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
-        if (a[mid] <= m) lo = mid;
+        if ((a[mid] >> 2) <= m) lo = mid;
         else hi = mid - 1;
     }
     return lo;
-}
-
-// bsearch_le for two keys at once (independent LDS reads in flight together)
-__device__ inline void bsearch_le2(const int *a, int n, int m0, int m1, int &g0, int &g1)
-{
-    int lo0 = 0, hi0 = n - 1, lo1 = 0, hi1 = n - 1;
-    while (lo0 < hi0 || lo1 < hi1) {
-        const int mid0 = (lo0 + hi0 + 1) >> 1, mid1 = (lo1 + hi1 + 1) >> 1;
-        const int v0 = a[mid0], v1 = a[mid1];
-        if (lo0 < hi0) {
-            if (v0 <= m0) lo0 = mid0;
-            else hi0 = mid0 - 1;
-        }
-        if (lo1 < hi1) {
-            if (v1 <= m1) lo1 = mid1;
-            else hi1 = mid1 - 1;
-        }
-    }
-    g0 = lo0;
-    g1 = lo1;
 }
 
 // a - b = s + e exactly (Knuth TwoSum of a and -b); returns s
@@ -312,173 +294,244 @@ __device__ inline float two_diff(float a, float b, float &e)
     return s;
 }
 
-// ---- pair energies of the buffered included groups ------------------------
-// lane <-> environment atom (float4 load, coalesced within a group), loop
-// over the fragment atoms held in LDS; FP64 terms into acc64 (default), or
-// FP32 terms with TwoSum into (acc, cmp) (fp32_coulomb and Ewald modes).
-// (cxd, cyd, czd): the trial centre; wrap: image shift per pair.
-template <int NT, bool STAGED, bool EW>
-__device__ inline int pair_pass(CRep &C, const Lds &L, int n, int nf, float &acc, float &cmp, double &acc64,
-                                double cxd, double cyd, double czd, bool wrap)
+__device__ __forceinline__ float uniform_f(float x)
 {
-    const int A = wg_scan<NT>(L.incn, n, L.misc, L.amap, L.map_cap);
-    const bool mapped = A <= L.map_cap;
-    const auto atom = gbl(C.atom);
-    const auto atype = gbl(C.atype);
-    const auto GPT = gbl(C.pair);
-    const float Lx = C.L[0], Ly = C.L[1], Lz = C.L[2];
-    const float ix = C.invL[0], iy = C.invL[1], iz = C.invL[2];
-    const float eb = C.ew_beta;
-    const bool c64 = !EW && C.coul64 != 0;
-    double accd = 0.0;
-    // one environment atom against every fragment atom; a thread takes atoms
-    // t, t + NT, t + 2 NT, ... in that order (the order of its sums)
-    auto pair_row = [&](const int f, const int ty) {
-        if constexpr (STAGED)
-            return L.pair[L.frow[f] + ty];
-        else
-            return GPT[L.frow[f] + ty];
-    };
-    // Default mode: every pair term in FP64.  The environment atom's
-    // position relative to the trial centre, image-shifted once per atom, and
-    // the fragment atom's (L.fragd) are exact differences of FP32 positions
-    // (to 2^-53); their difference needs no further image shift when
-    // Rep::nowrap holds, else it takes one per pair.  1/r: the FP32 estimate
-    // (relative error ~2^-22) and one FP64 Newton step (~1.5 2^-44).
-    const double Lxd = Lx, Lyd = Ly, Lzd = Lz, ixd = ix, iyd = iy, izd = iz;
-    auto atom_terms64 = [&](const float4 at, const int ty) {
-        double ax = (double)at.x - cxd, ay = (double)at.y - cyd, az = (double)at.z - czd;
-        ax = fma(-rint(ax * ixd), Lxd, ax);
-        ay = fma(-rint(ay * iyd), Lyd, ay);
-        az = fma(-rint(az * izd), Lzd, az);
-        const double qa = (double)at.w;
-        // the table entry of fragment atom f + 1 is fetched while atom f's
-        // terms are computed (the last fetch repeats atom nf - 1's)
-        float4 pn = pair_row(0, ty);
-        for (int f = 0; f < nf; ++f) {
-            const double4 F = L.fragd[f];
-            const float4 pp = pn;
-            pn = pair_row(min(f + 1, nf - 1), ty);
-            double ux = ax - F.x, uy = ay - F.y, uz = az - F.z;
-            if (wrap) {
-                ux = fma(-rint(ux * ixd), Lxd, ux);
-                uy = fma(-rint(uy * iyd), Lyd, uy);
-                uz = fma(-rint(uz * izd), Lzd, uz);
-            }
-            const double r2 = fma(uz, uz, fma(uy, uy, ux * ux));
-            double y = (double)__builtin_amdgcn_rsqf((float)r2);
-            y = y * fma(-0.5 * r2 * y, y, 1.5);
-            const double s2 = ((double)pp.x + (double)pp.z) * (y * y);   // 100 sigma^2 / r^2
-            const double s6 = s2 * s2 * s2;
-            accd = fma((double)pp.y, fma(s6, s6, -s6), accd);            // 4 eps (s^12 - s^6)
-            accd = fma(F.w * qa, y, accd);                                // K q_f q_a / r
-        }
-    };
-    // fp32_coulomb and Ewald modes: FP32 terms, TwoSum into (acc, cmp)
-    auto atom_terms = [&](const float4 at, const int ty) {
-        // the table entry of fragment atom f + 1 is fetched while atom f's
-        // terms are computed (the last fetch repeats atom nf - 1's)
-        float4 pn = pair_row(0, ty);
-        for (int f = 0; f < nf; ++f) {
-            const float4 fr = L.frag[f];
-            const float4 pp = pn;
-            pn = pair_row(min(f + 1, nf - 1), ty);
-            // displacement as an exact sum s + e (TwoSum); the image shift
-            // s - n L is exact for |n| <= 1 (Sterbenz)
-            float ex, ey, ez;
-            float dx = two_diff(at.x, fr.x, ex);
-            float dy = two_diff(at.y, fr.y, ey);
-            float dz = two_diff(at.z, fr.z, ez);
-            dx = fmaf(-rintf(dx * ix), Lx, dx);
-            dy = fmaf(-rintf(dy * iy), Ly, dy);
-            dz = fmaf(-rintf(dz * iz), Lz, dz);
-            const float r2h = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-            const float r2c = fmaf(dz, ez, fmaf(dy, ey, dx * ex));
-            const float r2 = fmaf(2.0f, r2c, r2h);
-            float ir = __builtin_amdgcn_rsqf(r2);
-            ir = ir * fmaf(-0.5f * r2 * ir, ir, 1.5f);     // one Newton step
-            // s^2 = 100 sigma^2 / r^2 to ~0.5 ulp: 100 sigma^2 held exactly as
-            // pp.x + pp.z, quotient with one residual correction.  s^12
-            // multiplies the relative error of s^2 by six, and a rounded
-            // table value would err alike on every pair of a type pair.
-            const float rr = __builtin_amdgcn_rcpf(r2);
-            float s2 = pp.x * rr;
-            s2 = fmaf(fmaf(-s2, r2, pp.x) + pp.z, rr, s2);
-            const float s6 = s2 * s2 * s2;
-            float lj = pp.y * fmaf(s6, s6, -s6);           // 4 eps (s^12 - s^6)
-            if (s2 > 1.0f) {
-                // inside sigma s^12 dominates and carries six times the
-                // relative error of r^2: this rare pair's LJ term in FP64,
-                // from the exact displacement
-                const double ux = (double)dx + (double)ex, uy = (double)dy + (double)ey,
-                             uz = (double)dz + (double)ez;
-                const double r2d = fma(uz, uz, fma(uy, uy, ux * ux));
-                double q = __builtin_amdgcn_rcp(r2d);
-                q = q * fma(-r2d, q, 2.0);
-                q = q * fma(-r2d, q, 2.0);
-                const double s2d = ((double)pp.x + (double)pp.z) * q;
-                const double s6d = s2d * s2d * s2d;
-                accd = fma((double)pp.y, fma(s6d, s6d, -s6d), accd);
-                lj = 0.0f;
-            }
-            float el = (fr.w * at.w) * ir;                  // K q_f q_a / r
-            if (EW) el *= erfcf(eb * (r2 * ir));            // Ewald real-space part
-            const float term = lj + el;
-            const float s = acc + term;                     // TwoSum
-            const float bp = s - acc;
-            const float err = (acc - (s - bp)) + (term - bp);
-            acc = s;
-            cmp += err;
-        }
-    };
-    // U atoms per thread per round, all loads issued before any is used: a
-    // thread takes atoms t, t + NT, t + 2 NT, ... in that order (the order of
-    // its sums, whatever U is)
-    constexpr int U = 3;
-    for (int t0 = threadIdx.x; t0 < A; t0 += U * NT) {
-        int a[U];
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+__device__ __forceinline__ int uniform_i(int x) { return __builtin_amdgcn_readfirstlane(x); }
+// lanes below this one whose bit is set
+__device__ __forceinline__ int rank_below(unsigned long long bal)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+}
+__device__ __forceinline__ int wave_scan_max(int x)
+{
+    return wave_scan(x, 0, [](int a, int b) { return b > a ? b : a; });
+}
+__device__ __forceinline__ int lane_up(int v, int src) { return __builtin_amdgcn_ds_bpermute(src * 4, v); }
+
+// ---- pair energies of a batch of included groups ----------------------------
+// One wave; lane <-> environment atom, two atoms per lane and round, the next
+// round's atoms loaded while this one's terms are computed; loop over the
+// fragment atoms held in LDS, ordered by type so that the pair-table entry of
+// a lane's atom is fetched once per type, not once per fragment atom.  A batch's
+// atoms serve one or two poses ("sets": the old and new pose of a translate or
+// rotate trial); bit s of a group's flags says that it is within the cutoff of
+// pose s's centre.  FP64 terms by default, FP32 terms (fp32_coulomb, Ewald)
+// added up in FP64.
+// Bound by FP64 issue (about 20 instructions and one FP32 rsq per pair).
+enum Terms : int { T_FP64, T_FP32, T_EWALD };   // FP32 terms with plain or Ewald real-space Coulomb
+
+template <bool STAGED, int TM>
+struct EnergyPass {
+    float x[2], y[2], z[2];   // centres of the poses (uniform)
+    int first, nset;          // poses first .. first + nset - 1
+    bool wrap;                // image shift per pair (else per environment atom)
+    int spi, nf;
+    double acc[2];            // this lane's sums
+
+    template <class T>
+    __device__ __forceinline__ T entry(CRep &C, const Lds &L, int i) const
+    {
+        if constexpr (STAGED) return ((const T *)L.pair)[i];
+        else return ((gptr<const T>)gbl(C.pair))[i];
+    }
+
+    // Every pair term in FP64.  The environment atom's position relative to the
+    // trial centre, image-shifted once per atom, and the fragment atom's (W.fragd)
+    // are exact differences of FP32 positions (to 2^-53); their difference needs
+    // no further image shift when Rep::nowrap holds, else it takes one per pair.
+    // 1/r: the FP32 estimate (relative error ~2^-22) and one FP64 Newton step
+    // (~1.5 2^-44).  LJ as (A r^-6 - B) r^-6 from the table's A, B; Coulomb's
+    // environment charge taken out of the sum.
+    template <bool WRAP, int U>
+    __device__ __forceinline__ void terms64(CRep &C, const Lds &L, const WaveLds &W, int s, const float4 *at,
+                                            const int *ty, const int *fl)
+    {
+        const double Lx = C.Ld[0], Ly = C.Ld[1], Lz = C.Ld[2], ix = C.invLd[0], iy = C.invLd[1], iz = C.invLd[2];
+        const double cx = s ? x[1] : x[0], cy = s ? y[1] : y[0], cz = s ? z[1] : z[0];
+        CSpecies &F = species_of(C, spi);
+        double ax[U], ay[U], az[U], lj[U], cq[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int tu = t0 + u * NT;
-            const int tq = tu < A ? tu : t0;
-            int g;
-            if (mapped) {
-                g = L.amap[tq];
-            } else {
-                int gx;
-                bsearch_le2(L.incn, n, tq, tq, g, gx);
-            }
-            a[u] = L.incs[g] + (tq - L.incn[g]);
+            ax[u] = (double)at[u].x - cx;
+            ay[u] = (double)at[u].y - cy;
+            az[u] = (double)at[u].z - cz;
+            ax[u] = fma(-rint(ax[u] * ix), Lx, ax[u]);
+            ay[u] = fma(-rint(ay[u] * iy), Ly, ay[u]);
+            az[u] = fma(-rint(az[u] * iz), Lz, az[u]);
+            lj[u] = cq[u] = 0.0;
         }
-        float4 at[U];
-        int ty[U];
+        const double4 *fd = W.fragd + s * MAXF;
+        const int nrun = F.nrun;
+        int f = 0, row = F.run_row[0], end = F.run_end[0];
+        double4 qn = fd[0];
+        double2 pn[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            at[u] = atom[a[u]];
-            ty[u] = atype[a[u]];
+        for (int u = 0; u < U; ++u) pn[u] = entry<double2>(C, L, row + ty[u]);
+        for (int r = 0; r < nrun; ++r) {
+            double2 p[U];
+            const int stop = end;
+#pragma unroll
+            for (int u = 0; u < U; ++u) p[u] = pn[u];
+            if (r + 1 < nrun) {
+                // the next type's entries arrive while this one's atoms are done
+                row = F.run_row[r + 1];
+                end = F.run_end[r + 1];
+#pragma unroll
+                for (int u = 0; u < U; ++u) pn[u] = entry<double2>(C, L, row + ty[u]);
+            }
+            for (; f < stop; ++f) {
+                // the next atom's position arrives while this one's terms are computed
+                const double4 q = qn;
+                qn = fd[f + 1];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    double ux = ax[u] - q.x, uy = ay[u] - q.y, uz = az[u] - q.z;
+                    if (WRAP) {
+                        ux = fma(-rint(ux * ix), Lx, ux);
+                        uy = fma(-rint(uy * iy), Ly, uy);
+                        uz = fma(-rint(uz * iz), Lz, uz);
+                    }
+                    const double r2 = fma(uz, uz, fma(uy, uy, ux * ux));
+                    double v = (double)__builtin_amdgcn_rsqf((float)r2);
+                    v = v * fma(-0.5 * r2 * v, v, 1.5);
+                    const double v2 = v * v, v6 = v2 * v2 * v2;
+                    lj[u] = fma(fma(p[u].x, v6, -p[u].y), v6, lj[u]);
+                    cq[u] = fma(q.w, v, cq[u]);
+                }
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (t0 + u * NT < A) {
-                if (c64) atom_terms64(at[u], ty[u]);
-                else atom_terms(at[u], ty[u]);
-            }
+            const double e = fma((double)at[u].w, cq[u], lj[u]);
+            const double m = ((fl[u] >> s) & 1) ? e : 0.0;
+            if (s) acc[1] += m;
+            else acc[0] += m;
         }
     }
-    __syncthreads();
-    acc64 += accd;
-    return A;
-}
 
-// the energy pass of eval_energy
-template <bool EW>
-struct EnergyPass {
-    double cx, cy, cz;   // trial centre
-    bool wrap;           // image shift per pair (else per environment atom)
-    template <int NT, bool STAGED>
-    __device__ int run(CRep &C, const Lds &L, int n, int nf, float &acc, float &cmp, double &acc64)
+    // FP32 terms (fp32_coulomb, Ewald) from the TwoSum-exact displacement
+    template <int U>
+    __device__ __forceinline__ void terms32(CRep &C, const Lds &L, const WaveLds &W, int s, const float4 *at,
+                                            const int *ty, const int *fl)
     {
-        return pair_pass<NT, STAGED, EW>(C, L, n, nf, acc, cmp, acc64, cx, cy, cz, wrap);
+        const float Lx = C.L[0], Ly = C.L[1], Lz = C.L[2], ix = C.invL[0], iy = C.invL[1], iz = C.invL[2];
+        const float eb = C.ew_beta;
+        CSpecies &F = species_of(C, spi);
+        const float4 *fs = (const float4 *)(W.fragd + s * MAXF);
+        double sum[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) sum[u] = 0.0;
+        const int nrun = F.nrun;
+        int f = 0;
+        for (int r = 0; r < nrun; ++r) {
+            const int row = F.run_row[r], stop = F.run_end[r];
+            float4 pp[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) pp[u] = entry<float4>(C, L, row + ty[u]);
+            for (; f < stop; ++f) {
+                const float4 fr = fs[f];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    // displacement as an exact sum s + e (TwoSum); the image shift
+                    // s - n L is exact for |n| <= 1 (Sterbenz)
+                    float ex, ey, ez;
+                    float dx = two_diff(at[u].x, fr.x, ex);
+                    float dy = two_diff(at[u].y, fr.y, ey);
+                    float dz = two_diff(at[u].z, fr.z, ez);
+                    dx = fmaf(-rintf(dx * ix), Lx, dx);
+                    dy = fmaf(-rintf(dy * iy), Ly, dy);
+                    dz = fmaf(-rintf(dz * iz), Lz, dz);
+                    const float r2h = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                    const float r2c = fmaf(dz, ez, fmaf(dy, ey, dx * ex));
+                    const float r2 = fmaf(2.0f, r2c, r2h);
+                    float ir = __builtin_amdgcn_rsqf(r2);
+                    ir = ir * fmaf(-0.5f * r2 * ir, ir, 1.5f);     // one Newton step
+                    // s^2 = 100 sigma^2 / r^2 to ~0.5 ulp: 100 sigma^2 held exactly as
+                    // pp.x + pp.z, quotient with one residual correction.  s^12
+                    // multiplies the relative error of s^2 by six, and a rounded
+                    // table value would err alike on every pair of a type pair.
+                    const float rr = __builtin_amdgcn_rcpf(r2);
+                    float s2 = pp[u].x * rr;
+                    s2 = fmaf(fmaf(-s2, r2, pp[u].x) + pp[u].z, rr, s2);
+                    const float s6 = s2 * s2 * s2;
+                    float lj = pp[u].y * fmaf(s6, s6, -s6);        // 4 eps (s^12 - s^6)
+                    if (s2 > 1.0f) {
+                        // inside sigma s^12 dominates and carries six times the
+                        // relative error of r^2: this rare pair's LJ term in FP64,
+                        // from the exact displacement
+                        const double ux = (double)dx + (double)ex, uy = (double)dy + (double)ey,
+                                     uz = (double)dz + (double)ez;
+                        const double r2d = fma(uz, uz, fma(uy, uy, ux * ux));
+                        double q = __builtin_amdgcn_rcp(r2d);
+                        q = q * fma(-r2d, q, 2.0);
+                        q = q * fma(-r2d, q, 2.0);
+                        const double s2d = ((double)pp[u].x + (double)pp[u].z) * q;
+                        const double s6d = s2d * s2d * s2d;
+                        sum[u] = fma((double)pp[u].y, fma(s6d, s6d, -s6d), sum[u]);
+                        lj = 0.0f;
+                    }
+                    float el = (fr.w * at[u].w) * ir;              // K q_f q_a / r
+                    if (TM == T_EWALD) el *= erfcf(eb * (r2 * ir));           // Ewald real-space part
+                    sum[u] += (double)(lj + el);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const double m = ((fl[u] >> s) & 1) ? sum[u] : 0.0;
+            if (s) acc[1] += m;
+            else acc[0] += m;
+        }
+    }
+
+    // g groups with A atoms in W's batch
+    __device__ __forceinline__ void run(CRep &C0, const Lds &L, const WaveLds &W, int g, int A)
+    {
+        CRep &C = fresh(C0);
+        constexpr int U = 1;
+        const int lane = fresh_lane();
+        const auto atom = gbl(C.atom);
+        const auto atype = gbl(C.atype);
+        const bool mapped = A <= WL_ATOMS;
+        int carry = 0;
+        float4 an[U];
+        int tn[U], fn[U];
+        auto fetch = [&](int base) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = base + u * 64 + lane, tq = min(t, A - 1);
+                int slot;
+                if (mapped) {
+                    slot = max(wave_scan_max(W.amap[t]), carry);
+                    carry = __builtin_amdgcn_readlane(slot, 63);
+                } else {
+                    slot = bsearch_off(W.goff, g, tq);
+                }
+                const int w = W.goff[slot], a = W.gdel[slot] + tq;
+                fn[u] = t < A ? w : 0;
+                an[u] = atom[a];
+                tn[u] = atype[a];
+            }
+        };
+        fetch(0);
+        for (int base = 0; base < A; base += 64 * U) {
+            float4 at[U];
+            int ty[U], fl[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                at[u] = an[u];
+                ty[u] = tn[u];
+                fl[u] = fn[u];
+            }
+            if (base + 64 * U < A) fetch(base + 64 * U);
+            for (int s = first; s < first + nset; ++s) {
+                if constexpr (TM != T_FP64) terms32<U>(C, L, W, s, at, ty, fl);
+                else if (wrap) terms64<true, U>(C, L, W, s, at, ty, fl);
+                else terms64<false, U>(C, L, W, s, at, ty, fl);
+            }
+        }
     }
 };
 
@@ -504,204 +557,340 @@ __device__ inline void stage_pair_table(CRep &C, const Lds &L)
         if (b + lane < n) __builtin_amdgcn_global_load_lds((const void *)(P + b + lane), (void *)&L.pair[b], 16, 0, 0);
 }
 
-// ---- calcEnergy over the cell list -----------------------------------------
-// Candidates: fixed and mobile groups of the stencil cells around the test
-// centre plus the overflow bucket; kept when gid != exclude and the FP32
-// distanceP test passes (gcmc_energy.h:152-191).  Needs L.spt loaded.
-// Thread 0 receives the results.
-template <int NT, bool STAGED, class Pass>
-__device__ __attribute__((always_inline)) inline void eval_energy_pass(CRep &C, float cx, float cy, float cz,
-                                                                       int nf, int exclude, const Lds &L, Pass &P,
-                                                                       double *outE, int *outN, uint32_t *outH,
-                                                                       int *outA, unsigned long long *ticks)
+// tables of a replica into LDS, complete for every wave on return
+template <int NT, bool STAGED>
+__device__ inline void stage_tables(CRep &C, const Lds &L, bool rep, bool tab)
 {
-    unsigned long long tk0 = wall_clock64(), tpair = 0;
-    constexpr int NW = NT / 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const auto stencil = gbl(C.stencil);
-    const auto cellv = gbl(C.cell);
-    const auto fix = gbl(C.fix);
-    const auto mob_rec = gbl(C.mob_rec);
-    const int cc = cell_index(C.L, C.start, C.inv_h, C.nc, cx, cy, cz);
-    const int c2 = cc % C.nc[2];
-    const int c1 = (cc / C.nc[2]) % C.nc[1];
-    const int c0 = cc / (C.nc[1] * C.nc[2]);
-    // the centre's position inside its cell
-    float u[3];
-    {
-        const int ci[3] = {c0, c1, c2};
-        cell_offset(C.L, C.start, C.cell_h, ci, cx, cy, cz, u);
+    if (rep) load_species_table(C, L);
+    if (STAGED && tab) {
+        stage_pair_table<NT>(C, L);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    const int ne = C.nst + 1;
-    for (int e = tid; e < ne; e += NT) {
-        int cell, fs, fc, mc;
-        if (e < C.nst) {
-            const int code = stencil[e];
-            const int d[3] = {(code & 255) - 128, ((code >> 8) & 255) - 128, ((code >> 16) & 255) - 128};
-            // cells whose box lies beyond rc + slack from the centre hold no
-            // group centre that passes the test: no loads for them
-            if (!stencil_cell_near(u, d, C.cell_h, C.prune, C.prune_r2)) {
-                fs = 0;
-                fc = 0;
-                mc = 0;
-                L.smob[e] = 0;
-            } else {
-                // stencil offsets span at most one box per axis: wrap by one add
-                int i0 = c0 + d[0];
-                int i1 = c1 + d[1];
-                int i2 = c2 + d[2];
-                i0 += i0 < 0 ? C.nc[0] : (i0 >= C.nc[0] ? -C.nc[0] : 0);
-                i1 += i1 < 0 ? C.nc[1] : (i1 >= C.nc[1] ? -C.nc[1] : 0);
-                i2 += i2 < 0 ? C.nc[2] : (i2 >= C.nc[2] ? -C.nc[2] : 0);
-                cell = (i0 * C.nc[1] + i1) * C.nc[2] + i2;
-                const int2 ci = cellv[cell];
-                fs = ci.x;
-                fc = cellv[cell + 1].x - fs;
-                mc = ci.y;
-                L.smob[e] = cell * C.cap;
-            }
-        } else {
-            fs = 0;
-            fc = 0;
-            mc = cellv[C.ncell].y;
-            L.smob[e] = C.ovf_base;
-        }
-        L.sfst[e] = fs;
-        L.sfix[e] = fc;
-        L.soff[e] = fc + mc;
-    }
-    __syncthreads();
-    const int M = wg_scan<NT>(L.soff, ne, L.misc, L.cand, L.map_cap);
-    const bool mapped = M <= L.map_cap;
-    const unsigned long long tk1 = wall_clock64();
-    float acc = 0.0f, cmp = 0.0f;
-    double acc64 = 0.0;  // FP64 pair terms (Coulomb)
-    int nin = 0, natom = 0;
-    uint32_t hs = 0;
-    // Candidates in chunks of R rounds of NT.  A thread first issues the
-    // record loads of its R candidates of the chunk (one memory round trip
-    // for all of them), then tests them in order; each wave appends the
-    // groups it includes to its own segment of SEG = 64 R slots, so no
-    // barrier is needed within a chunk; after a chunk the unused slots get
-    // zero atoms and one pair pass covers all segments (groups in segment
-    // order).
-    constexpr int R = INC_CAP / NT, SEG = 64 * R;
-    for (int base = 0; base < M; base += R * NT) {
-        float4 rec[R];
-        int2 rng[R];
-        bool fixed[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int m = base + r * NT + tid;
-            rec[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-            rng[r] = make_int2(0, 0);
-            fixed[r] = false;
-            if (m < M) {
-                const int e = mapped ? (int)L.cand[m] : bsearch_le(L.soff, ne, m);
-                const int local = m - L.soff[e];
-                const int fc = L.sfix[e];
-                if (local < fc) {
-                    const int q = L.sfst[e] + local;
-                    rec[r] = fix[q].p;
-                    rng[r] = fix[q].rng;
-                    fixed[r] = true;
-                } else {
-                    rec[r] = mob_rec[L.smob[e] + (local - fc)];
-                }
-            }
-        }
-        int cnt = 0;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int m = base + r * NT + tid;
-            bool inc = false;
-            int2 rr = rng[r];
-            if (m < M) {
-                const float4 p = rec[r];
-                int gid;
-                if (fixed[r]) {
-                    gid = __float_as_int(p.w);
-                } else {
-                    const int word = __float_as_int(p.w);
-                    gid = word & GID_MASK;
-                    const int4 sp = L.spt[word >> GID_BITS];   // (startRes, maxNum, atomBase, nf)
-                    rr = make_int2(sp.z + (gid - sp.x) * sp.w, sp.w);
-                }
-                inc = (gid != exclude) && within(cx, cy, cz, p.x, p.y, p.z, C.ax, C.r2max);
-                if (inc) {
-                    nin += 1;
-                    hs += group_hash((uint32_t)gid);
-                }
-            }
-            const unsigned long long bal = __ballot(inc);
-            if (inc) {
-                const int pos = wave * SEG + cnt + __popcll(bal & ((1ull << lane) - 1ull));
-                L.incs[pos] = rr.x;
-                L.incn[pos] = rr.y;
-            }
-            cnt += __popcll(bal);
-        }
-        for (int q = cnt + lane; q < SEG; q += 64) L.incn[wave * SEG + q] = 0;
-        // a staged pair table was loaded into LDS asynchronously (eval_item):
-        // every wave's copies have landed once the barrier passes
-        if (STAGED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        const unsigned long long tp0 = wall_clock64();
-        natom += P.template run<NT, STAGED>(C, L, INC_CAP, nf, acc, cmp, acc64);
-        tpair += wall_clock64() - tp0;
-    }
-    const double v = wave_scan_add((double)acc + (double)cmp + acc64);
-    nin = wave_scan_add(nin);
-    hs = wave_scan_add(hs);
-    if (lane == 63) {
-        L.dred[wave] = v;
-        L.misc[M_NIN + wave] = nin;
-        L.misc[M_HASH + wave] = (int)hs;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        double E = 0.0;
-        int N = 0;
-        uint32_t H = 0;
-        for (int w = 0; w < NW; ++w) {
-            E += L.dred[w];
-            N += L.misc[M_NIN + w];
-            H += (uint32_t)L.misc[M_HASH + w];
-        }
-        *outE = E;
-        *outN = N;
-        *outH = H;
-        *outA = natom;
-        if (ticks) {
-            const unsigned long long tk2 = wall_clock64();
-            ticks[1] = tk1 - tk0;
-            ticks[2] = (tk2 - tk1) - tpair;
-            ticks[3] = tpair;
-        }
-    }
-    __syncthreads();
+    if (rep || (STAGED && tab)) __syncthreads();
 }
 
-// pose_near: the pose in L.frag was generated from the species template or
-// the molecule's atoms (within the species' extent of the centre, the bound
-// Rep::nowrap rests on); poses given by a caller take the per-pair image shift.
-// Thread f reads L.frag[f] (written by thread f, or before a barrier) and
-// writes L.fragd[f]; eval_energy_pass has a barrier before its first pair
-// pass.
-template <int NT, bool STAGED, bool EW = false>
-__device__ __attribute__((always_inline)) inline void eval_energy(CRep &C, float cx, float cy, float cz, int nf,
-                                                                  int exclude, const Lds &L, double *outE, int *outN,
-                                                                  uint32_t *outH, int *outA,
-                                                                  unsigned long long *ticks = nullptr,
-                                                                  bool pose_near = false)
+// The FP32 group test (within, gcmc_math.h) of a wave's lanes at once: without
+// branches when no lane is past the shift table (one ballot), else literally.
+// Nested branches per axis kept a dozen execution masks alive and spilled the
+// scalar registers.
+struct GroupCut {
+    AxisCut ax[3];
+    float r2max;
+};
+__device__ __forceinline__ GroupCut group_cut(CRep &C)
 {
-    EnergyPass<EW> P{(double)cx, (double)cy, (double)cz, !(pose_near && C.nowrap != 0)};
-    const int tid = threadIdx.x;
-    if (tid < nf) {
-        const float4 q = L.frag[tid];
-        L.fragd[tid] = make_double4((double)q.x - P.cx, (double)q.y - P.cy, (double)q.z - P.cz, (double)q.w);
+    GroupCut g;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        g.ax[i].L = C.ax[i].L;
+        g.ax[i].t[0] = C.ax[i].t[0];
+        g.ax[i].t[1] = C.ax[i].t[1];
+        g.ax[i].t[2] = C.ax[i].t[2];
     }
-    eval_energy_pass<NT, STAGED>(C, cx, cy, cz, nf, exclude, L, P, outE, outN, outH, outA, ticks);
+    g.r2max = C.r2max;
+    return g;
+}
+__device__ __forceinline__ bool within_lanes(const float c[3], const float4 p, const GroupCut &g)
+{
+    const float d0 = c[0] - p.x, d1 = c[1] - p.y, d2 = c[2] - p.z;
+    const bool far = axis_far(d0, g.ax[0]) | axis_far(d1, g.ax[1]) | axis_far(d2, g.ax[2]);
+    float e0 = axis_near(d0, g.ax[0].L, g.ax[0].t[0], g.ax[0].t[1]);
+    float e1 = axis_near(d1, g.ax[1].L, g.ax[1].t[0], g.ax[1].t[1]);
+    float e2 = axis_near(d2, g.ax[2].L, g.ax[2].t[0], g.ax[2].t[1]);
+    if (__builtin_expect(__ballot(far) != 0ull, 0)) {
+        e0 = axis_delta(c[0], p.x, g.ax[0]);
+        e1 = axis_delta(c[1], p.y, g.ax[1]);
+        e2 = axis_delta(c[2], p.z, g.ax[2]);
+    }
+    return fmaf(e2, e2, fmaf(e1, e1, e0 * e0)) <= g.r2max;
+}
+
+// ---- candidate groups over the cell list --------------------------------------
+// One wave (or, with parts > 1, wave `part` of several that deal the stencil's
+// cells out among themselves): fixed and mobile groups of the stencil cells
+// around the trial centre plus the overflow bucket; kept when gid != exclude and
+// the FP32 distanceP test passes (gcmc_energy.h:152-191).  With two centres (a
+// translation's old and new) a group is kept when it passes either test.
+// Included groups are batched in W (slot -> atoms) for P.run.  Needs L.spt.
+//
+// No barriers: every step is a wave's own.  (With 256 threads per evaluation
+// the barriers between the steps, and the rounds of a step that fill a part of
+// the threads, left a third of the issue slots: 14.5 us per evaluation and
+// workgroup on the 64-system workload.)
+struct ScanSums {
+    int nin[2], nat[2];       // groups and their atoms within the cutoff, per centre (this lane's)
+    uint32_t hash[2];
+};
+
+template <class Pass>
+__device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLds &W, const float c0[3],
+                                            const float c1[3], int ncentre, int exclude, int part, int parts,
+                                            Pass &P, ScanSums &o)
+{
+    CRep &C = fresh(C0);
+    const int lane = fresh_lane();
+    const bool two = ncentre == 2;
+    int home[3];
+    // the centres' positions relative to the first one's cell
+    float base0[3], base1[3], hp[3];
+    cell_coords(C.L, C.start, C.inv_h, C.nc, c0[0], c0[1], c0[2], home);
+    {
+        float u0[3];
+        cell_offset(C.L, C.start, C.cell_h, home, c0[0], c0[1], c0[2], u0);
+        stencil_base(u0, C.cell_h, two ? C.prune_wide : C.prune, base0, hp);
+        for (int i = 0; i < 3; ++i) {
+            const float d = c1[i] - c0[i];
+            base0[i] = uniform_f(base0[i]);
+            base1[i] = hp[i] == 0.0f ? 0.0f : uniform_f(base0[i] + (d - rintf(d * C.invL[i]) * C.L[i]));
+            home[i] = uniform_i(home[i]) - 128;
+        }
+    }
+    const int nst = two ? C.nst_wide : C.nst, ne = nst + 1;
+    int g = 0, A = 0;             // groups and atoms in the batch
+    int b = 0, nl = 0, q0 = 0;    // next stencil entry; cells listed, cells taken from the list
+    int r0 = 0, T = 0;            // candidates of the listed cells at hand: next, total
+    int n = 0, off = 0, fixb = 0, thr = 0, mobb = 0, carry = 0;
+    auto clear_map = [&]() { ((int4 *)W.amap)[lane] = make_int4(0, 0, 0, 0); };
+    clear_map();
+    while (true) {
+        // ---- the next 128 candidates
+        bool done = false;
+        while (r0 >= T) {
+            if (q0 >= nl) {
+                if (b >= ne) {
+                    done = true;
+                    break;
+                }
+                // list the cells that can hold a group within the cutoff
+                constexpr int I = WL_CELLS / 64;
+                CRep &D = fresh(C);
+                const auto stencil = gbl(D.stencil) + (two ? D.nst : 0);
+                const int n0 = D.nc[0], n1 = D.nc[1], n2 = D.nc[2];
+                const float reach2 = D.prune_r2;
+                int code[I];
+#pragma unroll
+                for (int i = 0; i < I; ++i) {
+                    const int e = b + (i * 64 + lane) * parts + part;
+                    code[i] = e < nst ? stencil[e] : 0;
+                }
+                nl = 0;
+#pragma unroll
+                for (int i = 0; i < I; ++i) {
+                    if (b + i * 64 * parts >= ne) continue;
+                    const int e = b + (i * 64 + lane) * parts + part;
+                    // cells whose box lies beyond rc + slack from the centre hold no
+                    // group centre that passes the group test
+                    bool live = stencil_cell_near(code[i], base0, hp, reach2);
+                    if (two) live |= stencil_cell_near(code[i], base1, hp, reach2);
+                    // offsets span at most one box per axis: wrap by one add
+                    auto wrap = [](int q, int nq) {
+                        const unsigned x = min((unsigned)q, (unsigned)(q + nq));
+                        return min(x, x - (unsigned)nq);
+                    };
+                    const unsigned i0 = wrap(home[0] + (code[i] & 255), n0), i1 = wrap(home[1] + (code[i] >> 8 & 255), n1),
+                                   i2 = wrap(home[2] + (code[i] >> 16 & 255), n2);
+                    // at most 255 cells per axis: 24-bit products
+                    int cell = (int)(__umul24(__umul24(i0, n1) + i1, n2) + i2);
+                    live = e < nst ? live : e == nst;     // the last entry: the overflow bucket
+                    cell = e < nst ? cell : D.ncell;
+                    const unsigned long long bal = __ballot(live);
+                    if (live) W.list[nl + rank_below(bal)] = (uint32_t)cell;
+                    nl += __popcll(bal);
+                }
+                b += WL_CELLS * parts;
+                q0 = 0;
+                wave_sync();
+                continue;
+            }
+            // one listed cell per lane: its fixed records and mobile entries
+            int fs = 0, fc = 0, mc = 0;
+            mobb = 0;
+            if (q0 + lane < nl) {
+                CRep &D = fresh(C);
+                const auto cellv = gbl(D.cell);
+                const int cell = (int)W.list[q0 + lane], last = D.ncell;
+                const int2 ci = cellv[cell];
+                const int next = cellv[min(cell + 1, last)].x;   // (the overflow bucket has no fixed records)
+                fs = ci.x;
+                mc = ci.y;
+                fc = next - fs;
+                mobb = cell == last ? D.ovf_base : cell * D.cap;
+            }
+            n = fc + mc;
+            const int incl = wave_scan_add(n);
+            off = incl - n;
+            T = __builtin_amdgcn_readlane(incl, 63);
+            // candidate m of this chunk: record m + fixb below thr, entry m + mobb from thr on
+            fixb = fs - off;
+            thr = off + fc;
+            mobb -= thr;
+            q0 += 64;
+            r0 = 0;
+            carry = 0;
+        }
+        constexpr int R = 2;
+        int2 rr[R];
+        int flag[R], pos[R], at[R], ng = 0, tot = 0;
+        if (!done) {
+            // the cell of each candidate: cells mark their first candidate, a running
+            // maximum carries the mark on
+            ((uint16_t *)W.head)[lane] = 0;
+            wave_sync();
+            if (n > 0 && off >= r0 && off < r0 + 64 * R) W.head[off - r0] = (uint8_t)lane;
+            wave_sync();
+            float4 rec[R];
+            bool fixed[R];
+            CRep &D = fresh(C);
+            const auto fix = gbl(D.fix);
+            const auto mob_rec = gbl(D.mob_rec);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int own = max(wave_scan_max(W.head[r * 64 + lane]), carry);
+                carry = __builtin_amdgcn_readlane(own, 63);
+                const int m = r0 + r * 64 + lane;
+                const int fb = lane_up(fixb, own), th = lane_up(thr, own), mb = lane_up(mobb, own);
+                fixed[r] = m < th;
+                rec[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+                rr[r] = make_int2(0, 0);
+                if (m < T) {
+                    if (fixed[r]) {
+                        rec[r] = fix[m + fb].p;
+                        rr[r] = fix[m + fb].rng;
+                    } else {
+                        rec[r] = mob_rec[m + mb];
+                    }
+                }
+            }
+            const GroupCut cut = group_cut(D);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float4 p = rec[r];
+                const bool valid = r0 + r * 64 + lane < T;
+                int gid = __float_as_int(p.w);
+                if (valid && !fixed[r]) {
+                    const int4 sp = L.spt[gid >> GID_BITS];   // (startRes, maxNum, atomBase, nf)
+                    gid &= GID_MASK;
+                    rr[r] = make_int2(sp.z + (gid - sp.x) * sp.w, sp.w);
+                }
+                const bool able = valid && gid != exclude;
+                const uint32_t h = group_hash((uint32_t)gid);
+                const bool in0 = able && within_lanes(c0, p, cut);
+                const bool in1 = two ? able && within_lanes(c1, p, cut) : in0;
+                o.nin[0] += in0 ? 1 : 0;
+                o.nat[0] += in0 ? rr[r].y : 0;
+                o.hash[0] += in0 ? h : 0u;
+                if (two) {
+                    o.nin[1] += in1 ? 1 : 0;
+                    o.nat[1] += in1 ? rr[r].y : 0;
+                    o.hash[1] += in1 ? h : 0u;
+                }
+                flag[r] = rr[r].y > 0 ? (in0 ? 1 : 0) | (in1 ? 2 : 0) : 0;
+                const unsigned long long bal = __ballot(flag[r] != 0);
+                const int na = flag[r] ? rr[r].y : 0;
+                const int incl = wave_scan_add(na);
+                pos[r] = ng + rank_below(bal);
+                at[r] = tot + incl - na;
+                ng += __popcll(bal);
+                tot += __builtin_amdgcn_readlane(incl, 63);
+            }
+            r0 += 64 * R;
+        }
+        // ---- a full batch goes through the pair pass
+        if (done || g + ng > WL_GROUPS || A + tot > WL_ATOMS) {
+            if (g > 0) {
+                wave_sync();
+                P.run(C, L, W, g, A);
+                wave_sync();
+            }
+            if (done) break;
+            if (g > 0) clear_map();
+            g = 0;
+            A = 0;
+            wave_sync();
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (flag[r]) {
+                const int a = A + at[r];
+                W.goff[g + pos[r]] = a << 2 | flag[r];
+                W.gdel[g + pos[r]] = rr[r].x - a;
+                if (a < WL_ATOMS) W.amap[a] = (uint8_t)(g + pos[r]);
+            }
+        }
+        g += ng;
+        A += tot;
+    }
+}
+
+// ---- a pose, or a trial's two poses, against the environment --------------------
+struct PoseSums {
+    double e[2];
+    int nin[2], nat[2];
+    uint32_t hash[2];
+};
+static_assert(sizeof(PoseSums) <= TEAM_BYTES, "team slots");
+
+// W.frag[s * MAXF + a] (x, y, z, K q) of pose s's atoms -> the copies the pair
+// pass reads, in the order of F.slot (equal types side by side): FP64 relative
+// to the pose's centre, or FP32 absolute.  Lane a of the pose's wave.
+template <int TM>
+__device__ __forceinline__ void order_pose(CRep &C, CSpecies &F, const WaveLds &W, int s, int a, const float4 q,
+                                           const float c[3])
+{
+    W.frag[s * MAXF + a] = q;
+    const int i = s * MAXF + F.slot[a];
+    if (TM == T_FP64)
+        W.fragd[i] = make_double4((double)q.x - (double)c[0], (double)q.y - (double)c[1], (double)q.z - (double)c[2],
+                                  (double)q.w);
+    else
+        ((float4 *)(W.fragd + s * MAXF))[F.slot[a]] = q;
+}
+
+// Energies of the nset poses in W around centres c0 and c1 (equal for a
+// rotation), by one wave or its part of the cells; uniform results.
+// pose_near: the poses were generated from the species template or the
+// molecule's atoms (within the species' extent of the centre, the bound
+// Rep::nowrap rests on); poses given by a caller take the per-pair image shift.
+template <bool STAGED, int TM>
+__device__ __forceinline__ void eval_poses_wave(CRep &C, const Lds &L, const WaveLds &W, int spi, int nf, int nset,
+                                                const float c0[3], const float c1[3], bool same_centre, int exclude,
+                                                bool pose_near, int part, int parts, PoseSums &out)
+{
+    EnergyPass<STAGED, TM> P;
+    for (int i = 0; i < 2; ++i) P.acc[i] = 0.0;
+    P.x[0] = c0[0]; P.y[0] = c0[1]; P.z[0] = c0[2];
+    P.x[1] = c1[0]; P.y[1] = c1[1]; P.z[1] = c1[2];
+    P.wrap = !(pose_near && C.nowrap != 0);
+    P.spi = spi;
+    P.nf = nf;
+    ScanSums o{};
+    // two centres in one scan when the stencil is wide enough for both
+    const bool both = nset == 1 || same_centre || C.nst_wide > 0;
+    P.first = 0;
+    P.nset = both ? nset : 1;
+    for (int pass = 0; pass < (both ? 1 : 2); ++pass) {
+        ScanSums q{};
+        P.first = pass;
+        scan_groups(C, L, W, pass ? c1 : c0, c1, nset == 2 && both && !same_centre ? 2 : 1, exclude, part, parts, P, q);
+        if (pass == 0) o = q;
+        else {
+            o.nin[1] = q.nin[0];
+            o.nat[1] = q.nat[0];
+            o.hash[1] = q.hash[0];
+        }
+    }
+    if (nset == 2 && same_centre) {
+        o.nin[1] = o.nin[0];
+        o.nat[1] = o.nat[0];
+        o.hash[1] = o.hash[0];
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        out.e[s] = lane_d(wave_scan_add(P.acc[s]), 63);
+        out.nin[s] = __builtin_amdgcn_readlane(wave_scan_add(o.nin[s]), 63);
+        out.nat[s] = __builtin_amdgcn_readlane(wave_scan_add(o.nat[s]), 63);
+        out.hash[s] = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(o.hash[s]), 63);
+    }
 }
 
 __device__ inline uint32_t pose_hash(const float4 *p, int nf)
@@ -731,131 +920,133 @@ __device__ inline void count_add(T *p, T v)
     else __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// statistics of one evaluation (counters of the replica's State)
+// statistics of a wave's evaluations (counters of the replica's State), added
+// up in registers and published once per claim
 struct ItemStats {
-    unsigned long long ticks[4];
-    unsigned long long nat, nin, nf;
+    unsigned ticks[2];   // poses and adjacency, scan and pair passes
+    unsigned nat, nin, neval, nfat;
 };
 
 template <bool LOCAL>
-__device__ inline void add_item_stats(State &W, const ItemStats &s)
+__device__ inline void add_item_stats(State &W, const ItemStats &s, int nf)
 {
-    for (int i = 0; i < 4; ++i) count_add<LOCAL>(&W.t_sub[i], s.ticks[i]);
-    count_add<LOCAL>(&W.n_eval, 1ull);
-    count_add<LOCAL>(&W.n_pair, s.nat * s.nf);
-    count_add<LOCAL>(&W.n_atom, s.nat);
-    count_add<LOCAL>(&W.n_group, s.nin);
-    count_add<LOCAL>(&W.n_fatom, s.nf);
+    count_add<LOCAL>(&W.t_sub[0], (unsigned long long)s.ticks[0]);
+    count_add<LOCAL>(&W.t_sub[3], (unsigned long long)s.ticks[1]);
+    count_add<LOCAL>(&W.n_eval, (unsigned long long)s.neval);
+    count_add<LOCAL>(&W.n_pair, (unsigned long long)s.nat * nf);
+    count_add<LOCAL>(&W.n_atom, (unsigned long long)s.nat);
+    count_add<LOCAL>(&W.n_group, (unsigned long long)s.nin);
+    count_add<LOCAL>(&W.n_fatom, (unsigned long long)s.nfat);
 }
 
 // ---- Ewald reciprocal term of a pose ------------------------------------------
-// sum_f q_f phi(x_f) over the pose held in L.frag, phi the PME potential of the
-// current state.  When the molecule itself is in that state (base >= 0: its
+// sum_f q_f phi(x_f) over the pose in W.frag (set s), phi the PME potential of
+// the current state.  When the molecule itself is in that state (base >= 0: its
 // atoms y_g at C.atom[base..]), its own share of phi -- what the grid holds
 // for its charges, periodic images and neutralising background included --
 // is removed: sum_{f,g} q_f q_g Kgrid(x_f, y_g) (pme_spline.h).  What remains
 // is the reciprocal interaction with every other charge; for a rigid
 // molecule the Ewald self, intramolecular and self-image terms are constants
-// of the species, left out alike on insertion and deletion.  Called by every
-// thread; thread 0 gets the sum.
-template <int NT>
-__device__ inline double ewald_recip(CRep &C, CSpecies &F, const Lds &L, int nf, int base)
+// of the species, left out alike on insertion and deletion.  One wave (or its
+// part); every lane gets its sum.
+__device__ inline double ewald_recip(CRep &C, CSpecies &F, const WaveLds &W, int s, int nf, int base, int part,
+                                     int parts)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lane = threadIdx.x & 63;
     double v = 0.0;
-    if (tid < nf) {
-        const float4 x = L.frag[tid];
-        v = (double)F.tmpl[tid].w * (double)gcmc_spline::gather(C.pme_phi, C.pk, C.L, x.x, x.y, x.z);
+    const int K[3] = {C.pk[0], C.pk[1], C.pk[2]};
+    const float Lb[3] = {C.L[0], C.L[1], C.L[2]};
+    const int f0 = lane * parts + part;
+    if (f0 < nf) {
+        const float4 x = W.frag[s * MAXF + f0];
+        v = (double)F.tmpl[f0].w * (double)gcmc_spline::gather(C.pme_phi, K, Lb, x.x, x.y, x.z);
     }
     if (base >= 0) {
         const int nw = nf * nf * 7;
-        for (int w = tid; w < nw; w += NT) {
+        for (int w = part * 64 + lane; w < nw; w += 64 * parts) {
             const int f = w / (7 * nf), g = (w / 7) % nf, j0 = w % 7;
-            const float4 xf = L.frag[f];
+            const float4 xf = W.frag[s * MAXF + f];
             const float4 yg = C.atom[base + g];
             const float xv[3] = {xf.x, xf.y, xf.z}, yv[3] = {yg.x, yg.y, yg.z};
-            const float kv = gcmc_spline::pair_kernel_slab(C.pme_gk, C.pk, C.L, xv, yv, j0);
+            const float kv = gcmc_spline::pair_kernel_slab(C.pme_gk, K, Lb, xv, yv, j0);
             v -= (double)F.tmpl[f].w * (double)F.tmpl[g].w * (double)kv;
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    if (lane == 0) L.dred[wave] = v;
-    __syncthreads();
-    double t = 0.0;
-    if (tid == 0)
-        for (int q = 0; q < NT / 64; ++q) t += L.dred[q];
-    __syncthreads();
-    return t;
+    return lane_d(wave_scan_add(v), 63);
 }
 
-// ---- one trial evaluation ----------------------------------------------------
-// item < k: trial item (insert/delete) or E_old (translate/rotate);
-// item >= k: E_new of trial item-k (translate/rotate).
-template <int NT, bool STAGED, bool LOCAL, bool EW>
-// Thread 0 adds the statistics to S, or leaves them in *defer (thread 0's
-// copy) for the caller to add once the item's completion is published.
-__device__ inline void eval_item(CRep &C, const State &S, int item, const Lds &L, bool stage_rep = true,
-                                 bool stage_tab = true, ItemStats *defer = nullptr)
+// ---- one trial -----------------------------------------------------------------
+// A move's items are its trials: an insertion's or deletion's pose, or a
+// translation's or rotation's old and new pose in one pass over the neighbourhood.
+// A move of at most COOP_TRIALS trials is on its replica's critical path: its
+// trials' cells are shared by four waves.  In larger moves every trial is one
+// wave's.  The rule depends on the move alone: every form sums a pose's energy in
+// the same order.
+constexpr int COOP_TRIALS = 100, COOP = 4;
+
+struct Move {
+    int kind, spi, k, step, nset, nitems;   // nset: poses per trial
+    bool coop;
+};
+
+__device__ __forceinline__ Move make_move(int kind, int spi, int k, int step)
 {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    Move m;
+    m.kind = uniform_i(kind);
+    m.spi = uniform_i(spi);
+    m.k = uniform_i(k);
+    m.step = uniform_i(step);
+    m.nitems = m.k;
+    m.nset = m.kind >= K_TRN ? 2 : 1;
+    m.coop = m.k <= COOP_TRIALS;
+    return m;
+}
+__device__ __forceinline__ Move move_of(const State &S) { return make_move(S.kind, S.sp, S.k, S.step); }
+
+// Wave `part` of `parts`: the poses of trial t (0: the old one, or an insertion's
+// or deletion's only one, 1: the new one), its share of the adjacency row and of
+// the energies.
+template <bool STAGED, int TM>
+__device__ __forceinline__ void trial_wave(CRep &C0, const Move &mv, int t, int part, int parts, const Lds &L,
+                                           const WaveLds &W, PoseSums &out, ItemStats &st)
+{
+    CRep &C = fresh(C0);
+    const int lane = fresh_lane();
     const unsigned long long tq0 = wall_clock64();
-    const int kind = S.kind, spi = S.sp, k = S.k, step = S.step;
-    CSpecies &F = species_of(C, spi);
+    const int kind = mv.kind, k = mv.k, step = mv.step;
+    CSpecies &F = species_of(C, mv.spi);
     const int nf = F.nf;
     const auto tc = gbl(C.tc);
     const auto atom = gbl(C.atom);
-    // translate / rotate: item 2t is trial t's old pose, 2t + 1 its new pose;
-    // a claim of consecutive items evaluates both, the second reading the
-    // neighbourhood the first left in L1
-    int t = item, phase = 0;
-    if (kind >= K_TRN) {
-        t = item >> 1;
-        phase = item & 1;
-    }
-    // the species table stays in LDS while a workgroup keeps evaluating
-    // items of one replica (stage_rep = false), the pair table while it
-    // keeps evaluating items of replicas with that table (stage_tab = false)
-    if (stage_rep) load_species_table(C, L);
-    // the pair table is copied without a wait here: the pose, stencil and
-    // candidate work runs meanwhile, and the wait is before the first pair
-    // pass (eval_energy_pass)
-    if (STAGED && stage_tab) stage_pair_table<NT>(C, L);
-    const float4 tcv = tc[t];
-    const int slot = (kind == K_INS) ? -1 : gbl(C.tslot)[t];
+    const float4 tcl = tc[t];
+    const int slot = (kind == K_INS) ? -1 : uniform_i(gbl(C.tslot)[t]);
     const int gid = (kind == K_INS) ? -1 : F.startRes + slot;
-    const float4 cold = (gid >= 0) ? gbl(C.res_pos)[gid] : make_float4(0.f, 0.f, 0.f, 0.f);
-    float cx, cy, cz;
-    if (kind == K_INS || phase == 1 || kind == K_DEL) {
-        cx = tcv.x; cy = tcv.y; cz = tcv.z;
-    } else {
-        cx = cold.x; cy = cold.y; cz = cold.z;
+    const float cn[3] = {uniform_f(tcl.x), uniform_f(tcl.y), uniform_f(tcl.z)};
+    float co[3] = {cn[0], cn[1], cn[2]};
+    if (kind >= K_TRN) {
+        const float4 cold = gbl(C.res_pos)[gid];
+        co[0] = uniform_f(cold.x);
+        co[1] = uniform_f(cold.y);
+        co[2] = uniform_f(cold.z);
     }
-    const bool newpose = (kind == K_INS) || (kind == K_DEL) || (phase == 1);
-    // the first block of trial centres for the adjacency row below, loaded
-    // now so the load overlaps the pose work
-    const bool adjrow = kind != K_DEL && phase == 0;
-    float4 cj0 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (adjrow && tid < k) cj0 = tc[tid];
-    if (tid < nf) {
-        const int a = tid;
+    if (lane < nf) {
+        const int a = lane;
         const float4 tm = F.tmpl[a];
+        const float kq = F.kq[a];
         float px, py, pz;
         if (kind == K_INS) {
             const u32x4 y = draw(C.seed, (uint32_t)step, (uint32_t)t, P_ROTATION);
             float R[9], v[3];
             rotation_matrix(u01f(y.x), u01f(y.y), u01f(y.z), u01f(y.w) * 0x1.921fb6p+2f, R);
             rotate(R, tm.x, tm.y, tm.z, v);
-            px = v[0] + cx; py = v[1] + cy; pz = v[2] + cz;
+            px = v[0] + cn[0]; py = v[1] + cn[1]; pz = v[2] + cn[2];
         } else {
             const int base = F.atomBase + slot * nf;
             const float4 cur = atom[base + a];
-            if (kind == K_DEL || phase == 0) {
-                px = cur.x; py = cur.y; pz = cur.z;
-            } else if (kind == K_TRN) {
+            order_pose<TM>(C, F, W, 0, a, make_float4(cur.x, cur.y, cur.z, kq), co);
+            if (kind == K_TRN) {
                 const u32x4 x = draw(C.seed, (uint32_t)step, (uint32_t)t, P_JITTER);
                 const float u[3] = {u01f(x.x), u01f(x.y), u01f(x.z)};
-                const float co[3] = {cold.x, cold.y, cold.z};
                 float r[3];
                 for (int i = 0; i < 3; ++i) {
                     float d = u[i] * C.dx;
@@ -864,14 +1055,16 @@ __device__ inline void eval_item(CRep &C, const State &S, int item, const Lds &L
                     r[i] = d;
                 }
                 px = cur.x + r[0]; py = cur.y + r[1]; pz = cur.z + r[2];
-            } else {
-                float cen0 = 0.f, cen1 = 0.f, cen2 = 0.f;
+            } else if (kind == K_ROT) {
+                // each lane divides its own atom's coordinates, the sums run in
+                // atom order
                 const float fn = (float)nf;
+                const float s0 = cur.x / fn, s1 = cur.y / fn, s2 = cur.z / fn;
+                float cen0 = 0.f, cen1 = 0.f, cen2 = 0.f;
                 for (int b = 0; b < nf; ++b) {
-                    const float4 q = atom[base + b];
-                    cen0 = cen0 + q.x / fn;
-                    cen1 = cen1 + q.y / fn;
-                    cen2 = cen2 + q.z / fn;
+                    cen0 = cen0 + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s0), b));
+                    cen1 = cen1 + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s1), b));
+                    cen2 = cen2 + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s2), b));
                 }
                 const u32x4 y = draw(C.seed, (uint32_t)step, (uint32_t)t, P_ROTATION);
                 float R[9], v[3];
@@ -880,64 +1073,135 @@ __device__ inline void eval_item(CRep &C, const State &S, int item, const Lds &L
                 px = v[0] + cen0; py = v[1] + cen1; pz = v[2] + cen2;
             }
         }
-        L.frag[a] = make_float4(px, py, pz, F.kq[a]);
-        L.frow[a] = F.trow[a];
-        if (kind == K_INS || phase == 1) gbl(C.pose)[t * MAXF + a] = make_float4(px, py, pz, 0.f);
+        if (kind != K_DEL) {
+            order_pose<TM>(C, F, W, kind == K_INS ? 0 : 1, a, make_float4(px, py, pz, kq), cn);
+            if (part == 0) gbl(C.pose)[t * MAXF + a] = make_float4(px, py, pz, 0.f);
+        }
+    }
+    wave_sync();
+    // adjacency row of trial t over the trial centres (grouping of the accept
+    // phase), the loads of four blocks of 64 at a time
+    if (kind != K_DEL) {
+        constexpr int B = 4;
+        const GroupCut cut = group_cut(C);
+        for (int j0 = part * 64; j0 < k; j0 += B * 64 * parts) {
+            float4 cj[B];
+#pragma unroll
+            for (int q = 0; q < B; ++q) {
+                const int j = j0 + q * 64 * parts + lane;
+                cj[q] = tc[min(j, k - 1)];
+            }
+#pragma unroll
+            for (int q = 0; q < B; ++q) {
+                const int jq = j0 + q * 64 * parts, j = jq + lane;
+                if (jq >= k) break;
+                const bool b = within_lanes(cn, cj[q], cut) && j < k && j != t;
+                const unsigned long long bal = __ballot(b);
+                if (lane == 0) {
+                    const int wi = jq >> 5;
+                    gbl(C.adj)[t * ADJW + wi] = (uint32_t)bal;
+                    gbl(C.adj)[t * ADJW + wi + 1] = (uint32_t)(bal >> 32);
+                }
+            }
+        }
+    }
+    const unsigned long long tq1 = wall_clock64();
+    // a rotation keeps the centre
+    eval_poses_wave<STAGED, TM>(C, L, W, mv.spi, nf, mv.nset, co, cn, kind != K_TRN, gid, true, part, parts, out);
+    if (TM == T_EWALD) {
+        // the moving molecule (delete, translate, rotate) is in the PME grid
+        const int base = kind == K_INS ? -1 : F.atomBase + slot * nf;
+        out.e[0] += ewald_recip(C, F, W, 0, nf, base, part, parts);
+        if (mv.nset == 2) out.e[1] += ewald_recip(C, F, W, 1, nf, base, part, parts);
+    }
+    const unsigned long long tq2 = wall_clock64();
+    st.ticks[0] += (unsigned)(tq1 - tq0);
+    st.ticks[1] += (unsigned)(tq2 - tq1);
+}
+
+// energies of a trial to the replica's buffers, statistics, trace (one lane)
+__device__ inline void finish_trial(CRep &C, const Move &mv, int t, const WaveLds &W, const PoseSums &r, ItemStats &st)
+{
+    CSpecies &F = species_of(C, mv.spi);
+    const int nf = F.nf;
+    const bool two = mv.nset == 2;
+    const auto E = gbl(C.E);
+    E[t] = r.e[0];
+    if (two) E[mv.k + t] = r.e[1];
+    st.nat += (unsigned)(r.nat[0] + (two ? r.nat[1] : 0));
+    st.nin += (unsigned)(r.nin[0] + (two ? r.nin[1] : 0));
+    st.neval += mv.nset;
+    st.nfat += mv.nset * nf;
+    int row;
+    if (tracing(C, mv.step, row) && t < C.tr.max_k) {
+        const int q = row * C.tr.max_k + t;
+        for (int s = 0; s < mv.nset; ++s) {
+            C.tr.e[2 * q + s] = s ? r.e[1] : r.e[0];
+            C.tr.ninc[2 * q + s] = s ? r.nin[1] : r.nin[0];
+            C.tr.inchash[2 * q + s] = s ? r.hash[1] : r.hash[0];
+        }
+        const float4 tcv = gbl(C.tc)[t];
+        C.tr.posehash[q] = pose_hash(W.frag + (mv.nset - 1) * MAXF, nf);
+        C.tr.centre[3 * q + 0] = tcv.x;
+        C.tr.centre[3 * q + 1] = tcv.y;
+        C.tr.centre[3 * q + 2] = tcv.z;
+        C.tr.idx[q] = mv.kind == K_INS ? -1 : gbl(C.tslot)[t];
+    }
+}
+
+// four waves' shares of one pose (or two), added up in wave order; W's wave 0
+// of the team gets the sums.  Two barriers of the whole workgroup.
+template <int NT>
+__device__ __forceinline__ void team_sum(const Lds &L, PoseSums &r)
+{
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    auto slot = [&](int w) { return (PoseSums *)((char *)L.team + w * TEAM_BYTES); };
+    if (lane == 0) *slot(wave) = r;
+    __syncthreads();
+    if (wave % COOP == 0 && lane == 0) {
+        for (int w = 1; w < COOP; ++w) {
+            const PoseSums q = *slot(wave + w);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                r.e[s] += q.e[s];
+                r.nin[s] += q.nin[s];
+                r.nat[s] += q.nat[s];
+                r.hash[s] += q.hash[s];
+            }
+        }
     }
     __syncthreads();
+}
 
-    // adjacency row of trial t over the trial centres (grouping of the accept phase)
-    if (adjrow) {
-        for (int j0 = 0; j0 < k; j0 += NT) {
-            const int j = j0 + tid;
-            bool b = false;
-            if (j < k && j != t) {
-                const float4 cj = (j0 == 0) ? cj0 : tc[j];
-                b = within(tcv.x, tcv.y, tcv.z, cj.x, cj.y, cj.z, C.ax, C.r2max);
-            }
-            const unsigned long long bal = __ballot(b);
-            if (lane == 0) {
-                const int wi = (j0 + wave * 64) >> 5;
-                if (wi < ADJW) gbl(C.adj)[t * ADJW + wi] = (uint32_t)bal;
-                if (wi + 1 < ADJW) gbl(C.adj)[t * ADJW + wi + 1] = (uint32_t)(bal >> 32);
-            }
+// cnt trials from `item` on by the whole workgroup: teams of four waves, or the
+// waves each on their own, taking the next trial from L.misc[M_NEXT] (0 on
+// entry, written before a barrier)
+template <int NT, bool STAGED, int TM>
+__device__ __forceinline__ void eval_items(CRep &C, const Move &mv, int item, int cnt, const Lds &L, ItemStats &st)
+{
+    constexpr int NW = NT / 64, TEAMS = NW / COOP;
+    const int wave = fresh_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const WaveLds W = wave_lds(L, wave);
+    // one call site: the trial's code is long
+    int j0 = 0;
+    while (true) {
+        int j;
+        if (mv.coop) {
+            if (j0 >= cnt) break;
+            j = j0 + wave / COOP;
+            j0 += TEAMS;
+        } else {
+            j = 0;
+            if (lane == 0) j = atomicAdd(&L.misc[M_NEXT], 1);
+            j = uniform_i(j);
+            if (j >= cnt) break;
         }
-    }
-
-    double E;
-    int nin, nat;
-    uint32_t hh;
-    unsigned long long ticks[4];
-    ticks[0] = wall_clock64() - tq0;
-    eval_energy<NT, STAGED, EW>(C, cx, cy, cz, nf, gid, L, &E, &nin, &hh, &nat, ticks, true);
-    if (EW) {
-        // the moving molecule (delete, translate, rotate) is in the PME grid
-        const double er = ewald_recip<NT>(C, F, L, nf, kind == K_INS ? -1 : F.atomBase + slot * nf);
-        if (tid == 0) E += er;
-    }
-    if (tid == 0) {
-        gbl(C.E)[phase * k + t] = E;
-        ItemStats st;
-        for (int i = 0; i < 4; ++i) st.ticks[i] = ticks[i];
-        st.nat = (unsigned long long)nat;
-        st.nin = (unsigned long long)nin;
-        st.nf = (unsigned long long)nf;
-        if (defer) *defer = st;
-        else add_item_stats<LOCAL>(const_cast<State &>(S), st);
-        int row;
-        if (tracing(C, step, row) && t < C.tr.max_k) {
-            const int q = row * C.tr.max_k + t;
-            C.tr.e[2 * q + phase] = E;
-            C.tr.ninc[2 * q + phase] = nin;
-            C.tr.inchash[2 * q + phase] = hh;
-            if (newpose) {
-                C.tr.posehash[q] = pose_hash(L.frag, nf);
-                C.tr.centre[3 * q + 0] = tcv.x;
-                C.tr.centre[3 * q + 1] = tcv.y;
-                C.tr.centre[3 * q + 2] = tcv.z;
-                C.tr.idx[q] = slot;
-            }
-        }
+        const int t = item + min(j, cnt - 1), part = mv.coop ? wave % COOP : 0, parts = mv.coop ? COOP : 1;
+        PoseSums r;
+        trial_wave<STAGED, TM>(C, mv, t, part, parts, L, W, r, st);
+        if (mv.coop) team_sum<NT>(L, r);
+        if (lane == 0 && part == 0 && j < cnt) finish_trial(C, mv, t, W, r, st);
+        wave_sync();
     }
 }
 
@@ -992,7 +1256,7 @@ __device__ inline void cell_rename(CRep &C, int from, int to)
     C.mob_loc[from] = -1;
 }
 
-// ---- selection and Metropolis (one wave) --------------------------------------
+// ---- selection and Metropolis --------------------------------------------------
 // Greedy grouping in ascending trial order: leader = first unused trial,
 // members = unused trials within the cutoff of the leader; Boltzmann weights
 // relative to the group minimum; cumulative pick; acceptance
@@ -1000,10 +1264,7 @@ __device__ inline void cell_rename(CRep &C, int from, int to)
 //   move:    min(1, 1/(m P) exp(-beta dE))             (gcmc_move_trn.h:215-222)
 // On accept the unused trials within the cutoff of the pick are dropped.
 // Trial values are staged in L.val, adjacency rows in L.adjl (when the layout
-// has room; else read from C.adj).  The weight sum and the cumulative pick
-// are wave-parallel: lane l sums a contiguous chunk of the members in order,
-// the chunk sums are scanned across lanes, and the lane whose chunk holds
-// the crossing walks it -- one fixed FP64 summation order.
+// has room; else read from C.adj).
 __device__ inline uint32_t adj_word(CRep &C, const Lds &L, int nw, int t, int w)
 {
     return L.adjl ? L.adjl[t * nw + w] : C.adj[t * ADJW + w];
@@ -1052,127 +1313,203 @@ __device__ inline void load_next_move(CRep &C, const State &S, const Lds &L, con
     L.misc[M_NX + 5] = F.startRes;
 }
 
-__device__ inline void greedy_select(CRep &C, State &S, const Lds &L, int row, bool trace, const MoveCtx &mc)
+// FP64 keys whose unsigned order is the values' order
+__device__ inline unsigned long long order_key(double v)
 {
-    const int lane = threadIdx.x & 63;
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    return b >> 63 ? ~b : b | 0x8000000000000000ull;
+}
+__device__ inline double key_value(unsigned long long k)
+{
+    return __longlong_as_double((long long)(k >> 63 ? k & 0x7fffffffffffffffull : ~k));
+}
+
+// Moves of more than 64 trials.  The groups depend on each other only through
+// acceptances, so they are settled in batches as if none were: wave 0 forms a
+// batch's groups (bit operations only), the workgroup computes the members'
+// weights, and one lane per group sums them in trial order, picks and decides.
+// An accepted pick drops its neighbours from the later groups: the groups before
+// the first one that loses a member stand, the next batch starts there.  Batches
+// grow from 8 to SEL_GROUPS groups while all of them stand and shrink to the pace
+// at which they do not.
+// (One wave taking the groups one after another, weights included, spent
+// 1.3 us on each.)
+template <int NT>
+__device__ inline void select_groups(CRep &C, State &S, const Lds &L, int row, bool trace, const MoveCtx &mc)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kind = mc.kind, k = mc.k;
     const bool ins = kind == K_INS;
     const int nw = (k + 31) >> 5;
+    // wave 0: lane w holds the unused trials 32 w .. 32 w + 31
     uint32_t u = 0u;
     if (lane < nw) {
         const int hi = k - lane * 32;
         u = hi >= 32 ? 0xffffffffu : ((1u << hi) - 1u);
     }
-    int N = mc.N;
+    int N = mc.N, g0 = 0, na = 0, most = 8;
     const int maxN = mc.maxN;
-    const double cav = (double)C.cav;
-    int g = 0, na = 0;
+    const double cav = (double)C.cav, B = ins ? mc.B : 0.0;
     double et = mc.energy;
+    if (wave == 1) L.gmin[lane] = ~0ull;
     while (true) {
-        const unsigned long long bal = __ballot(u != 0u);
-        if (bal == 0ull) break;
-        const int f = __ffsll((long long)bal) - 1;
-        const uint32_t wf = __shfl(u, f, 64);
-        const int it = f * 32 + __ffs(wf) - 1;
-        uint32_t m = (lane < nw) ? (adj_word(C, L, nw, it, lane) & u) : 0u;
-        if (lane == (it >> 5)) m |= 1u << (it & 31);
-        u &= ~m;
-        const int cnt = __popc(m);
-        const int x = wave_scan_add(cnt);
-        const int mtot = __builtin_amdgcn_readlane(x, 63);
-        int o = x - cnt;
-        uint32_t mm = m;
-        while (mm) {
-            const int b = __ffs(mm) - 1;
-            mm &= mm - 1u;
-            L.members[o++] = lane * 32 + b;
-        }
-        wave_sync();
-        const double ran_sel = L.rsel[g];
-        const double ran_acc = L.racc[g];
-        int pick = it, pq = 0;
-        double sumP = 1.0, P = 1.0;
-        if (mtot > 1) {
-            double emin = __builtin_huge_val();
-            for (int q = lane; q < mtot; q += 64) {
-                const double v = L.val[L.members[q]];
-                emin = v < emin ? v : emin;
+        uint32_t v = u;
+        if (wave == 0) {
+            int n = 0, base = 0;
+            // the first unused trial and its row of the adjacency matrix
+            auto leader = [&](int &it, int &f, uint32_t &rw) {
+                const unsigned long long bal = __ballot(v != 0u);
+                if (bal == 0ull) return false;
+                f = __ffsll((long long)bal) - 1;
+                it = f * 32 + __ffs(__builtin_amdgcn_readlane((int)v, f)) - 1;
+                rw = lane < nw ? adj_word(C, L, nw, it, lane) : 0u;
+                return true;
+            };
+            int it = 0, f = 0;
+            uint32_t rw = 0u;
+            bool more = leader(it, f, rw);
+            while (more && n < most) {
+                uint32_t m = rw & v;
+                if (lane == f) m |= 1u << (it & 31);
+                v &= ~m;
+                more = leader(it, f, rw);   // its row arrives while this group is stored
+                const int cnt = __popc(m), incl = wave_scan_add(cnt);
+                if (lane < nw) {
+                    L.gmask[n * nw + lane] = m;
+                    L.goff[n * nw + lane] = (uint16_t)(base + incl - cnt);
+                }
+                if (lane == 0) L.gstart[n] = base;
+                base += __builtin_amdgcn_readlane(incl, 63);
+                ++n;
             }
-            emin = wave_min(emin);
-            for (int q = lane; q < mtot; q += 64) L.w[q] = exp(-BETA * (L.val[L.members[q]] - emin));
-            wave_sync();
-            // chunk sums in member order, scanned across lanes
-            const int per = (mtot + 63) >> 6;
-            const int q0 = min(lane * per, mtot), q1 = min(q0 + per, mtot);
-            double part = 0.0;
-            for (int q = q0; q < q1; ++q) part += L.w[q];
-            const double incl = wave_scan_add(part);
-            sumP = lane_d(incl, 63);
-            if (sumP != 0.0) {
-                // first member q with sum_{j<=q} w_j > ran_sel * sumP (the last one
-                // when rounding leaves the target at the total)
-                const double target = ran_sel * sumP;
-                const double excl = incl - part;
-                const unsigned long long hit = __ballot(q1 > q0 && excl <= target && target < incl);
-                int sel = mtot - 1;
-                if (hit) {
-                    const int l = __ffsll((long long)hit) - 1;
-                    int found = q1 - 1;
-                    if (lane == l) {
-                        double c = excl;
-                        for (int q = q0; q < q1; ++q) {
-                            c += L.w[q];
-                            if (target < c) {
-                                found = q;
-                                break;
-                            }
+            if (lane == 0) {
+                L.gstart[n] = base;
+                L.misc[M_GN] = n;
+            }
+        }
+        __syncthreads();
+        const int n = uniform_i(L.misc[M_GN]);
+        if (n == 0) break;
+        const int total = uniform_i(L.gstart[n]);
+        // the batch's trials in group and trial order, and each group's lowest
+        // value (NaN counts for none)
+        for (int q = tid; q < n * nw; q += NT) {
+            uint32_t m = L.gmask[q];
+            if (m == 0u) continue;
+            const int g = q / nw, t0 = (q - g * nw) * 32;
+            int o = L.goff[q];
+            for (; m; m &= m - 1u) {
+                const int t = t0 + __ffs(m) - 1;
+                const double x = L.val[t];
+                L.members[o++] = t | g << 16;
+                if (x == x) atomicMin(&L.gmin[g], order_key(x));
+            }
+        }
+        __syncthreads();
+        for (int p = tid; p < total; p += NT) {
+            const int e = L.members[p];
+            const unsigned long long key = L.gmin[e >> 16];
+            const double emin = key == ~0ull ? __builtin_huge_val() : key_value(key);
+            L.w[p] = exp(-BETA * (L.val[e & 0xffff] - emin));
+        }
+        __syncthreads();
+        if (wave == 1) L.gmin[lane] = ~0ull;
+        if (wave == 0) {
+            // lane g: group g0 + g
+            int pick = 0, rec = 0;
+            double ea = 0.0, cp = 0.0, ran_acc = 1.0;
+            if (lane < n) {
+                const int s = L.gstart[lane], e = L.gstart[lane + 1], cnt = e - s;
+                const u32x4 xr = draw(C.seed, (uint32_t)mc.step, (uint32_t)(g0 + lane), P_DECIDE);
+                const double ran_sel = u01d(xr.x, xr.y);
+                ran_acc = u01d(xr.z, xr.w);
+                double sum = 0.0, P = 1.0;
+                for (int p = s; p < e; p += 4) {
+                    const double w0 = L.w[p], w1 = L.w[min(p + 1, e - 1)], w2 = L.w[min(p + 2, e - 1)],
+                                 w3 = L.w[min(p + 3, e - 1)];
+                    sum += w0;
+                    sum += p + 1 < e ? w1 : 0.0;
+                    sum += p + 2 < e ? w2 : 0.0;
+                    sum += p + 3 < e ? w3 : 0.0;
+                }
+                int at = s;
+                if (cnt > 1 && sum != 0.0) {
+                    // first member with sum_{j<=q} w_j > ran_sel * sum (the last one
+                    // when rounding leaves the target at the total)
+                    const double target = ran_sel * sum;
+                    double c = 0.0;
+                    at = e - 1;
+                    for (int p = s; p < e; p += 2) {
+                        const double w0 = L.w[p], w1 = L.w[min(p + 1, e - 1)];
+                        c += w0;
+                        if (target < c) {
+                            at = p;
+                            break;
+                        }
+                        c += w1;
+                        if (target < c) {
+                            at = min(p + 1, e - 1);
+                            break;
                         }
                     }
-                    sel = __shfl(found, l, 64);
+                    P = L.w[at] / sum;
                 }
-                pq = sel;
-                pick = L.members[sel];
+                pick = L.members[at] & 0xffff;
+                ea = exp(B - BETA * L.val[pick]);
+                cp = (ins ? cav : 1.0) / ((double)cnt * P);
             }
-            P = sumP != 0.0 ? L.w[pq] / sumP : 1.0;
-        }
-        // (a single-member group has weight exp(0) = 1: pick = leader, P = 1)
-        const double vp = L.val[pick];
-        double pp;
-        if (ins)
-            pp = (cav / ((double)mtot * P)) / ((double)N + 1.0) * L.ea[pick];
-        else
-            pp = (1.0 / ((double)mtot * P)) * L.ea[pick];
-        const double p = pp < 1.0 ? pp : 1.0;
-        const bool acc = ran_acc < p;
-        int rec = acc ? 1 : 0;
-        if (acc) {
-            const uint32_t ap = (lane < nw) ? adj_word(C, L, nw, pick, lane) : 0u;
-            u &= ~ap;
-            if (ins) {
-                if (N < maxN) {
-                    if (lane == 0) L.accl[na] = make_int2(pick, N);
-                    N += 1;
+            auto decide = [&]() {
+                const double pp = ins ? cp / ((double)N + 1.0) * ea : cp * ea;
+                const double p = pp < 1.0 ? pp : 1.0;
+                return __ballot(lane < n && ran_acc < p);
+            };
+            unsigned long long am = decide();
+            int stand = n;
+            uint32_t drop = 0u;   // lane w: neighbours of the accepted picks
+            while (am != 0ull) {
+                const int g = __ffsll((long long)am) - 1;
+                const int ap = __builtin_amdgcn_readlane(pick, g);
+                if (lane < nw) {
+                    drop |= adj_word(C, L, nw, ap, lane);
+                    L.drop[lane] = drop;
+                }
+                if (lane == g) rec = ins && N >= maxN ? 2 : 1;
+                if (!(ins && N >= maxN)) {
+                    if (lane == 0) L.accl[na] = make_int2(ap, ins ? N : C.tslot[ap]);
+                    N += ins ? 1 : 0;
                     na += 1;
-                    et += vp;
-                } else {
-                    rec = 2;
+                    et += L.val[ap];
+                    if (ins) am = decide();
                 }
-            } else {
-                if (lane == 0) L.accl[na] = make_int2(pick, C.tslot[pick]);
-                na += 1;
-                et += vp;
+                // the first later group that loses a member
+                bool hit = false;
+                if (lane > g && lane < stand)
+                    for (int w = 0; w < nw; ++w) hit |= (L.gmask[lane * nw + w] & L.drop[w]) != 0u;
+                const unsigned long long hm = __ballot(hit);
+                if (hm) stand = __ffsll((long long)hm) - 1;
+                // accepted groups still to take: after g, among those that stand
+                am &= stand >= 64 ? ~0ull : (1ull << stand) - 1ull;
+                am &= g >= 63 ? 0ull : ~0ull << (g + 1);
             }
+            if (stand == n) {
+                u = v & ~drop;
+                most = min(4 * most, SEL_GROUPS);
+            } else {
+                for (int g = 0; g < stand; ++g)
+                    if (lane < nw) u &= ~L.gmask[g * nw + lane];
+                u &= ~drop;
+                most = min(max(2 * stand, 8), SEL_GROUPS);
+            }
+            if (trace && lane < stand && g0 + lane < C.tr.max_k) {
+                C.tr.gpick[row * C.tr.max_k + g0 + lane] = pick;
+                C.tr.gacc[row * C.tr.max_k + g0 + lane] = rec;
+            }
+            g0 += stand;
         }
-        if (trace && lane == 0 && g < C.tr.max_k) {
-            C.tr.gpick[row * C.tr.max_k + g] = pick;
-            C.tr.gacc[row * C.tr.max_k + g] = rec;
-        }
-        g += 1;
-        wave_sync();
     }
-    if (lane == 0) {
+    if (tid == 0) {
         L.misc[M_ACC] = na;
-        L.misc[M_NG] = g;
+        L.misc[M_NG] = g0;
         L.misc[M_N] = N;
         S.energy = et;
         // counters only: an atomic add without return keeps the load of
@@ -1181,11 +1518,10 @@ __device__ inline void greedy_select(CRep &C, State &S, const Lds &L, int row, b
     }
 }
 
-// greedy_select for k <= 64 with the per-trial values in registers: lane t
-// holds trial t's value, exp term, adjacency row (bit j: trial j within the
-// cutoff) and slot, and group t's two variates.  Group members are compacted
-// into lanes 0..m-1 in trial order (ds_permute), so the weights, their sums
-// and the decisions are those of greedy_select, bit for bit.  Wave 0 only.
+// At most 64 trials, per-trial values in registers: lane t holds trial t's
+// value, exp term, adjacency row (bit j: trial j within the cutoff) and slot,
+// and group t's two variates.  Group members are compacted into lanes 0..m-1
+// in trial order (ds_permute) and their weights summed by one scan.  Wave 0 only.
 __device__ inline void greedy_select64(CRep &C, State &S, const Lds &L, int row, bool trace, const MoveCtx &mc,
                                        double val, double ea, double rsel, double racc, unsigned long long adj,
                                        int tslot)
@@ -1439,20 +1775,8 @@ __device__ inline void accept_move(CRep &C, State &S, const Lds &L, const MoveCt
                 L.adjl[q] = C.adj[t * ADJW + w];
             }
         }
-        // everything of the serial selection that does not depend on earlier
-        // groups: the variates of group g (at most k groups) and each trial's
-        // exp(B - beta E) (insert) or exp(-beta dE) (move)
-        {
-            const double Bx = (kind == K_INS) ? mc.B : 0.0;
-            for (int t = tid; t < k; t += NT) {
-                const u32x4 xr = draw(C.seed, (uint32_t)step, (uint32_t)t, P_DECIDE);
-                L.rsel[t] = u01d(xr.x, xr.y);
-                L.racc[t] = u01d(xr.z, xr.w);
-                L.ea[t] = exp(Bx - BETA * L.val[t]);
-            }
-        }
         __syncthreads();
-        if ((tid >> 6) == 0) greedy_select(C, S, L, row, trace, mc);
+        select_groups<NT>(C, S, L, row, trace, mc);
         __syncthreads();
         commit_accepted<NT, EW>(C, S, L, row, trace, mc);
     }
@@ -1476,12 +1800,32 @@ __device__ inline void accept_step(CRep &C, State &S, const Lds &L)
     accept_move<NT, EW>(C, S, L, mc);
 }
 
+// a move without trials (insertion into full slots, no molecule to move): an
+// attempt, nothing else (accept_move's result for k = 0)
+__device__ inline void skip_move(CRep &C, State &S)
+{
+    if (threadIdx.x == 0) {
+        const int spi = S.sp, step = S.step;
+        count_add<false>(&S.att[spi * 4 + S.kind], 1ll);
+        int row;
+        if (tracing(C, step, row)) {
+            C.tr.k[row] = 0;
+            C.tr.ngroups[row] = 0;
+            C.tr.naccept[row] = 0;
+            C.tr.n_after[row] = S.totalNum[spi];
+            C.tr.etot[row] = S.energy;
+        }
+        S.step = step + 1;
+    }
+    __syncthreads();
+}
+
 // ---- prep phase: picks and trial centres of S.step ------------------------------
 // pre: the move's descriptor loaded with the previous move (for the same
 // species, the count that move's accept phase left in L.misc[M_N]), or null
 // use_pre: the move after prev (species prev_spi) was loaded into L.misc[M_NX..]
 template <int NT>
-__device__ inline int prep_step(CRep &C, State &S, const Lds &L, bool use_pre, int prev_step, int prev_spi)
+__device__ inline Move prep_step(CRep &C, State &S, const Lds &L, bool use_pre, int prev_step, int prev_spi)
 {
     const int tid = threadIdx.x;
     int step, mv, N, conf, maxNum, startRes;
@@ -1548,37 +1892,35 @@ __device__ inline int prep_step(CRep &C, State &S, const Lds &L, bool use_pre, i
         }
         C.tc[t] = make_float4(c[0], c[1], c[2], 0.f);
     }
-    const int nitems = (kind == K_TRN || kind == K_ROT) ? 2 * k : k;
     if (tid == 0) {
         S.kind = kind;
         S.sp = spi;
         S.k = k;
-        S.nitems = nitems;
+        S.nitems = k;
         S.done = 0;
     }
     __syncthreads();
-    return nitems;
+    return make_move(kind, spi, k, step);
 }
 
 template <int NT>
-__device__ inline int prep_step(CRep &C, State &S, const Lds &L)
+__device__ inline Move prep_step(CRep &C, State &S, const Lds &L)
 {
     return prep_step<NT>(C, S, L, false, 0, 0);
 }
 
-// Items a workgroup takes with one claim of a move of `unc` unclaimed items
-// in size class sz (0: at most 4, 1: 5-16, 2: more).  Consecutive items of one
-// move share the claim's round trips and acquire (an L1 invalidate), and the
-// workgroup's second and later evaluations find the move's data in L1: with
-// eight systems per XCD, a pass of the 64-system workload takes 700 instead of
-// 1150 ms with 4 items per claim of the largest moves and 2 of the middle
-// ones.  With few systems per XCD (nc < 4) the workgroups would idle while a
-// few of them work through a move's items one after another, so a claim then
-// takes no more than a fair share, ceil(unc / workgroups of the XCD).  Small
-// moves, a replica's critical path, take one item per claim.
-__device__ inline int claim_take(int sz, int unc, int nc, int nwx)
+// Trials a workgroup takes with one claim of a move of nitems trials, unc of
+// them unclaimed: of a small move (COOP_TRIALS) one per team, two while more than
+// 4 are left; of a larger move two per wave, so that waves whose trials end
+// early take over, and one per wave when few are left.  With few systems per XCD
+// (nc < 4) the workgroups would idle while a few of them work through a move's
+// trials, so a claim then takes no more than a fair share, ceil(unc / workgroups
+// of the XCD).
+template <int NT>
+__device__ inline int claim_take(int nitems, int unc, int nc, int nwx)
 {
-    const int want = sz == 2 ? 4 : (sz == 1 ? 2 : 1);
+    constexpr int NW = NT / 64;
+    const int want = nitems <= COOP_TRIALS ? (unc > 4 ? 2 : 1) * (NW / COOP) : NW;
     if (nc >= 4) return want;
     const int share = (unc + nwx - 1) / nwx;
     return min(want, max(share, 1));
@@ -1602,12 +1944,20 @@ __device__ inline int claim_prio(CRep &C, int step, int end)
     return 0xFFFFFF - (int)(left < 0xFFFFFFu ? left : 0xFFFFFFu);
 }
 
-// advance past empty moves and publish the next move with work (batched form)
+// Advance past empty moves, prepare the next move with trials and publish it
+// (batched form), the first `keep` of its trials (claim_take of the move, nc and
+// nwx as there) claimed for this workgroup, which goes on with them: a small
+// move then needs neither the other workgroups' polls nor a claim, and nothing
+// is published of a move that this workgroup takes whole.  None are kept where an
+// XCD has more replicas (nc) than workgroups (nwx): those left out would start only
+// when others have ended.
 // use_pre: the move after prev_step (species prev_spi) is in L.misc[M_NX..]
+// Returns the move (k = 0 at the end of the run) and the trials kept.
 template <int NT>
-__device__ inline void advance_and_publish(CRep &C, State &S, Sched *sch, const Lds &L, bool use_pre,
-                                           int prev_step, int prev_spi)
+__device__ inline Move advance_and_publish(CRep &C, State &S, Sched *sch, const Lds &L, bool use_pre,
+                                           int prev_step, int prev_spi, int nc, int nwx, int &keep)
 {
+    Move mv;
     while (true) {
         if (use_pre ? prev_step + 1 >= L.misc[M_NX + 0] : S.step >= S.end) {
             xcd_release();
@@ -1616,44 +1966,41 @@ __device__ inline void advance_and_publish(CRep &C, State &S, Sched *sch, const 
                 __hip_atomic_store(&S.claim, claim_word(0xFFFFFF, 0, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_fetch_add(&sch->finished, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            mv.k = keep = 0;
             break;
         }
-        int step, end;
-        if (use_pre) {
-            step = prev_step + 1;
-            end = L.misc[M_NX + 0];
-        } else {
-            step = S.step;
-            end = S.end;
-        }
-        const int nitems = prep_step<NT>(C, S, L, use_pre, prev_step, prev_spi);
+        int end;
+        if (use_pre) end = L.misc[M_NX + 0];
+        else end = S.end;
+        mv = prep_step<NT>(C, S, L, use_pre, prev_step, prev_spi);
         use_pre = false;
-        if (nitems > 0) {
-            const int prio = claim_prio(C, step, end);
+        if (mv.k > 0) {
+            keep = nc <= nwx ? min(claim_take<NT>(mv.nitems, mv.nitems, nc, nwx), mv.nitems) : 0;
             if (threadIdx.x == 0) {
                 S.t_pub = wall_clock64();
-                __hip_atomic_store(&S.done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                L.misc[M_NEXT] = 0;
             }
-            xcd_release();
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                // every thread's writes have completed: a CU whose L1 was
-                // invalidated after this time holds no older copy of them
-                S.t_data = wall_clock64();
+            if (keep < mv.nitems) {
+                const int prio = claim_prio(C, mv.step, end);
+                if (threadIdx.x == 0)
+                    __hip_atomic_store(&S.done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 xcd_release();
-                __hip_atomic_store(&S.claim, claim_word(prio, nitems, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __syncthreads();
+                if (threadIdx.x == 0) {
+                    // every thread's writes have completed: a CU whose L1 was
+                    // invalidated after this time holds no older copy of them
+                    S.t_data = wall_clock64();
+                    xcd_release();
+                    __hip_atomic_store(&S.claim, claim_word(prio, mv.nitems, keep), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
             break;
         }
-        accept_step<NT, false>(C, S, L);
+        skip_move(C, S);
     }
     __syncthreads();
-}
-
-template <int NT>
-__device__ inline void advance_and_publish(CRep &C, State &S, Sched *sch, const Lds &L)
-{
-    advance_and_publish<NT>(C, S, sch, L, false, 0, 0);
+    return mv;
 }
 
 // ---- kernels ---------------------------------------------------------------------
@@ -1682,18 +2029,29 @@ __global__ __launch_bounds__(NT) void k_start(const Rep *reps, State *st, Sched 
     extern __shared__ __align__(16) char smem[];
     const Lds L = carve(smem, lay);
     const int r = r0 + blockIdx.x;
-    if (batched) advance_and_publish<NT>(rep_of(reps, r), st[r], sch, L);
+    int keep;
+    if (batched) advance_and_publish<NT>(rep_of(reps, r), st[r], sch, L, false, 0, 0, 1, 0, keep);
     else if (st[r].step < st[r].end) prep_step<NT>(rep_of(reps, r), st[r], L);
 }
 
-template <int NT, bool STAGED, bool EW>
-__global__ __launch_bounds__(NT) void k_eval_plain(const Rep *reps, const State *st, int r, LdsLayout lay)
+// the current move's trials, as many per workgroup as it has teams or waves
+template <int NT, bool STAGED, int TM>
+__global__ __launch_bounds__(NT) void k_eval_plain(const Rep *reps, State *st, int r, LdsLayout lay)
 {
     extern __shared__ __align__(16) char smem[];
-    const State &S = st[r];
-    if (S.step >= S.end || (int)blockIdx.x >= S.nitems) return;
+    State &S = st[r];
+    if (S.step >= S.end) return;
+    const Move mv = move_of(S);
+    const int per = mv.coop ? NT / 64 / COOP : NT / 64;
+    const int item = blockIdx.x * per;
+    if (item >= mv.nitems) return;
     const Lds L = carve(smem, lay);
-    eval_item<NT, STAGED, false, EW>(rep_of(reps, r), S, blockIdx.x, L);
+    CRep &C = rep_of(reps, r);
+    if (threadIdx.x == 0) L.misc[M_NEXT] = 0;
+    stage_tables<NT, STAGED>(C, L, true, true);
+    ItemStats ist{};
+    eval_items<NT, STAGED, TM>(C, mv, item, min(per, mv.nitems - item), L, ist);
+    if ((threadIdx.x & 63) == 0 && ist.neval) add_item_stats<false>(S, ist, species_of(C, mv.spi).nf);
 }
 
 template <int NT, bool STAGED, bool EW>
@@ -1747,8 +2105,8 @@ __device__ inline int cu_acquire_needed(const State &S, const unsigned long long
 // accept and prep phases and publishes the next move.  Exits when every
 // replica finished, or when no replica advanced during spin_limit polls
 // (then sch->abort is set).
-template <int NT, bool STAGED>
-__global__ __launch_bounds__(NT, 768 / NT) void k_batched(const Rep *reps, State *st, int R, Sched *sch,
+template <int NT, bool STAGED, int TM>
+__global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, int R, Sched *sch,
                                                LdsLayout lay, int spin_limit, XcdMap xm, int aff)
 {
     extern __shared__ __align__(16) char smem[];
@@ -1764,154 +2122,176 @@ __global__ __launch_bounds__(NT, 768 / NT) void k_batched(const Rep *reps, State
     int idle = 0, seen = -1;
     // replica whose species table, and pair table (Rep::tab) that are in LDS
     int cached_rep = -1, cached_tab = -1;
+    // the trials this workgroup kept of a move it published (advance_and_publish)
+    int kept = 0, kept_rep = -1;
+    Move mv;
     while (true) {
-        if (tid < 64) {
-            // wave 0 polls every replica of this XCD at once, one claim word
-            // per lane.  Claim words are device-scope: a workgroup-scope load
-            // may hit this CU's L1, which only a claiming workgroup invalidates,
-            // so idle workgroups would keep seeing an old word.  Polls are
-            // loads; an atomic is issued only to claim (read-modify-writes of
-            // one address serialize).  The scheduler's words (progress,
-            // finished, abort) are read only when nothing could be claimed:
-            // a workgroup that finds work goes from its last item to its next
-            // with two memory round trips (the claim words, the claim).
-            const int lane = tid;
-            int found = -1, item = 0, cnt = 1;
-            for (int b0 = 0; b0 < nc && found < 0; b0 += 64) {
-                int r = -1;
-                unsigned long long w = 0ull;
-                if (b0 + lane < nc) {
-                    r = xm.cls_reps[c0 + (rot + b0 + lane) % nc];
-                    w = __hip_atomic_load(&st[r].claim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                bool avail = r >= 0 && (w & 0xFFFFFull) < ((w >> 20) & 0xFFFFFull);
-                // Moves with few unclaimed items first (up to 4, then up to
-                // 16): a replica waiting on one or a few evaluations is on its
-                // own critical chain.  Within those classes and among the
-                // larger moves, the replica with the most estimated work left
-                // first (claim_prio): the run ends with its last replica, and
-                // a large move occupies the XCD's workgroups for several
-                // rounds whichever order they come in.  (Fewest unclaimed
-                // items first among the large moves too: 5 % slower.)
-                const unsigned long long unc = ((w >> 20) & 0xFFFFFull) - (w & 0xFFFFFull);
-                unsigned size = unc <= 4ull ? 0u : (unc <= 16ull ? 1u : 2u);
-                // affinity (aff > 0): a move of at least aff unclaimed items
-                // of the replica whose tables this workgroup holds in LDS
-                // comes before the other such moves (its species table and
-                // staged pair table are reused)
-                if (aff > 0 && unc >= (unsigned long long)aff) size = (r == cached_rep) ? 2u : 3u;
-                const unsigned prio = (unsigned)(w >> 40) >> 8;
-                const int take_lane = claim_take((int)size, (int)unc, nc, nwx);
-                while (__ballot(avail) != 0ull) {
-                    const unsigned key =
-                        wave_min(avail ? ((size << 22) | (prio << 6) | (unsigned)lane) : 0xFFFFFFFFu);
-                    const int l = (int)(key & 63u);
-                    const int rr = __shfl(r, l, 64);
-                    const int take = __shfl(take_lane, l, 64);
-                    unsigned long long old = 0ull;
-                    if (lane == l)
-                        old = __hip_atomic_fetch_add(&st[rr].claim, (unsigned long long)take, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-                    old = __shfl(old, l, 64);
-                    const int c = (int)(old & 0xFFFFFull), n = (int)((old >> 20) & 0xFFFFFull);
-                    if (c < n) {
-                        found = rr;
-                        item = c;
-                        cnt = min(take, n - c);
-                        break;
+        int found, item, cnt;
+        if (kept > 0) {
+            found = kept_rep;
+            item = 0;
+            cnt = kept;
+        } else {
+            if (tid < 64) {
+                // wave 0 polls every replica of this XCD at once, one claim word
+                // per lane.  Claim words are device-scope: a workgroup-scope load
+                // may hit this CU's L1, which only a claiming workgroup invalidates,
+                // so idle workgroups would keep seeing an old word.  Polls are
+                // loads; an atomic is issued only to claim (read-modify-writes of
+                // one address serialize).  The scheduler's words (progress,
+                // finished, abort) are read only when nothing could be claimed:
+                // a workgroup that finds work goes from its last item to its next
+                // with two memory round trips (the claim words, the claim).
+                const int lane = tid;
+                int rfound = -1, ritem = 0, rcnt = 1;
+                for (int b0 = 0; b0 < nc && rfound < 0; b0 += 64) {
+                    int r = -1;
+                    unsigned long long w = 0ull;
+                    if (b0 + lane < nc) {
+                        r = xm.cls_reps[c0 + (rot + b0 + lane) % nc];
+                        w = __hip_atomic_load(&st[r].claim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-                    if (lane == l) avail = false;
+                    bool avail = r >= 0 && (w & 0xFFFFFull) < ((w >> 20) & 0xFFFFFull);
+                    // Moves with few unclaimed items first (up to 4, then up to
+                    // 16): a replica waiting on one or a few evaluations is on its
+                    // own critical chain.  Within those classes and among the
+                    // larger moves, the replica with the most estimated work left
+                    // first (claim_prio): the run ends with its last replica, and
+                    // a large move occupies the XCD's workgroups for several
+                    // rounds whichever order they come in.  (Fewest unclaimed
+                    // items first among the large moves too: 5 % slower.)
+                    const unsigned long long unc = ((w >> 20) & 0xFFFFFull) - (w & 0xFFFFFull);
+                    unsigned size = unc <= 4ull ? 0u : (unc <= 16ull ? 1u : 2u);
+                    // affinity (aff > 0): a move of at least aff unclaimed items
+                    // of the replica whose tables this workgroup holds in LDS
+                    // comes before the other such moves (its species table and
+                    // staged pair table are reused)
+                    if (aff > 0 && unc >= (unsigned long long)aff) size = (r == cached_rep) ? 2u : 3u;
+                    const unsigned prio = (unsigned)(w >> 40) >> 8;
+                    const int take_lane = claim_take<NT>((int)((w >> 20) & 0xFFFFFull), (int)unc, nc, nwx);
+                    while (__ballot(avail) != 0ull) {
+                        const unsigned key =
+                            wave_min(avail ? ((size << 22) | (prio << 6) | (unsigned)lane) : 0xFFFFFFFFu);
+                        const int l = (int)(key & 63u);
+                        const int rr = __shfl(r, l, 64);
+                        const int take = __shfl(take_lane, l, 64);
+                        unsigned long long old = 0ull;
+                        if (lane == l)
+                            old = __hip_atomic_fetch_add(&st[rr].claim, (unsigned long long)take, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
+                        old = __shfl(old, l, 64);
+                        const int c = (int)(old & 0xFFFFFull), n = (int)((old >> 20) & 0xFFFFFull);
+                        if (c < n) {
+                            rfound = rr;
+                            ritem = c;
+                            rcnt = min(take, n - c);
+                            break;
+                        }
+                        if (lane == l) avail = false;
+                    }
                 }
-            }
-            if (found == -1) {
-                int ctl[3] = {0, 0, 0};
+                if (rfound == -1) {
+                    int ctl[3] = {0, 0, 0};
+                    if (lane == 0) {
+                        ctl[0] = __hip_atomic_load(&sch->progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        ctl[1] = __hip_atomic_load(&sch->finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        ctl[2] = __hip_atomic_load(&sch->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    const int prog = __shfl(ctl[0], 0, 64), fin = __shfl(ctl[1], 0, 64), ab = __shfl(ctl[2], 0, 64);
+                    if (prog != seen) {
+                        seen = prog;
+                        idle = 0;
+                    }
+                    if (fin >= R || ab != 0) {
+                        rfound = -2;
+                    } else if (++idle > spin_limit) {
+                        // no replica advanced during spin_limit polls: stop instead of hanging
+                        if (lane == 0) __hip_atomic_store(&sch->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        rfound = -2;
+                    }
+                }
                 if (lane == 0) {
-                    ctl[0] = __hip_atomic_load(&sch->progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ctl[1] = __hip_atomic_load(&sch->finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ctl[2] = __hip_atomic_load(&sch->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                const int prog = __shfl(ctl[0], 0, 64), fin = __shfl(ctl[1], 0, 64), ab = __shfl(ctl[2], 0, 64);
-                if (prog != seen) {
-                    seen = prog;
-                    idle = 0;
-                }
-                if (fin >= R || ab != 0) {
-                    found = -2;
-                } else if (++idle > spin_limit) {
-                    // no replica advanced during spin_limit polls: stop instead of hanging
-                    if (lane == 0) __hip_atomic_store(&sch->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    found = -2;
+                    L.misc[M_FOUND] = rfound;
+                    L.misc[M_ITEM] = ritem;
+                    L.misc[M_CNT] = rcnt;
+                    L.misc[M_NEXT] = 0;
+                    L.misc[M_INV] = rfound >= 0 ? cu_acquire_needed(st[rfound], xm.cu_inv, slot) : 1;
                 }
             }
-            if (lane == 0) {
-                L.misc[M_FOUND] = found;
-                L.misc[M_ITEM] = item;
-                L.misc[M_CNT] = cnt;
-                L.misc[M_INV] = found >= 0 ? cu_acquire_needed(st[found], xm.cu_inv, slot) : 1;
+            __syncthreads();
+            // uniform across the workgroup: the replica's fields become scalar loads
+            found = __builtin_amdgcn_readfirstlane(L.misc[M_FOUND]);
+            item = __builtin_amdgcn_readfirstlane(L.misc[M_ITEM]);
+            cnt = __builtin_amdgcn_readfirstlane(L.misc[M_CNT]);
+            const int need_inv = __builtin_amdgcn_readfirstlane(L.misc[M_INV]);
+            __syncthreads();
+            if (found == -2) break;
+            if (found == -1) {
+                // about 0.9 us between polls of an idle workgroup (1.5 % faster
+                // than 0.2 us on short runs of the 64-replica workload, equal to
+                // 0.45-1.8 us on full runs; evaluation times do not change)
+                __builtin_amdgcn_s_sleep(32);
+                continue;
             }
-        }
-        __syncthreads();
-        // uniform across the workgroup: the replica's fields become scalar loads
-        const int found = __builtin_amdgcn_readfirstlane(L.misc[M_FOUND]);
-        const int item = __builtin_amdgcn_readfirstlane(L.misc[M_ITEM]);
-        const int cnt = __builtin_amdgcn_readfirstlane(L.misc[M_CNT]);
-        const int need_inv = __builtin_amdgcn_readfirstlane(L.misc[M_INV]);
-        __syncthreads();
-        if (found == -2) break;
-        if (found == -1) {
-            // about 0.9 us between polls of an idle workgroup (1.5 % faster
-            // than 0.2 us on short runs of the 64-replica workload, equal to
-            // 0.45-1.8 us on full runs; evaluation times do not change)
-            __builtin_amdgcn_s_sleep(32);
-            continue;
-        }
-        if (need_inv) {
-            const unsigned long long tinv = wall_clock64();
-            xcd_acquire();
-            if (tid == 0) {
-                // recorded once this wave's invalidate has executed
-                xcd_release();
-                __hip_atomic_store(&xm.cu_inv[slot], tinv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (need_inv) {
+                const unsigned long long tinv = wall_clock64();
+                xcd_acquire();
+                if (tid == 0) {
+                    // recorded once this wave's invalidate has executed
+                    xcd_release();
+                    __hip_atomic_store(&xm.cu_inv[slot], tinv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
+            mv = move_of(st[found]);
         }
         CRep &C = rep_of(reps, found);
         State &S = st[found];
         const unsigned long long te0 = wall_clock64();
         const int tab = C.tab;
-        ItemStats ist;
-        // the claimed items one after another; the last one's statistics are
-        // added after the completion count (the others' before it)
-        for (int j = 0; j < cnt; ++j) {
-            if (j > 0) __syncthreads();
-            eval_item<NT, STAGED, true, false>(C, S, item + j, L, j == 0 && found != cached_rep,
-                                               j == 0 && tab != cached_tab, j + 1 < cnt ? nullptr : &ist);
-        }
+        // the species table stays in LDS while a workgroup keeps evaluating
+        // trials of one replica, the pair table while it keeps to replicas with
+        // that table
+        stage_tables<NT, STAGED>(C, L, found != cached_rep, tab != cached_tab);
+        ItemStats ist{};
+        // a small move's evaluations are its replica's serial path: ahead of the
+        // large moves' waves sharing the SIMDs (3 % of a pass)
+        if (mv.k <= 16) __builtin_amdgcn_s_setprio(2);
+        eval_items<NT, STAGED, TM>(C, mv, item, cnt, L, ist);
+        __builtin_amdgcn_s_setprio(0);
         cached_rep = found;
         cached_tab = tab;
+        kept = 0;
         const unsigned long long te1 = wall_clock64();
-        xcd_release();
-        __syncthreads();
-        if (tid == 0) {
-            const int old = __hip_atomic_fetch_add(&S.done, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            L.misc[M_LAST] = (old + cnt == S.nitems) ? 1 : 0;
-            // statistics after the completion count: the release above does
-            // not wait for them
-            add_item_stats<true>(S, ist);
-            count_add<true>(&S.t_eval, te1 - te0);
+        bool last = cnt == mv.nitems;   // the whole move is this workgroup's
+        if (!last) {
+            xcd_release();
+            __syncthreads();
+            if (tid == 0) {
+                const int old = __hip_atomic_fetch_add(&S.done, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                L.misc[M_LAST] = (old + cnt == mv.nitems) ? 1 : 0;
+            }
+            __syncthreads();
+            last = uniform_i(L.misc[M_LAST]) != 0;
+            // other workgroups' energies and poses
+            if (last) xcd_acquire();
+        } else {
+            __syncthreads();
         }
-        __syncthreads();
-        if (L.misc[M_LAST]) {
+        // statistics after the completion count: the release above does not
+        // wait for them
+        if (tid == 0) count_add<true>(&S.t_eval, te1 - te0);
+        if ((tid & 63) == 0 && ist.neval) add_item_stats<true>(S, ist, species_of(C, mv.spi).nf);
+        if (last) {
             // accept and prep are this replica's serial critical path: issue
             // ahead of the evaluation waves sharing the SIMDs
             __builtin_amdgcn_s_setprio(3);
-            xcd_acquire();
             const unsigned long long ta0 = wall_clock64();
             const unsigned long long tpub = S.t_pub;
-            const int step0 = S.step;
-            const MoveCtx mc = move_ctx(C, S);
-            accept_move<NT, false>(C, S, L, mc, true);
+            const MoveCtx mc = move_ctx(fresh(C), S);
+            accept_move<NT, false>(fresh(C), S, L, mc, true);
             const unsigned long long ta1 = wall_clock64();
-            advance_and_publish<NT>(C, S, sch, L, true, mc.step, mc.spi);
+            mv = advance_and_publish<NT>(fresh(C), S, sch, L, true, mc.step, mc.spi, nc, nwx, kept);
+            kept_rep = found;
             if (tid == 0) {
                 const unsigned long long ta2 = wall_clock64();
                 // timers after the next move is published, off its path; the
@@ -1921,7 +2301,7 @@ __global__ __launch_bounds__(NT, 768 / NT) void k_batched(const Rep *reps, State
                 count_add<true>(&S.t_accept, ta1 - ta0);
                 count_add<true>(&S.t_prep, ta2 - ta1);
                 int row;
-                if (tracing(C, step0, row)) {
+                if (tracing(C, mc.step, row)) {
                     C.tr.tick[4 * row + 0] = tpub;
                     C.tr.tick[4 * row + 1] = ta0;
                     C.tr.tick[4 * row + 2] = ta1;
@@ -1930,7 +2310,6 @@ __global__ __launch_bounds__(NT, 768 / NT) void k_batched(const Rep *reps, State
                 __hip_atomic_fetch_add(&sch->progress, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __builtin_amdgcn_s_setprio(0);
-            cached_rep = cached_tab = -1;  // accept and prep reuse the evaluation region
         }
         __syncthreads();
     }
@@ -1942,40 +2321,44 @@ __global__ void k_xcc_probe(int *out)
     if (threadIdx.x == 0) out[blockIdx.x] = my_xcc();
 }
 
-// energies of given poses (tests and the adjoint's forward)
-template <int NT, bool STAGED, bool EW>
-__global__ __launch_bounds__(NT) void k_eval_poses(const Rep *reps, int r, int spi, const float *centres,
+// Energies of given poses: one wave per pose, or (few poses) four that share
+// its cells.
+template <int NT, bool STAGED, int TM, int PARTS>
+__global__ __launch_bounds__(NT) void k_eval_poses(const Rep *reps, int r, int spi, int npose, const float *centres,
                                                   const float *poses, const int *excl, double *E, int *ninc,
                                                   uint32_t *hash, LdsLayout lay)
 {
     extern __shared__ __align__(16) char smem[];
+    constexpr int PER = NT / 64 / PARTS;
     const Lds L = carve(smem, lay);
     CRep &C = rep_of(reps, r);
     CSpecies &F = species_of(C, spi);
-    const int nf = F.nf, i = blockIdx.x, tid = threadIdx.x;
-    if (STAGED) stage_pair_table<NT>(C, L);
-    load_species_table(C, L);
-    if (tid < nf) {
-        const float *p = poses + ((size_t)i * nf + tid) * 3;
-        L.frag[tid] = make_float4(p[0], p[1], p[2], F.kq[tid]);
-        L.frow[tid] = F.trow[tid];
-    }
-    __syncthreads();
-    double e;
-    int n, na;
-    uint32_t h;
-    eval_energy<NT, STAGED, EW>(C, centres[3 * i], centres[3 * i + 1], centres[3 * i + 2], nf, excl[i], L, &e, &n,
-                                &h, &na);
-    if (EW) {
-        const int x = excl[i];
-        const bool own = x >= F.startRes && x < F.startRes + F.maxNum;
-        const double er = ewald_recip<NT>(C, F, L, nf, own ? F.atomBase + (x - F.startRes) * nf : -1);
-        if (tid == 0) e += er;
-    }
-    if (tid == 0) {
-        E[i] = e;
-        ninc[i] = n;
-        hash[i] = h;
+    const int nf = F.nf, lane = threadIdx.x & 63, wave = uniform_i(threadIdx.x >> 6), part = wave % PARTS;
+    const WaveLds W = wave_lds(L, wave);
+    stage_tables<NT, STAGED>(C, L, true, true);
+    for (int i0 = blockIdx.x * PER; i0 < npose; i0 += gridDim.x * PER) {
+        const int i = i0 + wave / PARTS, q = min(i, npose - 1), x = uniform_i(excl[q]);
+        if (PARTS == 1 && i >= npose) break;
+        const float c[3] = {uniform_f(centres[3 * (size_t)q]), uniform_f(centres[3 * (size_t)q + 1]),
+                            uniform_f(centres[3 * (size_t)q + 2])};
+        if (lane < nf) {
+            const float *p = poses + ((size_t)q * nf + lane) * 3;
+            order_pose<TM>(C, F, W, 0, lane, make_float4(p[0], p[1], p[2], F.kq[lane]), c);
+        }
+        wave_sync();
+        PoseSums s;
+        eval_poses_wave<STAGED, TM>(C, L, W, spi, nf, 1, c, c, true, x, false, part, PARTS, s);
+        if (TM == T_EWALD) {
+            const bool own = x >= F.startRes && x < F.startRes + F.maxNum;
+            s.e[0] += ewald_recip(C, F, W, 0, nf, own ? F.atomBase + (x - F.startRes) * nf : -1, part, PARTS);
+        }
+        if (PARTS > 1) team_sum<NT>(L, s);
+        if (i < npose && part == 0 && lane == 0) {
+            E[i] = s.e[0];
+            ninc[i] = s.nin[0];
+            hash[i] = s.hash[0];
+        }
+        wave_sync();
     }
 }
 

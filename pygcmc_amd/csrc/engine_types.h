@@ -23,8 +23,13 @@ constexpr int MAXT = 32;             // species per system
 constexpr int MAXF = 20;             // atoms per fragment (AtomArray.atoms[20])
 constexpr int MAXK = 2048;           // trials per move (confBias)
 constexpr int ADJW = MAXK / 32;      // words of one adjacency row
-constexpr int MISC_INTS = 104;
-constexpr int INC_CAP = 1024;         // included-group slots per pair pass (a multiple of the workgroup size)        // scratch ints of a workgroup (see engine_kernels.h)
+constexpr int MISC_INTS = 104;       // scratch ints of a workgroup (see engine_kernels.h)
+// a wave's scratch (WaveLds): cells listed at a time, groups and atoms of a batch
+constexpr int WL_CELLS = 512, WL_GROUPS = 256, WL_ATOMS = 1024;
+constexpr int WL_BYTES = 2 * MAXF * (32 + 16) + WL_ATOMS + 4 * WL_CELLS + 8 * WL_GROUPS + 128;
+constexpr int SEL_GROUPS = 64;       // groups of a selection batch (select_groups: one lane each)
+constexpr int TEAM_BYTES = 48;       // a wave's sums of a shared trial (PoseSums)
+static_assert(WL_BYTES % 32 == 0 && WL_GROUPS <= 256 && WL_ATOMS == 1024, "wave scratch layout");
 // a mobile group's cell record carries its group id and species in one word
 constexpr int GID_BITS = 24;         // group ids below 2^24
 constexpr int GID_MASK = (1 << GID_BITS) - 1;
@@ -44,6 +49,9 @@ struct Species {
     float kq[MAXF];        // 1388.431112 * charge, rounded once
     int trow[MAXF];        // type * Y: row of the pair table
     int ttype[MAXF];       // type
+    // atoms ordered by type: place of each atom, row of the pair table per place,
+    // and the runs of equal type (end place, row)
+    int slot[MAXF], srow[MAXF], nrun, run_end[MAXF], run_row[MAXF];
 };
 
 struct DevTrace {
@@ -70,14 +78,18 @@ static_assert(sizeof(FixRec) == 32, "FixRec layout");
 struct Rep {
     AxisCut ax[3];
     float L[3], start[3], invL[3];
+    double Ld[3], invLd[3];  // L and invL again, in FP64 (scalar operands of the pair terms)
     float rc, r2max, dx, cav;
     float inv_h[3];
     int nc[3], ncell;
     int G, T, X, Y;
     int nfix, nres, natom, maxk;
     int cap, ovf_base, nst, nmoves;
+    int nst_wide;            // entries [nst, nst + nst_wide) also cover a centre up to grid_dx further along
+                             // each axis (a translation's new centre); 0: such moves are too wide for that
     int coul64, prune;       // Coulomb pair terms in FP64; bit i: stencil cells may be
                              // pruned along axis i by their distance from the trial centre
+    int prune_wide;          // the same for the wide stencil
     float cell_h[3];         // cell edges L / nc
     float prune_r2;          // (rc + stencil slack)^2
     uint32_t seed;
@@ -86,7 +98,6 @@ struct Rep {
                              // less than L/2 apart after one image shift of the atom around the
                              // trial centre (rc + group extents < L/2, host-checked)
     int tab;                 // replicas with equal tab have equal pair tables (one copy in LDS serves them)
-    int pad1;
     const float *grid;
     const int *moves;
     const uint32_t *wcum;    // [nmoves+1] estimated critical-path cost of moves [0, s), scaled (scheduling)
@@ -94,7 +105,8 @@ struct Rep {
     int2 *res_rng;
     float4 *atom;
     int *atype;
-    const float4 *pair;      // (100 sigma^2 hi, 4 eps, 100 sigma^2 lo, 0) per (fragment type, type)
+    const float4 *pair;      // per (fragment type, type): with coul64 and no Ewald double2 (4 eps S^6, 4 eps S^3)
+                             // with S = 100 sigma^2, else float4 (100 sigma^2 hi, 4 eps, 100 sigma^2 lo, 0)
     const Species *sp;
     // per cell c in [0, ncell]: (first fixed record, mobile count); the fixed
     // records of cell c are [cell[c].x, cell[c + 1].x), and cell[ncell].y
@@ -155,19 +167,16 @@ struct Sched {
 
 // byte offsets of the dynamic LDS carve-up (host computes, device applies)
 struct LdsLayout {
-    int smob, sfst, sfix, soff;    // stencil entries (int[nst+2]): mobile-slot base, fixed start, fixed count, offset
-    int incs, incn;                // included groups: first atom, atom count (int[inc_cap+1])
-    int frag, frow;                // fragment pose (float4[MAXF], int[MAXF])
-    int fragd;                     // fragment pose relative to the trial centre, FP64 (double4[MAXF])
+    int wave;                      // WL_BYTES per wave
+    int team;                      // sums of the waves that share a trial (TEAM_BYTES per wave)
     int pair;                      // float4[X*Y]: the pair table held in LDS, or -1
     int spt;                       // species table int4[MAXT] (startRes, maxNum, atomBase, nf)
-    int misc, dred;                // int[MISC_INTS], double[MAXWAVE]
+    int misc;                      // int[MISC_INTS]
     int members, w, val, accl;     // accept: int[maxk], double[maxk] x2, int2[maxk]
     int adjl;                      // accept: adjacency rows uint32[maxk * ceil(maxk/32)] or -1
-    int rsel, racc, ea;            // accept: double[maxk] each -- draws per group, exp terms per trial
+    int gmask, goff, gstart, gmin; // accept: uint32 and uint16[SEL_GROUPS * ceil(maxk/32)], int[SEL_GROUPS+1], uint64[64]
+    int drop;                      // accept: uint32[ceil(maxk/32)]
     int J;                         // prep: int[maxk]
-    int inc_cap;                   // included groups buffered before a pair pass
-    int cand, amap, map_cap;       // uint16[map_cap] each: candidate -> stencil entry, pair-pass atom -> group
     int total;
 };
 
@@ -181,22 +190,27 @@ __host__ __device__ inline unsigned long long claim_word(int prio, int nitems, i
 }
 
 // cell of a position (wrapped into the box), same float code on host and GPU
+__host__ __device__ inline void cell_coords(const float L[3], const float start[3], const float inv_h[3],
+                                            const int nc[3], float x, float y, float z, int c[3])
+{
+    const float p[3] = {x, y, z};
+    for (int i = 0; i < 3; ++i) {
+        float w = p[i] - start[i];
+        w = w - floorf(w / L[i]) * L[i];
+        const int ci = (int)(w * inv_h[i]);
+        c[i] = ci < 0 ? 0 : (ci >= nc[i] ? nc[i] - 1 : ci);
+    }
+}
 __host__ __device__ inline int cell_index(const float L[3], const float start[3],
                                           const float inv_h[3], const int nc[3],
                                           float x, float y, float z)
 {
-    float p[3] = {x, y, z};
     int c[3];
-    for (int i = 0; i < 3; ++i) {
-        float w = p[i] - start[i];
-        w = w - floorf(w / L[i]) * L[i];
-        int ci = (int)(w * inv_h[i]);
-        c[i] = ci < 0 ? 0 : (ci >= nc[i] ? nc[i] - 1 : ci);
-    }
+    cell_coords(L, start, inv_h, nc, x, y, z, c);
     return (c[0] * nc[1] + c[1]) * nc[2] + c[2];
 }
 
-// position of (x, y, z) inside its cell c[3] (cell_index's wrap), per axis
+// position of (x, y, z) inside its cell c[3] (cell_coords' wrap), per axis
 __host__ __device__ inline void cell_offset(const float L[3], const float start[3], const float h[3],
                                             const int c[3], float x, float y, float z, float u[3])
 {
@@ -208,17 +222,28 @@ __host__ __device__ inline void cell_offset(const float L[3], const float start[
     }
 }
 
-// Whether the cell at stencil offset d[3] from a centre at position u[3]
-// inside its cell may hold a group centre within the cutoff: false when the
+// Whether the cell of a stencil entry (offset + 128 per byte) may hold a group
+// centre within the cutoff of a centre at position u[3] relative to the home
+// cell (inside it, or past it by less than a translation): false when the
 // cell's box lies farther than sqrt(r2) (rc + slack) from the centre along
-// the axes whose bit is set in `prune`, true otherwise.
-__host__ __device__ inline bool stencil_cell_near(const float u[3], const int d[3], const float h[3], int prune,
-                                                  float r2)
+// the pruned axes, true otherwise.  base[i] = u[i] + 128 h[i] and h[i] of a pruned
+// axis, 0 of another (stencil_base).
+__host__ __device__ inline void stencil_base(const float u[3], const float h[3], int prune, float base[3], float hp[3])
+{
+    for (int i = 0; i < 3; ++i) {
+        const bool p = (prune >> i) & 1;
+        hp[i] = p ? h[i] : 0.0f;
+        base[i] = p ? u[i] + 128.0f * h[i] : 0.0f;
+    }
+}
+__host__ __device__ inline bool stencil_cell_near(int code, const float base[3], const float hp[3], float r2)
 {
     float g2 = 0.0f;
     for (int i = 0; i < 3; ++i) {
-        if (!((prune >> i) & 1)) continue;
-        const float g = d[i] > 0 ? (float)d[i] * h[i] - u[i] : (d[i] < 0 ? u[i] - (float)(d[i] + 1) * h[i] : 0.0f);
+        // distance from the centre to the cell's lower face, and from its upper
+        // face to the centre
+        const float lo = fmaf((float)(code >> (8 * i) & 255), hp[i], -base[i]);
+        const float g = fmaxf(fmaxf(lo, -lo - hp[i]), 0.0f);
         g2 = fmaf(g, g, g2);
     }
     return g2 <= r2;

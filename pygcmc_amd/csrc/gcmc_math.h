@@ -159,6 +159,17 @@ GC_HD bool within(float x0, float x1, float x2, float y0, float y1, float y2,
     return dist2_p(x0, x1, x2, y0, y1, y2, ax) <= r2max;
 }
 
+// |d| past the shift table (a centre or group several boxes away)?
+GC_HD bool axis_far(float d, const AxisCut& a) { return !(fabsf(d) < a.t[2]); }
+// d - shift L for |d| < t[2], without branches
+GC_HD float axis_near(float d, float L, float t0, float t1)
+{
+    const float m = fabsf(d);
+    float r = m >= t0 ? L : 0.0f;
+    r = m >= t1 ? L + L : r;      // 2 L is exact
+    return d - copysignf(r, d);
+}
+
 // order-independent hash of an included-group set, and a pose fingerprint
 GC_HD uint32_t group_hash(uint32_t g)
 {

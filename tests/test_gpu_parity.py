@@ -310,3 +310,18 @@ def test_xcd_assignment_never_changes_chains():
     for out in finals[1:]:
         for a, b in zip(out, finals[0]):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize('conf', [63, 64, 65, 96, 97, 130, 256, 300])
+def test_selection_by_number_of_trials(conf):
+    """Lock-step with the oracle at the trial counts where the selection changes
+    its form (64 trials in registers, above that batches of 64 groups): word
+    and wave boundaries of the member masks, moves of more groups than one
+    batch holds, acceptances inside a batch."""
+    from pygcmc_amd import synth
+    s = synth.water_sphere(mcsteps=40, conf=conf, n_fixed=3000, radius=25.0, box=100.0)
+    gt, ot, g, r, st = _lockstep(s, 40, 'batched', max_k=conf)
+    _compare(gt, ot, g, r)
+    print('groups', gt['ngroups'].max(), 'accepted', gt['naccept'].sum())
+    assert gt['naccept'].sum() > 0
+    assert conf < 256 or gt['ngroups'].max() > 64
