@@ -956,10 +956,12 @@ __device__ inline double ewald_recip(CRep &C, CSpecies &F, const WaveLds &W, int
     double v = 0.0;
     const int K[3] = {C.pk[0], C.pk[1], C.pk[2]};
     const float Lb[3] = {C.L[0], C.L[1], C.L[2]};
-    const int f0 = lane * parts + part;
-    if (f0 < nf) {
-        const float4 x = W.frag[s * MAXF + f0];
-        v = (double)F.tmpl[f0].w * (double)gcmc_spline::gather(C.pme_phi, K, Lb, x.x, x.y, x.z);
+    // 16 lanes per atom
+    for (int f0 = part * 4; f0 < nf; f0 += 4 * parts) {
+        const int f = f0 + (lane >> 4), q = min(f, nf - 1);
+        const float4 x = W.frag[s * MAXF + q];
+        const float phi = gcmc_spline::gather16(C.pme_phi, K, Lb, x.x, x.y, x.z, lane & 15);
+        if ((lane & 15) == 0 && f < nf) v += (double)F.tmpl[q].w * (double)phi;
     }
     if (base >= 0) {
         const int nw = nf * nf * 7;
@@ -1683,6 +1685,7 @@ __device__ inline void accept_move(CRep &C, State &S, const Lds &L, const MoveCt
         L.misc[M_ACC] = 0;
         L.misc[M_NG] = 0;
         L.misc[M_N] = mc.N;
+        if (EW) *C.pme_ndelta = 0;
     }
     __syncthreads();
     if (prefetch && tid == 64) load_next_move(C, S, L, mc);
@@ -2030,6 +2033,8 @@ __global__ __launch_bounds__(NT) void k_start(const Rep *reps, State *st, Sched 
     const Lds L = carve(smem, lay);
     const int r = r0 + blockIdx.x;
     int keep;
+    // (Ewald) the last move's charge changes are in the grid by now
+    if (rep_of(reps, r).ew && threadIdx.x == 0) *rep_of(reps, r).pme_ndelta = 0;
     if (batched) advance_and_publish<NT>(rep_of(reps, r), st[r], sch, L, false, 0, 0, 1, 0, keep);
     else if (st[r].step < st[r].end) prep_step<NT>(rep_of(reps, r), st[r], L);
 }
@@ -2102,11 +2107,14 @@ __device__ inline int cu_acquire_needed(const State &S, const unsigned long long
 
 // persistent form: workgroups of an XCD claim evaluations from that XCD's
 // replicas; the workgroup completing a replica's last evaluation runs its
-// accept and prep phases and publishes the next move.  Exits when every
-// replica finished, or when no replica advanced during spin_limit polls
-// (then sch->abort is set).
+// accept and prep phases and publishes the next move.  A replica with Ewald
+// electrostatics (TM == T_EWALD) stops after a move that changed its charges: the
+// potential has to be solved anew first (moves that change nothing, about half
+// of a slab's, go on at once).  Exits when `target` replicas (counted from the
+// scheduler's reset) finished or stopped, or when no replica advanced during
+// spin_limit polls (then sch->abort is set).
 template <int NT, bool STAGED, int TM>
-__global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, int R, Sched *sch,
+__global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, int target, Sched *sch,
                                                LdsLayout lay, int spin_limit, XcdMap xm, int aff)
 {
     extern __shared__ __align__(16) char smem[];
@@ -2202,7 +2210,7 @@ __global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, i
                         seen = prog;
                         idle = 0;
                     }
-                    if (fin >= R || ab != 0) {
+                    if (fin >= target || ab != 0) {
                         rfound = -2;
                     } else if (++idle > spin_limit) {
                         // no replica advanced during spin_limit polls: stop instead of hanging
@@ -2288,10 +2296,20 @@ __global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, i
             const unsigned long long ta0 = wall_clock64();
             const unsigned long long tpub = S.t_pub;
             const MoveCtx mc = move_ctx(fresh(C), S);
-            accept_move<NT, false>(fresh(C), S, L, mc, true);
+            accept_move<NT, TM == T_EWALD>(fresh(C), S, L, mc, true);
             const unsigned long long ta1 = wall_clock64();
-            mv = advance_and_publish<NT>(fresh(C), S, sch, L, true, mc.step, mc.spi, nc, nwx, kept);
-            kept_rep = found;
+            if (TM == T_EWALD && uniform_i(L.misc[M_ACC]) != 0) {
+                // stopped: k_start publishes the next move after the solve
+                xcd_release();
+                __syncthreads();
+                if (tid == 0) {
+                    __hip_atomic_store(&S.claim, claim_word(0xFFFFFF, 0, 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_fetch_add(&sch->finished, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            } else {
+                mv = advance_and_publish<NT>(fresh(C), S, sch, L, true, mc.step, mc.spi, nc, nwx, kept);
+                kept_rep = found;
+            }
             if (tid == 0) {
                 const unsigned long long ta2 = wall_clock64();
                 // timers after the next move is published, off its path; the

@@ -71,12 +71,7 @@ __device__ inline Spline3 splines(const float4 a, const Geo &g)
     return s;
 }
 
-// element i of a 4-vector held in registers (no indexed registers)
-__device__ inline float pick4(const float w[4], int i)
-{
-    const float a = (i & 1) ? w[1] : w[0], b = (i & 1) ? w[3] : w[2];
-    return (i & 2) ? b : a;
-}
+using gcmc_spline::pick4;
 
 // The fixed-point term rint(w01 w2 2^32) of one grid point.  Adding 1.5 2^52 puts
 // the rounded integer into the low bits of the sum (round half to even, as the
@@ -347,11 +342,6 @@ __global__ void k_pme_zero64(unsigned long long *p, size_t n)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0ull;
-}
-
-__global__ void k_pme_zero_count(int *c)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0;
 }
 
 // X: K0 x K1 x (K2/2+1) half spectrum; G same layout (real).  part (when the
@@ -705,19 +695,18 @@ int gcmc_pme_gather(gcmc_pme *p, int n, const float *xyz, float *phi, void *stre
 
 namespace gcmc_internal {
 // for the engine's Ewald mode: potential grid, grid shape, spread of a
-// device-counted list, counter reset
+// device-counted list
 const float *pme_phi(const gcmc_pme *p) { return p->Phi; }
 const float *pme_kernel(const gcmc_pme *p) { return p->Gk; }
 void pme_grid(const gcmc_pme *p, int K[3])
 {
     for (int i = 0; i < 3; ++i) K[i] = p->geo.K[i];
 }
-int pme_spread_counted(gcmc_pme *p, int cap, const int *count, const float4 *xyzq, int *reset, hipStream_t s)
+int pme_spread_counted(gcmc_pme *p, int cap, const int *count, const float4 *xyzq, hipStream_t s)
 {
     if (cap > 0)
         hipLaunchKernelGGL(gcmc_pme_k::k_pme_spread, dim3(std::min((cap + 3) / 4, 256)), dim3(256), 0, s, cap, count, xyzq, p->geo,
                            p->Qi);
-    if (reset) hipLaunchKernelGGL(gcmc_pme_k::k_pme_zero_count, dim3(1), dim3(64), 0, s, reset);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : pme_hip(e, "PME spread");
 }

@@ -54,14 +54,17 @@ __device__ inline float gather(const float *Phi, const int K[3], const float L[3
     spline4(scaled(y, L[1], K[1]), K[1], f1, w1);
     spline4(scaled(z, L[2], K[2]), K[2], f2, w2);
     float s = 0.0f;
+#pragma unroll
     for (int i0 = 0; i0 < 4; ++i0) {
         int k0 = f0 - i0;
         k0 += k0 < 0 ? K[0] : 0;
+#pragma unroll
         for (int i1 = 0; i1 < 4; ++i1) {
             int k1 = f1 - i1;
             k1 += k1 < 0 ? K[1] : 0;
             const float *row = Phi + ((size_t)k0 * K[1] + k1) * K[2];
             float r = 0.0f;
+#pragma unroll
             for (int i2 = 0; i2 < 4; ++i2) {
                 int k2 = f2 - i2;
                 k2 += k2 < 0 ? K[2] : 0;
@@ -73,6 +76,47 @@ __device__ inline float gather(const float *Phi, const int K[3], const float L[3
     return s;
 }
 
+// element i of a 4-vector held in registers (no indexed registers)
+__device__ inline float pick4(const float w[4], int i)
+{
+    const float a = (i & 1) ? w[1] : w[0], b = (i & 1) ? w[3] : w[2];
+    return (i & 2) ? b : a;
+}
+
+// gather() by 16 lanes (sub = lane & 15), each one z row of the 4 x 4; the rows
+// are added in gather()'s order, so every lane has its value bit for bit
+__device__ inline float gather16(const float *Phi, const int K[3], const float L[3], float x, float y, float z, int sub)
+{
+    int f0, f1, f2;
+    float w0[4], w1[4], w2[4];
+    spline4(scaled(x, L[0], K[0]), K[0], f0, w0);
+    spline4(scaled(y, L[1], K[1]), K[1], f1, w1);
+    spline4(scaled(z, L[2], K[2]), K[2], f2, w2);
+    int k0 = f0 - (sub >> 2), k1 = f1 - (sub & 3);
+    k0 += k0 < 0 ? K[0] : 0;
+    k1 += k1 < 0 ? K[1] : 0;
+    const float *row = Phi + ((size_t)k0 * K[1] + k1) * K[2];
+    float v[4], r = 0.0f;
+#pragma unroll
+    for (int i2 = 0; i2 < 4; ++i2) v[i2] = row[f2 - i2 + (f2 - i2 < 0 ? K[2] : 0)];
+#pragma unroll
+    for (int i2 = 0; i2 < 4; ++i2) r = fmaf(w2[i2], v[i2], r);
+    const float w = pick4(w0, sub >> 2) * pick4(w1, sub & 3);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s = fmaf(__shfl(w, j, 16), __shfl(r, j, 16), s);
+    return s;
+}
+
+// d modulo K for d in [-2 K, 2 K) (no integer remainder: a slab below would
+// spend 98 of them, some 4,000 instructions)
+__device__ inline int wrapped(int d, int K)
+{
+    d += d < 0 ? K : 0;
+    d += d < 0 ? K : 0;
+    return d >= K ? d - K : d;
+}
+
 // Potential at x of a unit charge at y as the grid represents it:
 // sum_{k, k'} W_x(k) W_y(k') Gk(k - k'), with Gk = IFFT(G) the periodic grid
 // kernel.  The weights factor per axis, so the 64 x 64 terms collapse to
@@ -82,31 +126,40 @@ __device__ inline float gather(const float *Phi, const int K[3], const float L[3
 __device__ inline float pair_kernel_slab(const float *Gk, const int K[3], const float L[3], const float x[3],
                                          const float y[3], int j0)
 {
-    int fx[3], fy[3];
-    float wx[3][4], wy[3][4], c[3][7];
+    int df[3];
+    float c[3][7];
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
-        spline4(scaled(x[a], L[a], K[a]), K[a], fx[a], wx[a]);
-        spline4(scaled(y[a], L[a], K[a]), K[a], fy[a], wy[a]);
+        int fx, fy;
+        float wx[4], wy[4];
+        spline4(scaled(x[a], L[a], K[a]), K[a], fx, wx);
+        spline4(scaled(y[a], L[a], K[a]), K[a], fy, wy);
+        df[a] = fx - fy;
+#pragma unroll
         for (int j = 0; j < 7; ++j) c[a][j] = 0.0f;
+#pragma unroll
         for (int i = 0; i < 4; ++i)
-            for (int ii = 0; ii < 4; ++ii) c[a][i - ii + 3] += wx[a][i] * wy[a][ii];
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) c[a][i - ii + 3] += wx[i] * wy[ii];
     }
-    int d0 = (fx[0] - fy[0]) - (j0 - 3);
-    d0 = ((d0 % K[0]) + K[0]) % K[0];
+    const int d0 = wrapped(df[0] - (j0 - 3), K[0]);
+    float c0 = c[0][0];
+#pragma unroll
+    for (int j = 1; j < 7; ++j) c0 = j == j0 ? c[0][j] : c0;
+    int d2[7];
+#pragma unroll
+    for (int j2 = 0; j2 < 7; ++j2) d2[j2] = wrapped(df[2] - (j2 - 3), K[2]);
     float s = 0.0f;
+#pragma unroll
     for (int j1 = 0; j1 < 7; ++j1) {
-        int d1 = (fx[1] - fy[1]) - (j1 - 3);
-        d1 = ((d1 % K[1]) + K[1]) % K[1];
+        const int d1 = wrapped(df[1] - (j1 - 3), K[1]);
         const float *row = Gk + ((size_t)d0 * K[1] + d1) * K[2];
         float r = 0.0f;
-        for (int j2 = 0; j2 < 7; ++j2) {
-            int d2 = (fx[2] - fy[2]) - (j2 - 3);
-            d2 = ((d2 % K[2]) + K[2]) % K[2];
-            r = fmaf(c[2][j2], row[d2], r);
-        }
+#pragma unroll
+        for (int j2 = 0; j2 < 7; ++j2) r = fmaf(c[2][j2], row[d2[j2]], r);
         s = fmaf(c[1][j1], r, s);
     }
-    return c[0][j0] * s;
+    return c0 * s;
 }
 
 }  // namespace gcmc_spline

@@ -186,3 +186,25 @@ def test_ewald_and_plain_systems_do_not_mix_in_batched_form():
         eng.run(5, 'batched')
     eng.run(5, 'plain')
     eng.close()
+
+
+@pytest.mark.parametrize('chunks', [(1, 2, 3), (9, 200), (300,)])
+def test_ewald_rounds_of_unequal_schedules_equal_plain(chunks):
+    """The batched and graph forms go in rounds that end where a system's
+    charges change, until the longest schedule is done: systems that end at
+    different moves (one of them before a chunk, one within), fewer moves than a
+    chunk of rounds has, and runs past the end, bit for bit the plain form."""
+    a = systems.copy(_state())
+    a['moves'] = a['moves'][:37].copy()
+    b = systems.multi(nsteps=400, n_fixed=1200, box=30.0, seed=78, conf_scale=0.2)
+    b['moves'] = b['moves'][:210].copy()
+    c = systems.copy(_state())
+    c['moves'] = c['moves'][:4].copy()
+    gp, phip, _, stp = _ewald_run([a, b, c], 'plain', chunks)
+    for mode in ('batched', 'graph'):
+        g, phi, _, st = _ewald_run([a, b, c], mode, chunks)
+        for r in range(3):
+            assert np.array_equal(g[r]['atoms'].view(np.uint8), gp[r]['atoms'].view(np.uint8)), (mode, r)
+            assert np.array_equal(phi[r].view(np.uint32), phip[r].view(np.uint32)), (mode, r)
+            assert st[r]['energy'] == stp[r]['energy']
+            assert np.array_equal(st[r]['attempts'], stp[r]['attempts'])
