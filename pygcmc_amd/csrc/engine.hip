@@ -141,6 +141,44 @@ void pme_grid(const gcmc_pme *p, int K[3]);
 int pme_spread_counted(gcmc_pme *p, int cap, const int *count, const float4 *xyzq, hipStream_t s);
 }  // namespace gcmc_internal
 
+// Buffers of an engine for given poses (inputs, then results), kept from call to
+// call.  A few poses (POSE_DIRECT) stay in pinned memory, where the kernel itself
+// reads the inputs and writes the results: 201 methanol poses take 37 us, 118 with
+// buffers allocated per call and six copies.  More go to device memory, at most
+// POSE_CHUNK at a time.
+constexpr int POSE_CHUNK = 65536;
+constexpr size_t POSE_DIRECT = 1 << 20;   // bytes of inputs and results
+
+struct PoseWork {
+    std::mutex lock;   // one call at a time
+    char *pinned = nullptr, *dev = nullptr;
+    size_t pinned_bytes = 0, dev_bytes = 0;
+
+    void release()
+    {
+        if (pinned) (void)hipHostFree(pinned);
+        if (dev) (void)hipFree(dev);
+        pinned = dev = nullptr;
+        pinned_bytes = dev_bytes = 0;
+    }
+    hipError_t reserve(size_t bytes)
+    {
+        const bool direct = bytes <= POSE_DIRECT;
+        char *&p = direct ? pinned : dev;
+        size_t &have = direct ? pinned_bytes : dev_bytes;
+        if (bytes <= have) return hipSuccess;
+        if (p) (void)(direct ? hipHostFree(p) : hipFree(p));
+        p = nullptr;
+        have = 0;
+        size_t want = 65536;
+        while (want < bytes) want *= 2;
+        const hipError_t e = direct ? hipHostMalloc(&p, want, hipHostMallocDefault) : hipMalloc(&p, want);
+        if (e == hipSuccess) have = want;
+        else p = nullptr;
+        return e;
+    }
+};
+
 struct gcmc_engine {
     gcmc_tuning tune{};
     std::vector<HostRep *> reps;
@@ -186,6 +224,7 @@ struct gcmc_engine {
         std::vector<std::pair<int, int>> tried;
         int runs = 0;
     } xs;
+    PoseWork poses;
     double *d_adj_work = nullptr;  // column-sum partials of the adjoint backward
     size_t adj_work_n = 0;
 };
@@ -827,29 +866,32 @@ template <int NT, bool S>
 struct RunEwaldRounds {
     static void run(gcmc_engine *E, int n) { launch_ewald_rounds<NT, S>(E, n); }
 };
-// Poses from which one wave each fills the GPU; fewer are shared by four waves.
-constexpr int POSE_WAVES = 4096;
+// Poses from which one wave each is faster; fewer are shared by four waves (a call
+// with benzene poses: 38 against 42 us at 700, 47 against 42 at 1,024, 70 against
+// 52 at 2,000).
+constexpr int POSE_WAVES = 1024;
 constexpr int ADJ_WAVES = 2048;   // the same for gradients
 
 template <int NT, bool S>
 struct RunPoses {
     template <int TM>
-    static void launch(gcmc_engine *E, int npose, int r, int species, const float *dc, const float *dp, const int *dx,
-                       double *de, int *dn, uint32_t *dh)
+    static void launch(gcmc_engine *E, int total, int npose, int r, int species, const float *dc, const float *dp,
+                       const int *dx, double *de, int *dn, uint32_t *dh)
     {
         // every workgroup stages the tables: no more of them than run at once
-        const bool few = npose < POSE_WAVES;
+        const bool few = total < POSE_WAVES;
         const int per = NT / 64 / (few ? COOP : 1), most = std::max(E->ncu, 1) * (1024 / NT);
         hipLaunchKernelGGL((few ? k_eval_poses<NT, S, TM, COOP> : k_eval_poses<NT, S, TM, 1>),
                            dim3(std::min((npose + per - 1) / per, most)), dim3(NT), E->lay.total, E->stream, E->d_rep, r,
                            species, npose, dc, dp, dx, de, dn, dh, E->lay);
     }
-    static void run(gcmc_engine *E, int npose, int r, int species, const float *dc, const float *dp, const int *dx,
-                    double *de, int *dn, uint32_t *dh)
+    // npose poses of a call with `total`
+    static void run(gcmc_engine *E, int total, int npose, int r, int species, const float *dc, const float *dp,
+                    const int *dx, double *de, int *dn, uint32_t *dh)
     {
-        if (E->reps[r]->pme) launch<T_EWALD>(E, npose, r, species, dc, dp, dx, de, dn, dh);
-        else if (E->tune.fp32_coulomb) launch<T_FP32>(E, npose, r, species, dc, dp, dx, de, dn, dh);
-        else launch<T_FP64>(E, npose, r, species, dc, dp, dx, de, dn, dh);
+        if (E->reps[r]->pme) launch<T_EWALD>(E, total, npose, r, species, dc, dp, dx, de, dn, dh);
+        else if (E->tune.fp32_coulomb) launch<T_FP32>(E, total, npose, r, species, dc, dp, dx, de, dn, dh);
+        else launch<T_FP64>(E, total, npose, r, species, dc, dp, dx, de, dn, dh);
     }
 };
 
@@ -1087,6 +1129,7 @@ int gcmc_engine_destroy(gcmc_engine *E)
     if (E->d_state_snap) hipFree(E->d_state_snap);
     if (E->d_adj_work) hipFree(E->d_adj_work);
     if (E->steps_host) hipHostFree(E->steps_host);
+    E->poses.release();
     if (E->ev0) hipEventDestroy(E->ev0);
     if (E->ev1) hipEventDestroy(E->ev1);
     if (E->evk0) hipEventDestroy(E->evk0);
@@ -1648,28 +1691,49 @@ int gcmc_engine_eval_poses(gcmc_engine *E, int r, int species, int npose, const 
     if (npose == 0) return 0;
     if (!centres || !poses || !energy) return fail(GCMC_E_ARG, "null array");
     const int nf = H.frag[species].num_atoms;
-    std::vector<int> ex(npose, -1);
-    if (exclude) ex.assign(exclude, exclude + npose);
-    DevBuf B;
-    float *dc = nullptr, *dp = nullptr;
-    int *dx = nullptr, *dn = nullptr;
-    double *de = nullptr;
-    uint32_t *dh = nullptr;
-    hipError_t e = put(&dc, B, centres, 3 * (size_t)npose);
-    if (e == hipSuccess) e = put(&dp, B, poses, 3 * (size_t)npose * nf);
-    if (e == hipSuccess) e = put(&dx, B, ex.data(), ex.size());
-    if (e == hipSuccess) e = B.alloc(&de, npose);
-    if (e == hipSuccess) e = B.alloc(&dn, npose);
-    if (e == hipSuccess) e = B.alloc(&dh, npose);
-    if (e == hipSuccess) {
-        dispatch<RunPoses>(E, npose, r, species, (const float *)dc, (const float *)dp, (const int *)dx, de, dn, dh);
+    PoseWork &P = E->poses;
+    std::lock_guard<std::mutex> own(P.lock);
+    // energies, counts, hashes; centres, poses, excluded molecules
+    const size_t per = sizeof(double) + 2 * sizeof(int) + (3 + 3 * nf + 1) * sizeof(float);
+    hipError_t e = P.reserve(per * std::min(npose, POSE_CHUNK));
+    const bool direct = per * std::min(npose, POSE_CHUNK) <= POSE_DIRECT;
+    std::vector<int> none;
+    for (int first = 0; first < npose && e == hipSuccess; first += POSE_CHUNK) {
+        const size_t n = std::min(npose - first, POSE_CHUNK);
+        double *de = (double *)(direct ? P.pinned : P.dev);
+        int *dn = (int *)(de + n);
+        uint32_t *dh = (uint32_t *)(dn + n);
+        float *dc = (float *)(dh + n), *dp = dc + 3 * n;
+        int *dx = (int *)(dp + 3 * n * nf);
+        const float *c = centres + 3 * (size_t)first, *p = poses + 3 * (size_t)first * nf;
+        if (direct) {
+            std::memcpy(dc, c, 3 * n * sizeof(float));
+            std::memcpy(dp, p, 3 * n * nf * sizeof(float));
+            if (exclude) std::memcpy(dx, exclude + first, n * sizeof(int));
+            else std::fill(dx, dx + n, -1);
+        } else {
+            if (!exclude) none.assign(n, -1);
+            e = hipMemcpyAsync(dc, c, 3 * n * sizeof(float), hipMemcpyHostToDevice, E->stream);
+            if (e == hipSuccess) e = hipMemcpyAsync(dp, p, 3 * n * nf * sizeof(float), hipMemcpyHostToDevice, E->stream);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(dx, exclude ? exclude + first : none.data(), n * sizeof(int), hipMemcpyHostToDevice,
+                                   E->stream);
+        }
+        if (e != hipSuccess) break;
+        dispatch<RunPoses>(E, npose, (int)n, r, species, (const float *)dc, (const float *)dp, (const int *)dx, de, dn, dh);
         e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(E->stream);
+        if (e != hipSuccess) break;
+        auto out = [&](void *to, const void *from, size_t bytes) {
+            if (!to || e != hipSuccess) return;
+            if (direct) std::memcpy(to, from, bytes);
+            else e = hipMemcpy(to, from, bytes, hipMemcpyDeviceToHost);
+        };
+        out(energy + first, de, n * sizeof(double));
+        out(ninc ? ninc + first : nullptr, dn, n * sizeof(int));
+        out(inchash ? inchash + first : nullptr, dh, n * sizeof(uint32_t));
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(E->stream);
-    if (e == hipSuccess) e = hipMemcpy(energy, de, npose * sizeof(double), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && ninc) e = hipMemcpy(ninc, dn, npose * sizeof(int), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && inchash) e = hipMemcpy(inchash, dh, npose * sizeof(uint32_t), hipMemcpyDeviceToHost);
-    B.release();
+    if (e != hipSuccess) (void)hipStreamSynchronize(E->stream);
     if (e != hipSuccess) return fail(GCMC_E_HIP, std::string("eval_poses: ") + hipGetErrorString(e));
     return 0;
 }

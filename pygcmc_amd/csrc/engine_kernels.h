@@ -2339,6 +2339,12 @@ __global__ void k_xcc_probe(int *out)
     if (threadIdx.x == 0) out[blockIdx.x] = my_xcc();
 }
 
+// lane i's value, in every lane
+__device__ __forceinline__ float lane_f(float x, int i)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), i));
+}
+
 // Energies of given poses: one wave per pose, or (few poses) four that share
 // its cells.
 template <int NT, bool STAGED, int TM, int PARTS>
@@ -2353,16 +2359,38 @@ __global__ __launch_bounds__(NT) void k_eval_poses(const Rep *reps, int r, int s
     CSpecies &F = species_of(C, spi);
     const int nf = F.nf, lane = threadIdx.x & 63, wave = uniform_i(threadIdx.x >> 6), part = wave % PARTS;
     const WaveLds W = wave_lds(L, wave);
+    if (threadIdx.x == 0) L.misc[M_NEXT] = PER;
     stage_tables<NT, STAGED>(C, L, true, true);
-    for (int i0 = blockIdx.x * PER; i0 < npose; i0 += gridDim.x * PER) {
-        const int i = i0 + wave / PARTS, q = min(i, npose - 1), x = uniform_i(excl[q]);
-        if (PARTS == 1 && i >= npose) break;
-        const float c[3] = {uniform_f(centres[3 * (size_t)q]), uniform_f(centres[3 * (size_t)q + 1]),
-                            uniform_f(centres[3 * (size_t)q + 2])};
-        if (lane < nf) {
-            const float *p = poses + ((size_t)q * nf + lane) * 3;
-            order_pose<TM>(C, F, W, 0, lane, make_float4(p[0], p[1], p[2], F.kq[lane]), c);
-        }
+    // this workgroup's poses; with one wave per pose each takes the next one when
+    // it is done (in turn: 133 us for 16,384 benzene poses, a wave with costly
+    // ones last; so: 106)
+    const int p0 = (int)((long long)npose * blockIdx.x / gridDim.x);
+    const int p1 = (int)((long long)npose * (blockIdx.x + 1) / gridDim.x);
+    // a pose by one load per lane: 3 nf coordinates, the centre, the excluded
+    // molecule (the arrays may lie in host memory)
+    auto fetch = [&](int k) {
+        const size_t q = (size_t)min(p0 + k, p1 - 1);
+        const int *src = (const int *)poses + q * 3 * nf + lane;
+        if (lane >= 60) src = lane < 63 ? (const int *)centres + 3 * q + (lane - 60) : excl + q;
+        return lane < 3 * nf || lane >= 60 ? *src : 0;
+    };
+    auto next = [&](int k) {
+        if (PARTS > 1) return k + PER;
+        int n = 0;
+        if (lane == 0) n = atomicAdd(&L.misc[M_NEXT], 1);
+        return uniform_i(n);
+    };
+    int k = wave / PARTS;
+    if (p0 >= p1) return;
+    int in = fetch(k);
+    while (p0 + (PARTS == 1 ? k : k - wave / PARTS) < p1) {
+        const int i = p0 + k, kn = next(k), v = in;
+        in = fetch(kn);
+        const float vf = __int_as_float(v), c[3] = {lane_f(vf, 60), lane_f(vf, 61), lane_f(vf, 62)};
+        const int x = __builtin_amdgcn_readlane(v, 63);
+        const float px = __shfl(vf, min(3 * lane, 63)), py = __shfl(vf, min(3 * lane + 1, 63)),
+                    pz = __shfl(vf, min(3 * lane + 2, 63));
+        if (lane < nf) order_pose<TM>(C, F, W, 0, lane, make_float4(px, py, pz, F.kq[lane]), c);
         wave_sync();
         PoseSums s;
         eval_poses_wave<STAGED, TM>(C, L, W, spi, nf, 1, c, c, true, x, false, part, PARTS, s);
@@ -2371,12 +2399,13 @@ __global__ __launch_bounds__(NT) void k_eval_poses(const Rep *reps, int r, int s
             s.e[0] += ewald_recip(C, F, W, 0, nf, own ? F.atomBase + (x - F.startRes) * nf : -1, part, PARTS);
         }
         if (PARTS > 1) team_sum<NT>(L, s);
-        if (i < npose && part == 0 && lane == 0) {
+        if (i < p1 && part == 0 && lane == 0) {
             E[i] = s.e[0];
             ninc[i] = s.nin[0];
             hash[i] = s.hash[0];
         }
         wave_sync();
+        k = kn;
     }
 }
 

@@ -53,6 +53,27 @@ def test_eval_poses_matches_fp64():
     eng.close()
 
 
+@pytest.mark.parametrize('n', [1, 5, 1023, 1024, 1025, 16000])
+def test_eval_poses_by_number(n):
+    """Poses shared by four waves (fewer than 1,024) or one wave's, one call's in
+    pinned memory or (16,000: above 1 MiB) in device memory: every form gives the
+    groups of a pose exactly and its energy to the order of an FP64 sum."""
+    s = systems.populated_water()
+    eng = Engine()
+    eng.add_system(s)
+    eng.upload()
+    c, p = systems.random_poses(s, 0, 1024, seed=9)
+    parts = [eng.eval_poses(0, 0, c[i:i + 64], p[i:i + 64]) for i in range(0, 1024, 64)]
+    ref = [np.concatenate([x[k] for x in parts]) for k in range(3)]
+    q = np.random.default_rng(n).integers(0, 1024, n)
+    E, N, H = eng.eval_poses(0, 0, c[q], p[q])
+    assert np.array_equal(N, ref[1][q]) and np.array_equal(H, ref[2][q])
+    # at most some 1,000 FP64 terms, the largest not above 100 times the sum of
+    # a pose that matters: 1e-10 of the energy, or of 1 kJ/mol
+    assert (np.abs(E - ref[0][q]) <= 1e-10 * np.maximum(np.abs(ref[0][q]), 1.0)).all()
+    eng.close()
+
+
 def test_water_fixture_on_gpu():
     """The reference's 3-water insertion (test/water/3water.pdb) on the GPU."""
     for ch, lj, key in ((True, False, 'expected_coulomb_kj'), (False, True, 'expected_lj_kj')):
