@@ -239,6 +239,11 @@ int gcmc_engine_adjoint(gcmc_engine *e, int replica, int species, int npose,
 int gcmc_engine_adjoint_backward(gcmc_engine *e, int npose, int per_pose, int ncol,
                                  const float *dEdx, const float *partial, const float *weights,
                                  float *grad_pose, float *grad_cols, void *stream);
+/* The same with FP64 weights, each rounded to FP32 where it is used (the energies
+ * are FP64, and so are the gradients that a loss hands back for them). */
+int gcmc_engine_adjoint_backward64(gcmc_engine *e, int npose, int per_pose, int ncol,
+                                   const float *dEdx, const float *partial, const double *weights,
+                                   float *grad_pose, float *grad_cols, void *stream);
 
 /* The same backward without any allocation: no counterpart in the reference
  * (pyGCMC has no adjoint); for callers that cannot allocate device memory --

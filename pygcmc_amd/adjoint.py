@@ -32,7 +32,7 @@ def _lib():
     if not getattr(L, '_adjoint_types_set', False):
         P, I = ctypes.c_void_p, ctypes.c_int
         L.gcmc_engine_adjoint.argtypes = [P, I, I, I, P, P, P, P, P, P, P, P, P]
-        L.gcmc_engine_adjoint_backward.argtypes = [P, I, I, I, P, P, P, P, P, P]
+        L.gcmc_engine_adjoint_backward64.argtypes = [P, I, I, I, P, P, P, P, P, P]
         L._adjoint_types_set = True
     return L
 
@@ -79,13 +79,13 @@ class PoseEnergy(torch.autograd.Function):
         dEdx, partial = ctx.saved_tensors
         n, nf, _ = dEdx.shape
         Y = ctx.Y
-        w = gE.to(torch.float32).contiguous()
+        w = gE.to(torch.float64).contiguous()   # (rounded to float32 where it is used)
         gpose = torch.empty_like(dEdx)
         gcols = torch.empty(3 * Y, dtype=torch.float32, device=dEdx.device)
         stream = ctypes.c_void_p(torch.cuda.current_stream(dEdx.device).cuda_stream)
-        _engine._check(_lib().gcmc_engine_adjoint_backward(ctx.eng._h, n, nf * 3, 3 * Y, _ptr(dEdx),
-                                                           _ptr(partial), _ptr(w), _ptr(gpose), _ptr(gcols),
-                                                           stream))
+        _engine._check(_lib().gcmc_engine_adjoint_backward64(ctx.eng._h, n, nf * 3, 3 * Y, _ptr(dEdx),
+                                                             _ptr(partial), _ptr(w), _ptr(gpose), _ptr(gcols),
+                                                             stream))
         gq, ge, gr = gcols.view(3, Y)
         return gpose, ge, gr, gq, None, None, None, None
 

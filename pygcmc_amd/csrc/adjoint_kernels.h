@@ -207,6 +207,7 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         P.A.dq[t] = dq ? dq[t] : 0.0f;
     }
     load_species_table(C, L);
+    if (tid == 0) L.misc[M_NEXT] = PER;
     // pair entries in FP64, rounded once to FP32 (as a host-built table is)
     for (int q = tid; q < X * Y; q += NT) {
         const int x = q / Y, y = q - x * Y;
@@ -217,15 +218,35 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         P.A.tab[q] = make_float4(hi, (float)(4.0 * sqrt(ee)), (float)(s2 - (double)hi), 0.0f);
     }
     __syncthreads();
-    for (int i0 = blockIdx.x * PER; i0 < npose; i0 += gridDim.x * PER) {
-        const int i = i0 + wave / PARTS, q = min(i, npose - 1);
-        if (PARTS == 1 && i >= npose) break;
-        const float c[3] = {uniform_f(centres[3 * (size_t)q]), uniform_f(centres[3 * (size_t)q + 1]),
-                            uniform_f(centres[3 * (size_t)q + 2])};
+    // this workgroup's poses; with one wave per pose each takes the next one when
+    // it is done
+    const int p0 = (int)((long long)npose * blockIdx.x / gridDim.x);
+    const int p1 = (int)((long long)npose * (blockIdx.x + 1) / gridDim.x);
+    // a pose by one load per lane: 3 nf coordinates, the centre
+    auto fetch = [&](int k) {
+        const size_t q = (size_t)min(p0 + k, p1 - 1);
+        const float *src = poses + q * 3 * nf + lane;
+        if (lane >= 60) src = centres + 3 * q + min(lane - 60, 2);
+        return lane < 3 * nf || lane >= 60 ? *src : 0.0f;
+    };
+    int k = wave / PARTS;
+    if (p0 >= p1) return;
+    float in = fetch(k);
+    while (p0 + (PARTS == 1 ? k : k - wave / PARTS) < p1) {
+        const int i = p0 + k;
+        int kn = k + PER;
+        if (PARTS == 1) {
+            if (lane == 0) kn = atomicAdd(&L.misc[M_NEXT], 1);
+            kn = uniform_i(kn);
+        }
+        const float v = in;
+        in = fetch(kn);
+        const float c[3] = {lane_f(v, 60), lane_f(v, 61), lane_f(v, 62)};
+        const float px = __shfl(v, min(3 * lane, 63)), py = __shfl(v, min(3 * lane + 1, 63)),
+                    pz = __shfl(v, min(3 * lane + 2, 63));
         if (lane < nf) {
-            const float *p = poses + ((size_t)q * nf + lane) * 3;
             const float kq = dq ? KCOUL_F * (F.tmpl[lane].w + dq[F.ttype[lane]]) : F.kq[lane];
-            ((float4 *)W.fragd)[F.slot[lane]] = make_float4(p[0], p[1], p[2], kq);
+            ((float4 *)W.fragd)[F.slot[lane]] = make_float4(px, py, pz, kq);
         }
         if (part == 0)
             for (int t = lane; t < 3 * Y + 6 * MAXF; t += 64) P.A.gq[t] = 0.0f;
@@ -262,7 +283,7 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
                 for (int k = 0; k < 6; ++k) s[k] = P.A.red[6 * lane + k];
         }
         wave_sync();
-        if (part == 0 && i < npose) {
+        if (part == 0 && i < p1) {
             // the place's atom (Species::slot is the other way round)
             if (lane < nf) {
                 int a = 0;
@@ -283,48 +304,69 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         }
         wave_sync();
         if (PARTS > 1) __syncthreads();
+        k = kn;
     }
 }
 
-// tmp[c][j] = sum over poses p of chunk c of w[p] partial[p][j] (FP64);
-// block (64 columns x 16 pose lanes), grid (column blocks, chunks)
-__global__ __launch_bounds__(1024) void k_adjoint_colsum(int npose, int m, const float *partial, const float *w,
-                                                        double *tmp)
+// The backward in one launch, or two when there are many poses (three, with the
+// chunks' sums one after another, took 13 us for 64 poses):
+//   workgroups 0 .. nscale - 1: grad[p][k] = w[p] dEdx[p][k], 4096 elements each;
+//   the others, 64 columns of a chunk of poses each, 16 poses at a time: the sum
+//   over the chunk's poses of w[p] partial[p][j] (FP64), to `out` when there is one
+//   chunk, else to tmp[chunk][j], which k_adjoint_chunksum adds up.
+constexpr int BACK_SCALE = 4096;
+
+template <class W>   // weights are rounded to FP32
+__global__ __launch_bounds__(1024) void k_adjoint_back(int npose, int per, int m, int nscale, int nch,
+                                                      const float *dEdx, const float *partial, const W *w,
+                                                      float *grad, double *tmp, float *out)
 {
     __shared__ double red[16][64];
-    const int j = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int pl = threadIdx.x >> 6;
-    const int nch = gridDim.y;
-    const int per = (npose + nch - 1) / nch;
-    const int p0 = blockIdx.y * per, p1 = min(npose, p0 + per);
+    if ((int)blockIdx.x < nscale) {
+        const size_t n = (size_t)npose * per;
+#pragma unroll
+        for (int k = 0; k < BACK_SCALE; k += 1024) {
+            const size_t q = (size_t)blockIdx.x * BACK_SCALE + k + threadIdx.x;
+            if (q < n) grad[q] = (w ? (float)w[q / per] : 1.0f) * dEdx[q];
+        }
+        return;
+    }
+    const int ncb = (m + 63) / 64, b = blockIdx.x - nscale, ch = b / ncb;
+    const int j = (b - ch * ncb) * 64 + (threadIdx.x & 63), pl = threadIdx.x >> 6;
+    const int each = (npose + nch - 1) / nch, p0 = ch * each, p1 = min(npose, p0 + each);
     double s = 0.0;
-    if (j < m)
-        for (int p = p0 + pl; p < p1; p += 16) s += (double)(w ? w[p] : 1.0f) * (double)partial[(size_t)p * m + j];
+    if (j < m) {
+#pragma unroll 4
+        for (int p = p0 + pl; p < p1; p += 16) s += (double)(w ? (float)w[p] : 1.0f) * (double)partial[(size_t)p * m + j];
+    }
     red[pl][threadIdx.x & 63] = s;
     __syncthreads();
     if (pl == 0 && j < m) {
         double t = 0.0;
+#pragma unroll
         for (int q = 0; q < 16; ++q) t += red[q][threadIdx.x & 63];
-        tmp[(size_t)blockIdx.y * m + j] = t;
+        if (nch == 1) out[j] = (float)t;
+        else tmp[(size_t)ch * m + j] = t;
     }
 }
 
-__global__ void k_adjoint_chunksum(int nch, int m, const double *tmp, float *out)
+// out[j] = sum over the chunks of tmp[c][j]: 64 columns per workgroup, 16 chunks at
+// a time (one thread per column: 8.4 us for 32 chunks)
+__global__ __launch_bounds__(1024) void k_adjoint_chunksum(int nch, int m, const double *tmp, float *out)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= m) return;
-    double t = 0.0;
-    for (int c = 0; c < nch; ++c) t += tmp[(size_t)c * m + j];
-    out[j] = (float)t;
-}
-
-// out[p][k] = w[p] x[p][k]
-__global__ void k_scale_rows(int npose, int per, const float *x, const float *w, float *out)
-{
-    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (size_t)npose * per) return;
-    const int p = (int)(q / per);
-    out[q] = (w ? w[p] : 1.0f) * x[q];
+    __shared__ double red[16][64];
+    const int j = blockIdx.x * 64 + (threadIdx.x & 63), cl = threadIdx.x >> 6;
+    double s = 0.0;
+    if (j < m)
+        for (int c = cl; c < nch; c += 16) s += tmp[(size_t)c * m + j];
+    red[cl][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (cl == 0 && j < m) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) t += red[q][threadIdx.x & 63];
+        out[j] = (float)t;
+    }
 }
 
 }  // namespace gcmc

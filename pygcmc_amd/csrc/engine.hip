@@ -872,6 +872,24 @@ struct RunEwaldRounds {
 constexpr int POSE_WAVES = 1024;
 constexpr int ADJ_WAVES = 2048;   // the same for gradients
 
+// The adjoint's backward: poses are summed in chunks of 64 to ADJ_CHUNKS chunks,
+// work holding ADJ_CHUNKS x ncol sums.
+constexpr int ADJ_CHUNKS = 32;
+
+template <class W>
+void launch_backward(int npose, int per_pose, int ncol, const float *dEdx, const float *partial, const W *weights,
+                     float *grad_pose, float *grad_cols, double *work, hipStream_t s)
+{
+    const size_t nx = (size_t)npose * per_pose;
+    const int nscale = (int)((nx + BACK_SCALE - 1) / BACK_SCALE), ncb = (ncol + 63) / 64;
+    const int nch = std::min(std::max((npose + 63) / 64, 1), ADJ_CHUNKS);
+    if (nscale + ncb == 0) return;
+    hipLaunchKernelGGL(k_adjoint_back<W>, dim3(nscale + ncb * nch), dim3(1024), 0, s, npose, per_pose, ncol, nscale, nch,
+                       dEdx, partial, weights, grad_pose, work, grad_cols);
+    if (nch > 1 && ncb > 0)
+        hipLaunchKernelGGL(k_adjoint_chunksum, dim3(ncb), dim3(1024), 0, s, nch, ncol, work, grad_cols);
+}
+
 template <int NT, bool S>
 struct RunPoses {
     template <int TM>
@@ -1842,9 +1860,10 @@ int gcmc_engine_adjoint(gcmc_engine *E, int r, int species, int npose, const flo
     l.adjl = -1;
     l.team = NT / 64 * WL_BYTES;
     l.spt = l.team + NT / 64 * TEAM_BYTES;
-    const int adj_off = l.spt + 16 * MAXT;
+    l.misc = l.spt + 16 * MAXT;
+    const int adj_off = (l.misc + 4 * MISC_INTS + 15) & ~15;
     const int lds = l.total = adj_off + adj_lds_bytes(X, Y, NT / 64);
-    if (lds > 65536) return fail(GCMC_E_ARG, "adjoint LDS layout exceeds 64 KiB (too many atom types)");
+    if (lds > 163840) return fail(GCMC_E_ARG, "adjoint LDS layout exceeds 160 KiB (too many atom types)");
     hipStream_t s = (hipStream_t)stream;
     // one wave per pose when they fill the GPU, else four; no more workgroups
     // than run at once (each builds the pair table)
@@ -1864,17 +1883,19 @@ int gcmc_engine_adjoint(gcmc_engine *E, int r, int species, int npose, const flo
     return 0;
 }
 
-int gcmc_engine_adjoint_backward(gcmc_engine *E, int npose, int per_pose, int ncol, const float *dEdx,
-                                 const float *partial, const float *weights, float *grad_pose, float *grad_cols,
-                                 void *stream)
+}  // extern "C"
+
+namespace {
+template <class W>
+int adjoint_backward(gcmc_engine *E, int npose, int per_pose, int ncol, const float *dEdx, const float *partial,
+                     const W *weights, float *grad_pose, float *grad_cols, void *stream)
 {
     if (!E) return fail(GCMC_E_ARG, "null engine");
     if (npose < 0 || per_pose < 0 || ncol < 0) return fail(GCMC_E_ARG, "negative size");
     if ((npose > 0 && per_pose > 0 && (!dEdx || !grad_pose)) || (ncol > 0 && (!partial || !grad_cols)))
         return fail(GCMC_E_ARG, "null array");
     hipStream_t s = (hipStream_t)stream;
-    constexpr int NCH = 32;
-    const size_t need = (size_t)NCH * std::max(ncol, 1);
+    const size_t need = (size_t)ADJ_CHUNKS * std::max(ncol, 1);
     if (E->adj_work_n < need) {
         if (E->d_adj_work) (void)hipFree(E->d_adj_work);
         E->d_adj_work = nullptr;
@@ -1882,19 +1903,27 @@ int gcmc_engine_adjoint_backward(gcmc_engine *E, int npose, int per_pose, int nc
         HIPX(hipMalloc(&E->d_adj_work, need * sizeof(double)));
         E->adj_work_n = need;
     }
-    const size_t nx = (size_t)npose * per_pose;
-    if (nx > 0)
-        hipLaunchKernelGGL(k_scale_rows, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, s, npose, per_pose, dEdx,
-                           weights, grad_pose);
-    if (ncol > 0) {
-        hipLaunchKernelGGL(k_adjoint_colsum, dim3((ncol + 63) / 64, NCH), dim3(1024), 0, s, npose, ncol, partial,
-                           weights, E->d_adj_work);
-        hipLaunchKernelGGL(k_adjoint_chunksum, dim3((ncol + 255) / 256), dim3(256), 0, s, NCH, ncol, E->d_adj_work,
-                           grad_cols);
-    }
+    launch_backward(npose, per_pose, ncol, dEdx, partial, weights, grad_pose, grad_cols, E->d_adj_work, s);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(GCMC_E_HIP, std::string("adjoint backward: ") + hipGetErrorString(e));
     return 0;
+}
+}  // namespace
+
+extern "C" {
+
+int gcmc_engine_adjoint_backward(gcmc_engine *E, int npose, int per_pose, int ncol, const float *dEdx,
+                                 const float *partial, const float *weights, float *grad_pose, float *grad_cols,
+                                 void *stream)
+{
+    return adjoint_backward(E, npose, per_pose, ncol, dEdx, partial, weights, grad_pose, grad_cols, stream);
+}
+
+int gcmc_engine_adjoint_backward64(gcmc_engine *E, int npose, int per_pose, int ncol, const float *dEdx,
+                                   const float *partial, const double *weights, float *grad_pose, float *grad_cols,
+                                   void *stream)
+{
+    return adjoint_backward(E, npose, per_pose, ncol, dEdx, partial, weights, grad_pose, grad_cols, stream);
 }
 
 }  // extern "C"
@@ -1905,10 +1934,9 @@ int gcmc_engine_adjoint_backward(gcmc_engine *E, int npose, int per_pose, int nc
 // writes all the entries it then reads, so nothing needs clearing; calls
 // that overlap on one device race).
 namespace {
-constexpr int ADJ_NOALLOC_NCH = 32;
 constexpr int ADJ_NOALLOC_MAX_COLS = 4096;
 constexpr int ADJ_NOALLOC_MAX_DEVICES = 64;
-__device__ __align__(256) double scratch[ADJ_NOALLOC_NCH * ADJ_NOALLOC_MAX_COLS];
+__device__ __align__(256) double scratch[ADJ_CHUNKS * ADJ_NOALLOC_MAX_COLS];
 
 std::mutex g_scratch_mu;
 double *g_scratch_ptr[ADJ_NOALLOC_MAX_DEVICES] = {};
@@ -1948,16 +1976,7 @@ int gcmc_adjoint_backward_noalloc(int npose, int per_pose, int ncol, const float
     int rc = scratch_address(&work);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const size_t nx = (size_t)npose * per_pose;
-    if (nx > 0)
-        hipLaunchKernelGGL(k_scale_rows, dim3((unsigned)((nx + 255) / 256)), dim3(256), 0, s, npose, per_pose, dEdx,
-                           weights, grad_pose);
-    if (ncol > 0) {
-        hipLaunchKernelGGL(k_adjoint_colsum, dim3((ncol + 63) / 64, ADJ_NOALLOC_NCH), dim3(1024), 0, s, npose, ncol,
-                           partial, weights, work);
-        hipLaunchKernelGGL(k_adjoint_chunksum, dim3((ncol + 255) / 256), dim3(256), 0, s, ADJ_NOALLOC_NCH, ncol, work,
-                           grad_cols);
-    }
+    launch_backward(npose, per_pose, ncol, dEdx, partial, weights, grad_pose, grad_cols, work, s);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(GCMC_E_HIP, std::string("adjoint backward: ") + hipGetErrorString(e));
     return 0;

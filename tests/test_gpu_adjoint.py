@@ -131,3 +131,46 @@ def test_adjoint_rejects_bad_shapes(case):
                             torch.tensor(p[:, :-1], device='cuda'), eps, rmin)
     with pytest.raises(TypeError):
         adjoint.pose_energy(eng, 0, 0, torch.tensor(c), torch.tensor(p), eps, rmin)
+
+
+@pytest.mark.parametrize('n', [1, 2047, 2048, 2049])
+def test_adjoint_by_number_of_poses(case, n):
+    """Poses shared by four waves (fewer than 2,048) or one wave's: energies to the
+    order of an FP64 sum, coordinate gradients within this file's bar."""
+    s, eng, eps, rmin, poses = case
+    c, p = poses[2]
+    E0, pt0, *_ = _gpu(eng, 2, c, p, eps, rmin)
+    G0, = torch.autograd.grad(E0.sum(), pt0)
+    q = np.random.default_rng(n).integers(0, len(c), n)
+    E, pt, *_ = _gpu(eng, 2, c[q], p[q], eps, rmin)
+    G, = torch.autograd.grad(E.sum(), pt)
+    e0, g0 = E0.detach().cpu().numpy()[q], G0.cpu().numpy()[q].reshape(n, -1)
+    e, g = E.detach().cpu().numpy(), G.cpu().numpy().reshape(n, -1)
+    assert (np.abs(e - e0) <= 1e-10 * np.maximum(np.abs(e0), 1.0)).all()
+    assert (np.linalg.norm(g - g0, axis=1) <= 1e-4 * np.linalg.norm(g0, axis=1)).all()
+
+
+@pytest.mark.parametrize('n,per,m', [(0, 9, 3), (1, 9, 3), (64, 36, 64), (65, 60, 65), (2048, 3, 198), (2111, 9, 1)])
+def test_backward_sums(case, n, per, m):
+    """One chunk of poses (up to 64), several, more than the workspace has chunks
+    for; FP64 weights, rounded to FP32: the scaled rows exactly, column sums to
+    the rounding of their FP32 result and of FP64 additions.  (No poses: torch's
+    empty tensors have no address, which is refused.)"""
+    from pygcmc_amd import engine as _engine
+    eng, L = case[1], adjoint._lib()
+    g = torch.Generator(device='cpu').manual_seed(n)
+    x, y = torch.randn(n, per, generator=g), torch.randn(n, m, generator=g) * 10
+    w = torch.rand(n, generator=g, dtype=torch.float64)
+    xd, yd, wd = x.cuda(), y.cuda(), w.cuda()
+    gp, gc = torch.full((n, per), float('nan'), device='cuda'), torch.full((m,), float('nan'), device='cuda')
+    rc = L.gcmc_engine_adjoint_backward64(eng._h, n, per, m, *(adjoint._ptr(t) for t in (xd, yd, wd, gp, gc)),
+                                          adjoint.ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    if n == 0:
+        assert rc < 0
+        return
+    _engine._check(rc)
+    w32 = w.float()
+    assert torch.equal(gp.cpu(), w32[:, None] * x)
+    terms = w32.double()[:, None] * y.double()
+    ref, size = terms.sum(0), terms.abs().sum(0)
+    assert ((gc.cpu().double() - ref).abs() <= 2.0 ** -24 * ref.abs() * 1.001 + 1e-12 * size).all()
