@@ -179,6 +179,31 @@ struct PoseWork {
     }
 };
 
+// Buffers of an engine's downloads, for its largest system.
+struct Download {
+    std::mutex lock;   // one at a time
+    char *dev = nullptr;
+    size_t bytes = 0;
+    std::vector<char> host;
+
+    void release()
+    {
+        if (dev) (void)hipFree(dev);
+        dev = nullptr;
+        bytes = 0;
+    }
+    hipError_t reserve(size_t head, size_t body)
+    {
+        if (host.size() < head) host.resize(head);
+        if (head + body <= bytes) return hipSuccess;
+        release();
+        const hipError_t e = hipMalloc(&dev, head + body);
+        if (e == hipSuccess) bytes = head + body;
+        else dev = nullptr;
+        return e;
+    }
+};
+
 struct gcmc_engine {
     gcmc_tuning tune{};
     std::vector<HostRep *> reps;
@@ -225,6 +250,7 @@ struct gcmc_engine {
         int runs = 0;
     } xs;
     PoseWork poses;
+    Download down;
     double *d_adj_work = nullptr;  // column-sum partials of the adjoint backward
     size_t adj_work_n = 0;
 };
@@ -1148,6 +1174,7 @@ int gcmc_engine_destroy(gcmc_engine *E)
     if (E->d_adj_work) hipFree(E->d_adj_work);
     if (E->steps_host) hipHostFree(E->steps_host);
     E->poses.release();
+    E->down.release();
     if (E->ev0) hipEventDestroy(E->ev0);
     if (E->ev1) hipEventDestroy(E->ev1);
     if (E->evk0) hipEventDestroy(E->evk0);
@@ -1521,30 +1548,27 @@ int gcmc_engine_download(gcmc_engine *E, int r, AtomArray *frag, residue *res, A
     if (r < 0 || r >= (int)E->reps.size()) return fail(GCMC_E_ARG, "bad replica");
     HostRep &H = *E->reps[r];
     const InfoStruct &I = H.info;
+    Download &D = E->down;
+    std::lock_guard<std::mutex> own(D.lock);
+    // the atoms as the caller's records, copied straight to them; counts and group
+    // centres in one copy to `host`
+    const size_t head = ((size_t)I.fragTypeNum + 3 * (size_t)I.totalResNum) * sizeof(int);
+    const size_t body = (size_t)I.totalAtomNum * sizeof(Atom);
+    HIPX(D.reserve(head, body));
+    const int nwork = std::max(std::max(5 * I.totalAtomNum, 3 * I.totalResNum), I.fragTypeNum);
+    hipLaunchKernelGGL(k_pack_state, dim3((unsigned)std::max((nwork + 255) / 256, 1)), dim3(256), 0, E->stream, E->d_rep,
+                       E->d_state, r, I.fragTypeNum, I.totalResNum, I.totalAtomNum, (int *)D.dev, (int *)(D.dev + head));
+    HIPX(hipGetLastError());
+    HIPX(hipMemcpyAsync(D.host.data(), D.dev, head, hipMemcpyDeviceToHost, E->stream));
+    if (atoms && body) HIPX(hipMemcpyAsync(atoms, D.dev + head, body, hipMemcpyDeviceToHost, E->stream));
     HIPX(hipStreamSynchronize(E->stream));
-    State S;
-    HIPX(hipMemcpy(&S, E->d_state + r, sizeof(S), hipMemcpyDeviceToHost));
-    std::vector<float4> res_pos(I.totalResNum), atom(I.totalAtomNum);
-    std::vector<int> atype(I.totalAtomNum);
-    HIPX(hipMemcpy(res_pos.data(), H.rep.res_pos, res_pos.size() * sizeof(float4), hipMemcpyDeviceToHost));
-    HIPX(hipMemcpy(atom.data(), H.rep.atom, atom.size() * sizeof(float4), hipMemcpyDeviceToHost));
-    HIPX(hipMemcpy(atype.data(), H.rep.atype, atype.size() * sizeof(int), hipMemcpyDeviceToHost));
+    const int *counts = (const int *)D.host.data();
+    const float *centre = (const float *)(counts + I.fragTypeNum);
     if (frag)
-        for (int s = 0; s < I.fragTypeNum; ++s) frag[s].totalNum = S.totalNum[s];
+        for (int s = 0; s < I.fragTypeNum; ++s) frag[s].totalNum = counts[s];
     if (res)
-        for (int g = 0; g < I.totalResNum; ++g) {
-            res[g].position[0] = res_pos[g].x;
-            res[g].position[1] = res_pos[g].y;
-            res[g].position[2] = res_pos[g].z;
-        }
-    if (atoms)
-        for (int a = 0; a < I.totalAtomNum; ++a) {
-            atoms[a].position[0] = atom[a].x;
-            atoms[a].position[1] = atom[a].y;
-            atoms[a].position[2] = atom[a].z;
-            atoms[a].charge = atom[a].w;
-            atoms[a].type = atype[a];
-        }
+        for (int g = 0; g < I.totalResNum; ++g)
+            for (int i = 0; i < 3; ++i) res[g].position[i] = centre[3 * (size_t)g + i];
     return 0;
 }
 
