@@ -83,7 +83,7 @@ const char *gcmc_last_error(void);
 typedef struct gcmc_engine gcmc_engine;
 
 typedef struct gcmc_tuning {
-    float cell_size;     /* target edge (A) of the group-centre cell list; 0 = 5 A */
+    float cell_size;     /* target edge (A) of the group-centre cell list; 0 = 6.5 A */
     int persistent_wgs;  /* workgroups of the batched kernel; 0 = per CU by wg_size */
     int bucket_cap;      /* mobile groups per cell before overflow; 0 = auto */
     int pair_lds;        /* 0 (default) or 1 = hold the system's LJ pair table (X x Y

@@ -20,7 +20,10 @@
 // type so that a table entry and 1/sigma serve all atoms of a type), adds
 // environment-type terms once per environment atom to LDS accumulators, and
 // writes, per pose, dE/dx [nf][3] and the per-type derivatives [3][Y] (dq, eps,
-// rmin).  FP32 arithmetic; gradients accumulate in FP32, the energy in FP64.
+// rmin).  FP32 terms, those of the derivatives inside sigma in FP64; the energy and
+// the type sums in LDS accumulate in FP64, a lane's share of an atom's sums in FP32
+// (all sums in FP32 left some eps gradients 1.3e-6 off 64 bits where four waves'
+// shorter sums had been 6e-7 off).
 #pragma once
 
 #include "engine_kernels.h"
@@ -34,19 +37,19 @@ struct AdjLds {
     float4 *tab;    // [X*Y] (100 sigma^2 hi, 4 epsilon, 100 sigma^2 lo, 0) from the per-type parameters
     float *dq;      // [Y]
     float *inv2e;   // [Y] 1 / (2 |eps|), 0 where eps = 0
-    float *gq, *ge, *gr;  // [Y] per-type derivative sums of this wave's pose
+    double *gq, *ge, *gr; // [Y] per-type derivative sums of this wave's pose
     float *red;     // [6*MAXF] per-fragment-atom sums of a shared pose
 };
 
-// the tables, then per wave the type sums and the per-atom sums
-__host__ __device__ inline int adj_wave_bytes(int Y) { return (12 * Y + 4 * 6 * MAXF + 15) & ~15; }
-__host__ __device__ inline int adj_lds_bytes(int X, int Y, int nw)
+// the tables, then per pose in hand the type sums and the per-atom sums
+__host__ __device__ inline int adj_pose_bytes(int Y) { return (24 * Y + 4 * 6 * MAXF + 15) & ~15; }
+__host__ __device__ inline int adj_lds_bytes(int X, int Y, int poses)
 {
     auto up = [](int x) { return (x + 15) & ~15; };
-    return up(16 * X * Y) + 2 * up(4 * Y) + nw * adj_wave_bytes(Y);
+    return up(16 * X * Y) + 2 * up(4 * Y) + poses * adj_pose_bytes(Y);
 }
 
-// own: the wave whose sums these are (the team's first for a shared pose)
+// own: which of the workgroup's poses these sums are for
 __device__ inline AdjLds adj_carve(char *b, int X, int Y, int own)
 {
     auto up = [](int x) { return (x + 15) & ~15; };
@@ -54,10 +57,10 @@ __device__ inline AdjLds adj_carve(char *b, int X, int Y, int own)
     A.tab = (float4 *)b; b += up(16 * X * Y);
     A.dq = (float *)b; b += up(4 * Y);
     A.inv2e = (float *)b; b += up(4 * Y);
-    b += own * adj_wave_bytes(Y);
-    A.gq = (float *)b; b += 4 * Y;
-    A.ge = (float *)b; b += 4 * Y;
-    A.gr = (float *)b; b += 4 * Y;
+    b += own * adj_pose_bytes(Y);
+    A.gq = (double *)b; b += 8 * Y;
+    A.ge = (double *)b; b += 8 * Y;
+    A.gr = (double *)b; b += 8 * Y;
     A.red = (float *)b;
     return A;
 }
@@ -136,28 +139,43 @@ struct AdjPass {
                     const float lj = pp.y * (s12 - s6);
                     const float el = (fr.w * qa) * ir;
                     acc += (double)(lj + el);
+                    // the derivatives' LJ terms; inside sigma, where s^12 carries six times
+                    // the rounding of s^2 and one pair can outweigh all others, from FP64
+                    float l = lj, h = pp.y * fmaf(2.0f, s12, -s6);   // 4 eps (s^12 - s^6), 4 eps (2 s^12 - s^6)
+                    if (s2 > 1.0f) {
+                        const double ux = (double)dx + (double)ex, uy = (double)dy + (double)ey,
+                                     uz = (double)dz + (double)ez;
+                        const double r2d = fma(uz, uz, fma(uy, uy, ux * ux));
+                        double q = __builtin_amdgcn_rcp(r2d);
+                        q = q * fma(-r2d, q, 2.0);
+                        q = q * fma(-r2d, q, 2.0);
+                        const double s2d = ((double)pp.x + (double)pp.z) * q, s6d = s2d * s2d * s2d;
+                        const double e6 = (double)pp.y * s6d;
+                        l = (float)fma(e6, s6d, -e6);
+                        h = (float)fma(2.0 * e6, s6d, -e6);
+                    }
                     // dE/d(r^2); with d = x_a - x_f, dE/dx_f = -2 dE/d(r^2) d
-                    const float dr2 = (pp.y * fmaf(-6.0f, s12, 3.0f * s6) - 0.5f * el) * ir2;
+                    const float dr2 = fmaf(-3.0f, h, -0.5f * el) * ir2;
                     const float gs = -2.0f * dr2;
                     gx[f] = fmaf(gs, dx + ex, gx[f]);
                     gy[f] = fmaf(gs, dy + ey, gy[f]);
                     gz[f] = fmaf(gs, dz + ez, gz[f]);
-                    // dE/dsigma_pair = 4 eps (12 s^12 - 6 s^6) / sigma_pair;
+                    // dE/dsigma_pair = 6 h / sigma_pair;
                     // dsigma_pair/drmin = 2^(5/6)/20 on each side
-                    const float ds = pp.y * fmaf(12.0f, s12, -6.0f * s6) * isg * (0.5f * SIGMA_PER_RMINHALF);
+                    const float ds = 6.0f * h * isg * (0.5f * SIGMA_PER_RMINHALF);
                     sr[f] += ds;
                     tr += ds;
                     // dE/deps[t] = lj / (2 |eps[t]|) on each side
-                    se[f] += lj;
-                    te += lj;
+                    se[f] += l;
+                    te += l;
                     // dE/dq: K q_a / r to the fragment side (K applied later), K q_f / r here
                     sq[f] = fmaf(qa, ir, sq[f]);
                     tq = fmaf(fr.w, ir, tq);
                 }
             }
-            atomicAdd(&A.gr[ty], tr);
-            atomicAdd(&A.ge[ty], te * A.inv2e[ty]);
-            atomicAdd(&A.gq[ty], tq);
+            atomicAdd(&A.gr[ty], (double)tr);
+            atomicAdd(&A.ge[ty], (double)(te * A.inv2e[ty]));
+            atomicAdd(&A.gq[ty], (double)tq);
         }
     }
 };
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform_i(tid >> 6), part = wave % PARTS;
     const WaveLds W = wave_lds(L, wave);
     AdjPass<NF> P;
-    P.A = adj_carve(smem + adj_off, X, Y, wave - part);
+    P.A = adj_carve(smem + adj_off, X, Y, wave / PARTS);
     CSpecies &F = species_of(C, spi);
     const int nf = F.nf;
     P.spi = spi;
@@ -248,8 +266,10 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
             const float kq = dq ? KCOUL_F * (F.tmpl[lane].w + dq[F.ttype[lane]]) : F.kq[lane];
             ((float4 *)W.fragd)[F.slot[lane]] = make_float4(px, py, pz, kq);
         }
-        if (part == 0)
-            for (int t = lane; t < 3 * Y + 6 * MAXF; t += 64) P.A.gq[t] = 0.0f;
+        if (part == 0) {
+            for (int t = lane; t < 3 * Y; t += 64) P.A.gq[t] = 0.0;
+            for (int t = lane; t < 6 * MAXF; t += 64) P.A.red[t] = 0.0f;
+        }
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             P.gx[f] = P.gy[f] = P.gz[f] = 0.0f;
@@ -293,13 +313,13 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
                 o[0] = s[0];
                 o[1] = s[1];
                 o[2] = s[2];
-                atomicAdd(&P.A.gr[tf], s[3]);
-                atomicAdd(&P.A.ge[tf], s[4] * P.A.inv2e[tf]);
-                atomicAdd(&P.A.gq[tf], s[5] * KCOUL_F);
+                atomicAdd(&P.A.gr[tf], (double)s[3]);
+                atomicAdd(&P.A.ge[tf], (double)(s[4] * P.A.inv2e[tf]));
+                atomicAdd(&P.A.gq[tf], (double)(s[5] * KCOUL_F));
             }
             wave_sync();
             float *pp = partial + (size_t)i * 3 * Y;
-            for (int t = lane; t < 3 * Y; t += 64) pp[t] = P.A.gq[t];
+            for (int t = lane; t < 3 * Y; t += 64) pp[t] = (float)P.A.gq[t];
             if (lane == 0) E[i] = ps.e[0];
         }
         wave_sync();

@@ -1886,13 +1886,13 @@ int gcmc_engine_adjoint(gcmc_engine *E, int r, int species, int npose, const flo
     l.spt = l.team + NT / 64 * TEAM_BYTES;
     l.misc = l.spt + 16 * MAXT;
     const int adj_off = (l.misc + 4 * MISC_INTS + 15) & ~15;
-    const int lds = l.total = adj_off + adj_lds_bytes(X, Y, NT / 64);
+    // one wave per pose when they fill the GPU (and the sums of four poses fit),
+    // else four; no more workgroups than run at once (each builds the pair table)
+    const bool few = npose < ADJ_WAVES || adj_off + adj_lds_bytes(X, Y, NT / 64) > 163840;
+    const int per = few ? 1 : NT / 64, wgs = std::min((npose + per - 1) / per, std::max(E->ncu, 1) * 4);
+    const int lds = l.total = adj_off + adj_lds_bytes(X, Y, per);
     if (lds > 163840) return fail(GCMC_E_ARG, "adjoint LDS layout exceeds 160 KiB (too many atom types)");
     hipStream_t s = (hipStream_t)stream;
-    // one wave per pose when they fill the GPU, else four; no more workgroups
-    // than run at once (each builds the pair table)
-    const bool few = npose < ADJ_WAVES;
-    const int per = few ? 1 : NT / 64, wgs = std::min((npose + per - 1) / per, std::max(E->ncu, 1) * 4);
 #define ADJ_LAUNCH(NFV)                                                                                            \
     hipLaunchKernelGGL((few ? k_adjoint<NT, NFV, COOP> : k_adjoint<NT, NFV, 1>), dim3(wgs), dim3(NT), lds, s, E->d_rep, \
                        r, species, npose, centres, poses, eps_kcal, rmin_half, dq, energy, dEdx, partial, l, adj_off)

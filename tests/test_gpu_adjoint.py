@@ -174,3 +174,33 @@ def test_backward_sums(case, n, per, m):
     terms = w32.double()[:, None] * y.double()
     ref, size = terms.sum(0), terms.abs().sum(0)
     assert ((gc.cpu().double() - ref).abs() <= 2.0 ** -24 * ref.abs() * 1.001 + 1e-12 * size).all()
+
+
+@pytest.mark.parametrize('few', [True, False])
+def test_type_gradients_inside_sigma(case, few):
+    """Type gradients of close contacts, where one pair outweighs the others,
+    four waves per pose and one.  The terms inside sigma are rounded to FP32
+    once (s^12 would carry six times the rounding of an FP32 s^2).  Roundings of
+    2^-24 at most: table entry and its root 2, 1/sigma 2, constants and products
+    6, a lane's and the wave's additions 16: 26 2^-24 of the largest derivative."""
+    s, eng, eps, rmin, poses = case
+    e64, r64 = eps.double().cpu().numpy(), rmin.double().cpu().numpy()
+    ref, got = [], []
+    c, p = poses[5]
+    at = s['atoms']['position'][:int(s['res'][int(s['frag'][0]['startRes']) - 1]['atomStart'])].astype(np.float64)
+    L = s['info'][0]['cryst'].astype(np.float64)
+    for i in range(4):
+        # moved so that the first atom lies 2.2 A from the nearest fixed one
+        d = p[i][0].astype(np.float64) - at
+        d -= np.rint(d / L) * L
+        j = int(np.argmin((d ** 2).sum(1)))
+        v = d[j] * (2.2 / np.linalg.norm(d[j]) - 1.0)
+        q, x = (p[i] + v).astype(np.float32)[None], (c[i] + v).astype(np.float32)[None]
+        ref.append(np.stack(O.adjoint(s, 5, x[0], q[0], e64, r64)[3:5]))
+        n = 1 if few else 2048
+        E, pt, e, r, _ = _gpu(eng, 5, np.repeat(x, n, 0), np.repeat(q, n, 0), eps, rmin)
+        ge, gr = torch.autograd.grad(E.sum() / n, (e, r))
+        got.append(np.stack([ge.cpu().numpy(), gr.cpu().numpy()]))
+    for a, b in zip(got, ref):
+        for k in range(2):
+            assert np.linalg.norm(a[k] - b[k]) <= 26 * 2.0 ** -24 * np.linalg.norm(b[k]), k
