@@ -344,7 +344,7 @@ def adjoint_bench(npose, reps=5):
     nfix = int(s['frag'][0]['startRes'])
     env = int(s['res'][nfix - 1]['atomStart'] + s['res'][nfix - 1]['atomNum'])
     return {'poses': per * T, 'ms': round(ms, 3), 'poses_per_s': round(per * T / (ms / 1e3), 1),
-            'env_atoms': env, 'dtype': 'fp32 (energies fp64 from compensated fp32)'}
+            'env_atoms': env, 'dtype': 'fp32 terms, energies and type sums added in fp64'}
 
 
 def ewald_bench(moves, warm=32):
