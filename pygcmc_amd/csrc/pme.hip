@@ -344,6 +344,17 @@ __global__ void k_pme_zero64(unsigned long long *p, size_t n)
     if (i < n) p[i] = 0ull;
 }
 
+// the influence function as a spectrum, for a plan's grid kernel
+__global__ void k_pme_spectrum(const float *G, hipfftComplex *X, size_t n)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    hipfftComplex x;
+    x.x = G[i];
+    x.y = 0.0f;
+    X[i] = x;
+}
+
 // X: K0 x K1 x (K2/2+1) half spectrum; G same layout (real).  part (when the
 // energy is wanted): each workgroup's energy sum, added up by k_pme_energy.  (One
 // FP64 atomic per workgroup on a single address: 67 us on 150 x 150 x 120 points
@@ -453,6 +464,7 @@ struct gcmc_pme {
     hipfftComplex *X = nullptr;
     hipfftHandle fwd = 0, inv = 0;
     bool have_fwd = false, have_inv = false;
+    char *work = nullptr;     // the buffers below
     double *part = nullptr;   // energy sums of k_pme_convolve's workgroups
     // many charges: per-tile counts (zero between calls) and starts, and room
     // for `room` sorted charges; more are spread in pieces of that many, so a
@@ -512,11 +524,7 @@ int gcmc_pme_destroy(gcmc_pme *p)
     if (p->Phi) (void)hipFree(p->Phi);
     if (p->G) (void)hipFree(p->G);
     if (p->X) (void)hipFree(p->X);
-    if (p->part) (void)hipFree(p->part);
-    if (p->tcount) (void)hipFree(p->tcount);
-    if (p->tstart) (void)hipFree(p->tstart);
-    if (p->where) (void)hipFree(p->where);
-    if (p->sorted) (void)hipFree(p->sorted);
+    if (p->work) (void)hipFree(p->work);
     delete p;
     return 0;
 }
@@ -548,7 +556,6 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
     if (e == hipSuccess) e = hipMalloc(&p->Phi, p->ngrid * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&p->G, p->nhalf * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&p->X, p->nhalf * sizeof(hipfftComplex));
-    if (e == hipSuccess) e = hipMalloc(&p->part, CONV_WGS * sizeof(double));
     p->tiles.n[0] = (K0 + TS0 - 1) / TS0;
     p->tiles.n[1] = (K1 + TS1 - 1) / TS1;
     p->tiles.n[2] = (K2 + TS2 - 1) / TS2;
@@ -556,11 +563,26 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
     // a quarter as many charges as grid points: more than water's density on a
     // 1 A grid (0.1 per point)
     p->room = (int)std::min<size_t>(std::max<size_t>(p->ngrid / 4, TILED_FROM), (size_t)1 << 24);
-    if (e == hipSuccess) e = hipMalloc(&p->tcount, (size_t)p->tiles.total * CPAD * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&p->tstart, (p->tiles.total + 1) * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&p->where, p->room * sizeof(int2));
-    if (e == hipSuccess) e = hipMalloc(&p->sorted, p->room * sizeof(Placed));
-    if (e == hipSuccess) e = hipMemset(p->tcount, 0, (size_t)p->tiles.total * CPAD * sizeof(int));
+    // the work buffers in one allocation
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return o;
+    };
+    const size_t count_bytes = (size_t)p->tiles.total * CPAD * sizeof(int);
+    const size_t o_part = take(CONV_WGS * sizeof(double)), o_count = take(count_bytes),
+                 o_start = take(((size_t)p->tiles.total + 1) * sizeof(int)),
+                 o_where = take((size_t)p->room * sizeof(int2)), o_sorted = take((size_t)p->room * sizeof(Placed));
+    if (e == hipSuccess) e = hipMalloc(&p->work, at);
+    if (e == hipSuccess) {
+        p->part = (double *)(p->work + o_part);
+        p->tcount = (int *)(p->work + o_count);
+        p->tstart = (int *)(p->work + o_start);
+        p->where = (int2 *)(p->work + o_where);
+        p->sorted = (Placed *)(p->work + o_sorted);
+        e = hipMemset(p->tcount, 0, count_bytes);
+    }
     if (e != hipSuccess) {
         gcmc_pme_destroy(p);
         return pme_hip(e, "PME buffers");
@@ -604,12 +626,9 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
     }
     p->have_inv = true;
     // grid kernel: the potential grid of a unit charge at grid point 0
-    std::vector<hipfftComplex> Gc(p->nhalf);
-    for (size_t i = 0; i < p->nhalf; ++i) {
-        Gc[i].x = G[i];
-        Gc[i].y = 0.0f;
-    }
-    e = hipMemcpy(p->X, Gc.data(), p->nhalf * sizeof(hipfftComplex), hipMemcpyHostToDevice);
+    hipLaunchKernelGGL(k_pme_spectrum, dim3((unsigned)((p->nhalf + 255) / 256)), dim3(256), 0, nullptr,
+                       (const float *)p->G, p->X, p->nhalf);
+    e = hipGetLastError();
     if (e != hipSuccess) {
         gcmc_pme_destroy(p);
         return pme_hip(e, "PME grid kernel");
