@@ -328,6 +328,11 @@ int gcmc_pme_spread(gcmc_pme *p, int n, const float *xyzq, void *stream);
 int gcmc_pme_solve(gcmc_pme *p, double *energy, void *stream);
 int gcmc_pme_gather(gcmc_pme *p, int n, const float *xyz, float *phi, void *stream);
 
+/* Host check of gcmc_pme_spread's rule: 1 when n charges on grid[3] points are
+ * sorted by grid tile, 0 when they are added one by one.  The charge grid is the
+ * same either way (whole-number sums). */
+int gcmc_host_pme_tiled(int n, const int *grid);
+
 /* Counter calibration (no counterpart in the reference): `copies` plain
  * device-to-device copies of `bytes` bytes (a multiple of 16), so a profiler's
  * FETCH_SIZE / WRITE_SIZE readings can be scaled to bytes moved. */

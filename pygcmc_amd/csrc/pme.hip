@@ -482,9 +482,31 @@ using namespace gcmc_pme_k;
 
 constexpr int CONV_WGS = 1024;   // workgroups of k_pme_convolve: four per CU, one energy part each
 
-// Charges from which the tiles pay: a wave per charge is one launch instead of
-// four, and 16,384 charges' atomics take 20 us, as long as the four launches.
-constexpr int TILED_FROM = 16384;
+// Charges from which the tiles pay.  A wave per charge takes 4 us + 0.93 ns per
+// charge whatever the grid; the tiles take four launches (15 us), 4 ns per tile
+// (its counter in the scan, its workgroup) and 0.2 to 0.9 ns per charge where each
+// CU has a tile.  In us, a wave per charge / tiles: 16,384 charges on 150 x 150 x 120
+// points (2,888 tiles) 19 / 29, 32,768 34 / 32, 300,000 283 / 83; 131,072 charges on
+// 256^3 (16,384 tiles) 126 / 115, 65,536 65 / 103; 300,000 on 400^3 (62,500 tiles) 289 /
+// 450, a million 964 / 546.  With fewer tiles than CUs the others idle: 65,536 charges
+// on 32^3 points (32 tiles) 65 / 336, 131,072 on 45 x 50 x 63 (168) 127 / 196, and on
+// 64^3 (256) 126 / 104.
+constexpr int TILED_FROM = 24576, TILES_FROM = 256, CHARGES_PER_TILE = 8;
+
+Tiles tiles_of(const int K[3])
+{
+    Tiles t;
+    t.n[0] = (K[0] + TS0 - 1) / TS0;
+    t.n[1] = (K[1] + TS1 - 1) / TS1;
+    t.n[2] = (K[2] + TS2 - 1) / TS2;
+    t.total = t.n[0] * t.n[1] * t.n[2];
+    return t;
+}
+
+bool tiles_pay(const Tiles &t, int n)
+{
+    return t.total >= TILES_FROM && n >= TILED_FROM && n / CHARGES_PER_TILE >= t.total;
+}
 
 // |b(m)|^2 of the order-4 spline for frequency m of K points
 double bmod2(int m, int K)
@@ -556,13 +578,11 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
     if (e == hipSuccess) e = hipMalloc(&p->Phi, p->ngrid * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&p->G, p->nhalf * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&p->X, p->nhalf * sizeof(hipfftComplex));
-    p->tiles.n[0] = (K0 + TS0 - 1) / TS0;
-    p->tiles.n[1] = (K1 + TS1 - 1) / TS1;
-    p->tiles.n[2] = (K2 + TS2 - 1) / TS2;
-    p->tiles.total = p->tiles.n[0] * p->tiles.n[1] * p->tiles.n[2];
+    p->tiles = tiles_of(grid);
     // a quarter as many charges as grid points: more than water's density on a
-    // 1 A grid (0.1 per point)
-    p->room = (int)std::min<size_t>(std::max<size_t>(p->ngrid / 4, TILED_FROM), (size_t)1 << 24);
+    // 1 A grid (0.1 per point); 10 bytes per grid point.  None for grids of few tiles
+    const bool tiled = p->tiles.total >= TILES_FROM;
+    p->room = tiled ? (int)std::min<size_t>(std::max<size_t>(p->ngrid / 4, TILED_FROM), (size_t)1 << 24) : 0;
     // the work buffers in one allocation
     size_t at = 0;
     auto take = [&](size_t bytes) {
@@ -570,9 +590,9 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
         at += (bytes + 255) & ~(size_t)255;
         return o;
     };
-    const size_t count_bytes = (size_t)p->tiles.total * CPAD * sizeof(int);
+    const size_t counted = tiled ? (size_t)p->tiles.total : 0, count_bytes = counted * CPAD * sizeof(int);
     const size_t o_part = take(CONV_WGS * sizeof(double)), o_count = take(count_bytes),
-                 o_start = take(((size_t)p->tiles.total + 1) * sizeof(int)),
+                 o_start = take((counted + 1) * sizeof(int)),
                  o_where = take((size_t)p->room * sizeof(int2)), o_sorted = take((size_t)p->room * sizeof(Placed));
     if (e == hipSuccess) e = hipMalloc(&p->work, at);
     if (e == hipSuccess) {
@@ -581,7 +601,7 @@ int gcmc_pme_create(gcmc_pme **out, const int *grid, const float *box, float bet
         p->tstart = (int *)(p->work + o_start);
         p->where = (int2 *)(p->work + o_where);
         p->sorted = (Placed *)(p->work + o_sorted);
-        e = hipMemset(p->tcount, 0, count_bytes);
+        if (tiled) e = hipMemset(p->tcount, 0, count_bytes);
     }
     if (e != hipSuccess) {
         gcmc_pme_destroy(p);
@@ -658,24 +678,28 @@ int gcmc_pme_spread(gcmc_pme *p, int n, const float *xyzq, void *stream)
     if (n == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const float4 *q = (const float4 *)xyzq;
-    if (n >= TILED_FROM) {
-        for (int o = 0; o < n;) {
-            const int m = std::min(n - o, p->room);
-            const unsigned nb = (unsigned)((m + 255) / 256);
-            hipLaunchKernelGGL(k_pme_bin, dim3(nb), dim3(256), 0, s, m, q + o, p->geo, p->tiles, p->tcount, p->where);
-            hipLaunchKernelGGL(k_pme_bin_scan, dim3(1), dim3(1024), 0, s, p->tiles.total, p->tcount, p->tstart);
-            hipLaunchKernelGGL(k_pme_bin_sort, dim3(nb), dim3(256), 0, s, m, q + o, p->geo,
-                               (const int2 *)p->where, (const int *)p->tstart, p->sorted);
-            hipLaunchKernelGGL(k_pme_spread_tiles, dim3((unsigned)p->tiles.total), dim3(256), 0, s,
-                               (const Placed *)p->sorted, (const int *)p->tstart, p->geo, p->tiles, p->Qi);
-            o += m;
-        }
-    } else {
-        hipLaunchKernelGGL(k_pme_spread, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, s, n, (const int *)nullptr, q,
-                           p->geo, p->Qi);
+    int o = 0;
+    while (o < n && tiles_pay(p->tiles, n - o)) {
+        const int m = std::min(n - o, p->room);
+        const unsigned nb = (unsigned)((m + 255) / 256);
+        hipLaunchKernelGGL(k_pme_bin, dim3(nb), dim3(256), 0, s, m, q + o, p->geo, p->tiles, p->tcount, p->where);
+        hipLaunchKernelGGL(k_pme_bin_scan, dim3(1), dim3(1024), 0, s, p->tiles.total, p->tcount, p->tstart);
+        hipLaunchKernelGGL(k_pme_bin_sort, dim3(nb), dim3(256), 0, s, m, q + o, p->geo,
+                           (const int2 *)p->where, (const int *)p->tstart, p->sorted);
+        hipLaunchKernelGGL(k_pme_spread_tiles, dim3((unsigned)p->tiles.total), dim3(256), 0, s,
+                           (const Placed *)p->sorted, (const int *)p->tstart, p->geo, p->tiles, p->Qi);
+        o += m;
     }
+    if (o < n)
+        hipLaunchKernelGGL(k_pme_spread, dim3((unsigned)(((size_t)(n - o) + 3) / 4)), dim3(256), 0, s, n - o,
+                           (const int *)nullptr, q + o, p->geo, p->Qi);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : pme_hip(e, "PME spread");
+}
+
+int gcmc_host_pme_tiled(int n, const int *grid)
+{
+    return n > 0 && grid && tiles_pay(tiles_of(grid), n) ? 1 : 0;
 }
 
 int gcmc_pme_solve(gcmc_pme *p, double *energy, void *stream)

@@ -145,3 +145,35 @@ def test_pme_spread_of_many_charges(K, n):
     assert np.array_equal(phi.view(np.uint32), phi1.view(np.uint32)) and e == e1
     ref = _spme64(a, K, np.float32(L).astype(np.float64), float(np.float32(0.34)))
     assert np.abs(phi - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize('K', [(4, 130, 260), (130, 129, 5), (9, 297, 50), (129, 145, 18), (64, 64, 64)])
+@pytest.mark.parametrize('n', [24575, 24576, 'room', 'room+5'])
+def test_pme_spread_by_tiles(K, n):
+    """At and past the line from which charges are sorted by tile, on grids of 256
+    tiles and more: axes of one tile, last tiles of one or two points, as many
+    charges as are sorted at once (a quarter of the points) and a few more.  Bit
+    for bit the grid of charges added a few at a time, and the FP64 potential:
+    2e-5 of the largest for FP32 weights, transforms and sums, 2e-7 per point of
+    the longest axis for FP32 scaled positions (two roundings of 2^-23)."""
+    room = max(K[0] * K[1] * K[2] // 4, 24576)
+    n = {'room': room, 'room+5': room + 5}.get(n, n)
+    rng = np.random.default_rng(n + K[0])
+    L = np.array([0.9 * k for k in K])
+    a = np.concatenate([(rng.random((n, 3)) * 3.0 - 1.0) * L, rng.normal(0, 0.3, (n, 1))], 1).astype(np.float32)
+    a[:, 3] -= a[:, 3].mean()
+    a[::97, 3] = 0.0
+    t = torch.tensor(a, device='cuda')
+    out = []
+    for step in (n, 5000):
+        p = PME(K, L, 0.34)
+        p.clear()
+        for i in range(0, n, step):
+            p.spread(t[i:i + step])
+        e = p.solve()
+        out.append((p.gather(t[:, :3].contiguous()).cpu().numpy(), float(e.item())))
+        p.close()
+    (phi, e), (phi1, e1) = out
+    assert np.array_equal(phi.view(np.uint32), phi1.view(np.uint32)) and e == e1
+    ref = _spme64(a, K, np.float32(L).astype(np.float64), float(np.float32(0.34)))
+    assert np.abs(phi - ref).max() <= (2e-5 + 2e-7 * max(K)) * np.abs(ref).max()

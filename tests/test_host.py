@@ -160,6 +160,20 @@ def test_pruned_stencil_covers_cutoff_pairs_at_cell_faces(cell):
     assert cov[inc].all()
 
 
+@pytest.mark.parametrize('n,grid,tiled', [
+    (24575, (150, 150, 120), 0), (24576, (150, 150, 120), 1),      # 2,888 tiles
+    (300000, (64, 64, 48), 0), (300000, (64, 64, 64), 1),          # 192 and 256 tiles
+    (16384, (32, 32, 32), 0), (1000000, (32, 32, 32), 0),
+    (131071, (256, 256, 256), 0), (131072, (256, 256, 256), 1),    # 16,384 tiles
+    (16384, (512, 512, 512), 0), (1048576, (512, 512, 512), 1),
+    (2 ** 31 - 1, (4096, 4096, 4096), 1), (0, (64, 64, 64), 0), (1, (4, 4, 4), 0)])
+def test_pme_tile_rule(n, grid, tiled):
+    """Charges are sorted by tile where there are enough of them for the grid's
+    tiles and enough tiles for the GPU: not few charges on many tiles, nor any
+    number on a few."""
+    assert engine.lib().gcmc_host_pme_tiled(n, (ctypes.c_int * 3)(*grid)) == tiled
+
+
 def _lpt(w, ncls):
     order = sorted(range(len(w)), key=lambda r: -w[r])
     load, cls = [0.0] * ncls, [0] * len(w)
