@@ -362,6 +362,11 @@ int gcmc_host_xcd_exchange(int nclass, int n, const int *best, const double *fin
 int gcmc_host_stencil_covers(int n, const float *centres, const float *groups, const float *cryst,
                              const float *startxyz, float cutoff, float cell_size,
                              unsigned char *out);
+/* The same for translations by up to grid_dx per axis, from centres[i] to
+ * moved[i]: bit 0 of out[i] when the group's cell is scanned for the old centre,
+ * bit 1 for the new one.  One scan serves both up to a grid_dx of 2 A. */
+int gcmc_host_move_covers(int n, const float *centres, const float *moved, const float *groups, const float *cryst,
+                          const float *startxyz, float cutoff, float grid_dx, float cell_size, unsigned char *out);
 
 #ifdef __cplusplus
 }

@@ -361,6 +361,9 @@ std::vector<int> make_stencil(const float L[3], const int nc[3], float rc, float
 // pose in one scan of a stencil wide enough for both centres; the wider ones
 // scan twice (the union of two distant neighbourhoods would be scanned for each).
 constexpr float WIDE_DX = 2.0f;
+// The stencil reaches further towards positive offsets only: negative steps scan
+// twice.
+bool one_scan(float dx) { return dx >= 0.0f && dx <= WIDE_DX; }
 
 template <class T>
 hipError_t put(T **dst, DevBuf &b, const T *src, size_t n)
@@ -621,7 +624,7 @@ int upload_rep(gcmc_engine *E, HostRep &H)
     // not wrap onto itself) the box distance is measured from the centre's
     // position in its cell; other axes count no distance.
     stencil_prune(R.L, R.nc, R.rc, 0.0f, R.cell_h, &R.prune, &R.prune_r2);
-    if (R.dx <= WIDE_DX) {
+    if (one_scan(R.dx)) {
         const std::vector<int> wide = make_stencil(R.L, R.nc, R.rc, R.dx);
         R.nst_wide = (int)wide.size();
         st.insert(st.end(), wide.begin(), wide.end());
@@ -2039,42 +2042,72 @@ int gcmc_host_within(int n, const float *a, const float *b, const float *cryst, 
     return 0;
 }
 
+}  // extern "C"
+
+namespace {
+// whether the group's cell is scanned: a stencil cell around the home cell of
+// c0 that is near c0, or (c1 not null) near the centre c1
+bool cell_scanned(const std::vector<int> &sten, const float L[3], const float st[3], const float inv_h[3], const int nc[3],
+                  const float h[3], int prune, float r2, const float *c0, const float *c1, const float *group)
+{
+    int ci[3];
+    cell_coords(L, st, inv_h, nc, c0[0], c0[1], c0[2], ci);
+    const int cg = cell_index(L, st, inv_h, nc, group[0], group[1], group[2]);
+    float u[3], base0[3], base1[3], hp[3];
+    cell_offset(L, st, h, ci, c0[0], c0[1], c0[2], u);
+    stencil_base(u, h, prune, base0, hp);
+    if (c1)
+        for (int i = 0; i < 3; ++i) base1[i] = hp[i] == 0.0f ? 0.0f : moved_base(base0[i], c1[i] - c0[i], L[i], 1.0f / L[i]);
+    for (int code : sten) {
+        // the kernel skips other cells
+        if (!stencil_cell_near(code, base0, hp, r2) && !(c1 && stencil_cell_near(code, base1, hp, r2))) continue;
+        int i[3];
+        for (int a = 0; a < 3; ++a) {
+            const int q = ci[a] + (code >> (8 * a) & 255) - 128;
+            i[a] = ((q % nc[a]) + nc[a]) % nc[a];
+        }
+        if ((i[0] * nc[1] + i[1]) * nc[2] + i[2] == cg) return true;
+    }
+    return false;
+}
+}  // namespace
+
+extern "C" {
+
 int gcmc_host_stencil_covers(int n, const float *centres, const float *groups, const float *cryst,
                              const float *startxyz, float cutoff, float cell_size, unsigned char *out)
 {
     if (n < 0 || (n > 0 && (!centres || !groups || !out)) || !cryst || !startxyz)
         return fail(GCMC_E_ARG, "bad arguments");
-    int nc[3];
-    float inv_h[3], L[3], st[3];
-    for (int i = 0; i < 3; ++i) {
-        L[i] = cryst[i];
-        st[i] = startxyz[i];
-    }
-    cell_geometry(L, cell_size, nc, inv_h);
-    const std::vector<int> sten = make_stencil(L, nc, cutoff, 0.0f);
-    float h[3], r2;
-    int prune;
-    stencil_prune(L, nc, cutoff, 0.0f, h, &prune, &r2);
+    int nc[3], prune;
+    float inv_h[3], h[3], r2;
+    cell_geometry(cryst, cell_size, nc, inv_h);
+    const std::vector<int> sten = make_stencil(cryst, nc, cutoff, 0.0f);
+    stencil_prune(cryst, nc, cutoff, 0.0f, h, &prune, &r2);
+    for (int q = 0; q < n; ++q)
+        out[q] = cell_scanned(sten, cryst, startxyz, inv_h, nc, h, prune, r2, centres + 3 * q, nullptr, groups + 3 * q);
+    return 0;
+}
+
+int gcmc_host_move_covers(int n, const float *centres, const float *moved, const float *groups, const float *cryst,
+                          const float *startxyz, float cutoff, float grid_dx, float cell_size, unsigned char *out)
+{
+    if (n < 0 || (n > 0 && (!centres || !moved || !groups || !out)) || !cryst || !startxyz)
+        return fail(GCMC_E_ARG, "bad arguments");
+    int nc[3], prune;
+    float inv_h[3], h[3], r2;
+    cell_geometry(cryst, cell_size, nc, inv_h);
+    const bool one = one_scan(grid_dx);
+    const float ext = one ? grid_dx : 0.0f;
+    const std::vector<int> sten = make_stencil(cryst, nc, cutoff, ext);
+    stencil_prune(cryst, nc, cutoff, ext, h, &prune, &r2);
     for (int q = 0; q < n; ++q) {
-        const int cc = cell_index(L, st, inv_h, nc, centres[3 * q], centres[3 * q + 1], centres[3 * q + 2]);
-        const int cg = cell_index(L, st, inv_h, nc, groups[3 * q], groups[3 * q + 1], groups[3 * q + 2]);
-        const int c0 = cc / (nc[1] * nc[2]), c1 = (cc / nc[2]) % nc[1], c2 = cc % nc[2];
-        const int ci[3] = {c0, c1, c2};
-        float u[3];
-        cell_offset(L, st, h, ci, centres[3 * q], centres[3 * q + 1], centres[3 * q + 2], u);
-        float base[3], hp[3];
-        stencil_base(u, h, prune, base, hp);
-        out[q] = 0;
-        for (int code : sten) {
-            if (!stencil_cell_near(code, base, hp, r2)) continue;     // the kernel skips this cell
-            int i0 = c0 + (code & 255) - 128, i1 = c1 + ((code >> 8) & 255) - 128, i2 = c2 + ((code >> 16) & 255) - 128;
-            i0 = ((i0 % nc[0]) + nc[0]) % nc[0];
-            i1 = ((i1 % nc[1]) + nc[1]) % nc[1];
-            i2 = ((i2 % nc[2]) + nc[2]) % nc[2];
-            if ((i0 * nc[1] + i1) * nc[2] + i2 == cg) {
-                out[q] = 1;
-                break;
-            }
+        const float *c0 = centres + 3 * q, *c1 = moved + 3 * q, *g = groups + 3 * q;
+        if (one) {
+            out[q] = cell_scanned(sten, cryst, startxyz, inv_h, nc, h, prune, r2, c0, c1, g) ? 3 : 0;
+        } else {
+            out[q] = (cell_scanned(sten, cryst, startxyz, inv_h, nc, h, prune, r2, c0, nullptr, g) ? 1 : 0) |
+                     (cell_scanned(sten, cryst, startxyz, inv_h, nc, h, prune, r2, c1, nullptr, g) ? 2 : 0);
         }
     }
     return 0;

@@ -641,7 +641,7 @@ __device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLd
         for (int i = 0; i < 3; ++i) {
             const float d = c1[i] - c0[i];
             base0[i] = uniform_f(base0[i]);
-            base1[i] = hp[i] == 0.0f ? 0.0f : uniform_f(base0[i] + (d - rintf(d * C.invL[i]) * C.L[i]));
+            base1[i] = hp[i] == 0.0f ? 0.0f : uniform_f(moved_base(base0[i], d, C.L[i], C.invL[i]));
             home[i] = uniform_i(home[i]) - 128;
         }
     }

@@ -236,6 +236,12 @@ __host__ __device__ inline void stencil_base(const float u[3], const float h[3],
         base[i] = p ? u[i] + 128.0f * h[i] : 0.0f;
     }
 }
+// base of a second centre (along a pruned axis), d away from the first: by d's
+// nearest image
+__host__ __device__ inline float moved_base(float base0, float d, float L, float invL)
+{
+    return base0 + (d - rintf(d * invL) * L);
+}
 __host__ __device__ inline bool stencil_cell_near(int code, const float base[3], const float hp[3], float r2)
 {
     float g2 = 0.0f;

@@ -93,6 +93,7 @@ def lib():
         L.gcmc_engine_eval_poses.argtypes = [P, I, I, I, P, P, P, P, P, P]
         L.gcmc_host_within.argtypes = [I, P, P, P, ctypes.c_float, P]
         L.gcmc_host_stencil_covers.argtypes = [I, P, P, P, P, ctypes.c_float, ctypes.c_float, P]
+        L.gcmc_host_move_covers.argtypes = [I, P, P, P, P, P, ctypes.c_float, ctypes.c_float, ctypes.c_float, P]
         L.gcmc_host_xcd_exchange.argtypes = [I, I, P, P, P, P, P]
         L.runGCMC_hip.argtypes = [P, P, P, P, P, P, P]
         _lib = L
@@ -136,6 +137,18 @@ def host_stencil_covers(centres, groups, cryst, startxyz, cutoff, cell_size=0.0)
     _check(lib().gcmc_host_stencil_covers(len(a), _p(a), _p(b), _p(c), _p(st), float(cutoff),
                                           float(cell_size), _p(out)))
     return out.astype(bool)
+
+
+def host_move_covers(centres, moved, groups, cryst, startxyz, cutoff, grid_dx, cell_size=0.0):
+    """Whether each group's cell is scanned for the old and for the new centre
+    of the paired translation (host check): two boolean arrays."""
+    a, b, g = (np.ascontiguousarray(x, np.float32).reshape(-1, 3) for x in (centres, moved, groups))
+    c = np.ascontiguousarray(cryst, np.float32)
+    st = np.ascontiguousarray(startxyz, np.float32)
+    out = np.zeros(len(a), np.uint8)
+    _check(lib().gcmc_host_move_covers(len(a), _p(a), _p(b), _p(g), _p(c), _p(st), float(cutoff), float(grid_dx),
+                                       float(cell_size), _p(out)))
+    return (out & 1).astype(bool), (out & 2).astype(bool)
 
 
 def host_xcd_exchange(best, fin, evt):

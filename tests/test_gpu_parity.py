@@ -154,6 +154,19 @@ def test_lockstep_multi_fragment(wg_size):
     print(f'multi batched: max |dE| {err:.3e}, {ng} groups, {mism} mismatches, N={g["frag"]["totalNum"]}')
 
 
+@pytest.mark.parametrize('dx', [-1.5, 2.0, 3.0])
+def test_lockstep_translation_steps(dx):
+    """Translations whose two centres are served by one scan (up to 2 A), and by
+    two (wider or negative steps)."""
+    s = systems.multi(nsteps=600)
+    s['info']['grid_dx'] = dx
+    gt, ot, g, r, st = _lockstep(s, 600, 'batched')
+    err, ng, mism = _compare(gt, ot, g, r)
+    trn = st['attempts'][:, 2].sum()
+    print(f'grid_dx {dx}: max |dE| {err:.3e}, {ng} groups, {mism} mismatches, {trn} translations')
+    assert trn > 50 and (gt['k'][s['moves'][:600] % 4 == 2] > 0).sum() > 20
+
+
 @pytest.mark.parametrize('wg_size', [256, 1024])
 def test_plain_batched_graph_identical(wg_size):
     s = systems.multi(nsteps=300, seed=11)

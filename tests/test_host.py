@@ -160,6 +160,41 @@ def test_pruned_stencil_covers_cutoff_pairs_at_cell_faces(cell):
     assert cov[inc].all()
 
 
+@pytest.mark.parametrize('dx', [-2.5, -1.0, 0.0, 1.0, 2.0, 3.0])
+@pytest.mark.parametrize('L,cell', [((54.31, 80.0, 124.07), 5.0), ((54.31, 80.0, 124.07), 6.5),
+                                    ((30.0, 33.0, 47.0), 6.5), ((36.0, 41.0, 90.0), 2.5)])
+def test_translation_scan_covers_both_centres(L, cell, dx):
+    """A translation's old centre on and next to cell and box faces, the new one
+    up to grid_dx further (either sign) and through the box: the cells scanned
+    hold every group within the cutoff of either centre, in boxes whose axes
+    the scan wraps around too."""
+    rng = np.random.default_rng(37)
+    L = np.array(L)
+    start = np.array([-1.25, 0.5, 3.0])
+    rc = 15.0 if L.min() > 50 else 12.0
+    nc = np.maximum(1, np.floor(L / cell)).astype(int)
+    fr = np.array([0.0, 1e-5, 0.25, 0.5, 1.0 - 1e-5])
+    c = rng.integers(0, nc, (1500, 3))
+    c[:300] = np.where(rng.random((300, 3)) < 0.5, 0, nc - 1)    # cells at the box's faces
+    a = (start + (c + rng.choice(fr, c.shape)) * (L / nc)).astype(np.float32)
+    L32, s32 = L.astype(np.float32), start.astype(np.float32)
+    d = rng.choice(np.float32([0.0, 0.5, 1.0 - 2.0 ** -24]), a.shape) * np.float32(dx)
+    d = np.where(a + d > L32 + s32, d - L32, d)
+    d = np.where(a + d < s32, d + L32, d).astype(np.float32)
+    b = a + d
+    dirs = rng.normal(size=(12, 3))
+    dirs = np.concatenate([dirs, np.eye(3), -np.eye(3)])
+    dirs /= np.linalg.norm(dirs, axis=1)[:, None]
+    for frm in (a, b):
+        for v in dirs:
+            g = (frm + v * rc * (1.0 - 1e-6)).astype(np.float32)
+            old, new = engine.host_move_covers(a, b, g, L, start, rc, dx, cell)
+            assert old[engine.host_within(a, g, L, rc)].all()
+            assert new[engine.host_within(b, g, L, rc)].all()
+    far = (a + rng.random(a.shape) * L).astype(np.float32)
+    assert not all(x.all() for x in engine.host_move_covers(a, b, far, L, start, rc, dx, cell)) or L.min() < 50
+
+
 @pytest.mark.parametrize('n,grid,tiled', [
     (24575, (150, 150, 120), 0), (24576, (150, 150, 120), 1),      # 2,888 tiles
     (300000, (64, 64, 48), 0), (300000, (64, 64, 64), 1),          # 192 and 256 tiles
