@@ -23,7 +23,9 @@
 // rmin).  FP32 terms, those of the derivatives inside sigma in FP64; the energy and
 // the type sums in LDS accumulate in FP64, a lane's share of an atom's sums in FP32
 // (all sums in FP32 left some eps gradients 1.3e-6 off 64 bits where four waves'
-// shorter sums had been 6e-7 off).
+// shorter sums had been 6e-7 off), the charge derivatives' from batch to batch in
+// FP64 (2,100 poses of nine species, five systems each: 1.30e-7 off 64 bits in the
+// geometric mean, 1.51e-7 with one FP32 sum per lane and pose; no time).
 #pragma once
 
 #include "engine_kernels.h"
@@ -38,11 +40,11 @@ struct AdjLds {
     float *dq;      // [Y]
     float *inv2e;   // [Y] 1 / (2 |eps|), 0 where eps = 0
     double *gq, *ge, *gr; // [Y] per-type derivative sums of this wave's pose
-    float *red;     // [6*MAXF] per-fragment-atom sums of a shared pose
+    float *red;     // [5*MAXF] per-fragment-atom sums of a shared pose
 };
 
 // the tables, then per pose in hand the type sums and the per-atom sums
-__host__ __device__ inline int adj_pose_bytes(int Y) { return (24 * Y + 4 * 6 * MAXF + 15) & ~15; }
+__host__ __device__ inline int adj_pose_bytes(int Y) { return (24 * Y + 4 * 5 * MAXF + 15) & ~15; }
 __host__ __device__ inline int adj_lds_bytes(int X, int Y, int poses)
 {
     auto up = [](int x) { return (x + 15) & ~15; };
@@ -71,6 +73,7 @@ struct AdjPass {
     int spi, nf;
     double acc;
     float gx[NF], gy[NF], gz[NF], sr[NF], se[NF], sq[NF];   // in the order of Species::slot
+    double qsum;                                            // lane f: the batches' sums of sq[f]
 
     __device__ __forceinline__ void run(CRep &C, const Lds &L, const WaveLds &W, int g, int At)
     {
@@ -177,6 +180,16 @@ struct AdjPass {
             atomicAdd(&A.ge[ty], (double)(te * A.inv2e[ty]));
             atomicAdd(&A.gq[ty], (double)tq);
         }
+        // sq's sums cancel most (charges of both signs), so they go on in FP64 from here:
+        // 16 terms of a lane at most are added in FP32
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            if (f < nf) {
+                const double x = lane_d(wave_scan_add((double)sq[f]), 63);
+                qsum += lane == f ? x : 0.0;
+                sq[f] = 0.0f;
+            }
+        }
     }
 };
 
@@ -268,26 +281,26 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         }
         if (part == 0) {
             for (int t = lane; t < 3 * Y; t += 64) P.A.gq[t] = 0.0;
-            for (int t = lane; t < 6 * MAXF; t += 64) P.A.red[t] = 0.0f;
+            for (int t = lane; t < 5 * MAXF; t += 64) P.A.red[t] = 0.0f;
         }
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             P.gx[f] = P.gy[f] = P.gz[f] = 0.0f;
             P.sr[f] = P.se[f] = P.sq[f] = 0.0f;
         }
-        P.acc = 0.0;
+        P.acc = P.qsum = 0.0;
         if (PARTS > 1) __syncthreads();
         wave_sync();
         ScanSums o{};
         scan_groups(C, L, W, c, c, 1, -1, part, PARTS, P, o);
         // lane f of the first wave: the sums of the atom in place f
-        float s[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             if (f < nf) {
-                const float v[6] = {P.gx[f], P.gy[f], P.gz[f], P.sr[f], P.se[f], P.sq[f]};
+                const float v[5] = {P.gx[f], P.gy[f], P.gz[f], P.sr[f], P.se[f]};
 #pragma unroll
-                for (int k = 0; k < 6; ++k) {
+                for (int k = 0; k < 5; ++k) {
                     const float x = wave_sum_f(v[k]);
                     if (lane == f) s[k] = x;
                 }
@@ -295,27 +308,29 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         }
         PoseSums ps{};
         ps.e[0] = lane_d(wave_scan_add(P.acc), 63);
+        // the place's atom (Species::slot is the other way round)
+        int a = 0, tf = 0;
+        if (lane < nf) {
+            for (int b = 0; b < nf; ++b) a = F.slot[b] == lane ? b : a;
+            tf = F.ttype[a];
+            atomicAdd(&P.A.gq[tf], P.qsum * (double)KCOUL_F);
+        }
         if (PARTS > 1) {
             if (lane < nf)
-                for (int k = 0; k < 6; ++k) atomicAdd(&P.A.red[6 * lane + k], s[k]);
+                for (int k = 0; k < 5; ++k) atomicAdd(&P.A.red[5 * lane + k], s[k]);
             team_sum<NT>(L, ps);
             if (lane < nf)
-                for (int k = 0; k < 6; ++k) s[k] = P.A.red[6 * lane + k];
+                for (int k = 0; k < 5; ++k) s[k] = P.A.red[5 * lane + k];
         }
         wave_sync();
         if (part == 0 && i < p1) {
-            // the place's atom (Species::slot is the other way round)
             if (lane < nf) {
-                int a = 0;
-                for (int b = 0; b < nf; ++b) a = F.slot[b] == lane ? b : a;
-                const int tf = F.ttype[a];
                 float *o = dEdx + ((size_t)i * nf + a) * 3;
                 o[0] = s[0];
                 o[1] = s[1];
                 o[2] = s[2];
                 atomicAdd(&P.A.gr[tf], (double)s[3]);
                 atomicAdd(&P.A.ge[tf], (double)(s[4] * P.A.inv2e[tf]));
-                atomicAdd(&P.A.gq[tf], (double)(s[5] * KCOUL_F));
             }
             wave_sync();
             float *pp = partial + (size_t)i * 3 * Y;
