@@ -167,8 +167,10 @@ int gcmc_engine_counters(gcmc_engine *e, int replica, unsigned long long *out5);
  * evaluations (summed over workgroups), [1] in accept phases, [2] in prep
  * phases, [3] from publishing a move to its last evaluation finishing. */
 int gcmc_engine_phase_ticks(gcmc_engine *e, int replica, unsigned long long *out4);
-/* Ticks inside evaluations (summed): [0] pose and adjacency, [1] stencil
- * counts and scan, [2] candidate group tests, [3] pair passes. */
+/* Ticks inside evaluations, summed over the waves that evaluate (one per trial,
+ * four where a move has at most 100 trials): [0] pose and adjacency, [1] stencil
+ * cells and their counts, [2] candidate group tests, [3] pair passes.  One trial
+ * in eight is timed and counts eight times. */
 int gcmc_engine_sub_ticks(gcmc_engine *e, int replica, unsigned long long *out4);
 
 /* ---- step trace (parity tests) --------------------------------------------

@@ -292,7 +292,8 @@ __global__ __launch_bounds__(NT) void k_adjoint(const Rep *reps, int r, int spi,
         if (PARTS > 1) __syncthreads();
         wave_sync();
         ScanSums o{};
-        scan_groups(C, L, W, c, c, 1, -1, part, PARTS, P, o);
+        NoTicks nt;
+        scan_groups(C, L, W, c, c, 1, -1, part, PARTS, P, o, nt);
         // lane f of the first wave: the sums of the atom in place f
         float s[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll

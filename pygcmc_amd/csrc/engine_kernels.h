@@ -86,6 +86,7 @@ __device__ __forceinline__ CSpecies &species_of(CRep &C, int s) { return ((CSpec
 
 // scratch ints of a workgroup (Lds::misc)
 enum Misc : int {
+    M_TICKS = 74,    // [74, 78)  time of the claimed trials by phase, summed over the waves
     M_GN = 78,       // groups in the batch (select_groups)
     M_NEXT = 79,     // next of the claimed trials (eval_items)
     M_ACC = 80,      // accept: decision / count of accepted
@@ -622,10 +623,39 @@ struct ScanSums {
     uint32_t hash[2];
 };
 
-template <class Pass>
+// Time of a trial by phase (device ticks), added up in LDS for the workgroup:
+// poses and adjacency, cells and their records, group tests, pair passes.  A read
+// of the clock holds a wave up for some 100 ns, about seven times in a share of a
+// trial, so one trial in TICKED is timed, picked by a hash of step and trial, and
+// counts TICKED times: 400 one-trial moves take 5.40 ms, as without (5.39), 5.58
+// with every trial timed.
+enum Phase : int { S_POSE, S_LIST, S_TEST, S_PAIRS };
+constexpr int TICKED_BITS = 3, TICKED = 1 << TICKED_BITS;
+struct Ticks {
+    int *sum;         // the workgroup's
+    unsigned mark;    // when the present phase began
+    bool on;
+    __device__ __forceinline__ Ticks(int *s, int step, int t) : sum(s), mark(0u)
+    {
+        on = ((unsigned)step * 0x9E3779B1u + (unsigned)t * 0x85EBCA77u) >> (32 - TICKED_BITS) == 0u;
+        if (on) mark = (unsigned)wall_clock64();
+    }
+    __device__ __forceinline__ void end(Phase p)
+    {
+        if (!on) return;
+        const unsigned now = (unsigned)wall_clock64();
+        if (fresh_lane() == 0) atomicAdd(&sum[p], (int)(now - mark));
+        mark = now;
+    }
+};
+struct NoTicks {
+    __device__ __forceinline__ void end(Phase) {}
+};
+
+template <class Pass, class TK>
 __device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLds &W, const float c0[3],
                                             const float c1[3], int ncentre, int exclude, int part, int parts,
-                                            Pass &P, ScanSums &o)
+                                            Pass &P, ScanSums &o, TK &tk)
 {
     CRep &C = fresh(C0);
     const int lane = fresh_lane();
@@ -655,6 +685,8 @@ __device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLd
     while (true) {
         // ---- the next 128 candidates
         bool done = false;
+        const bool list = r0 >= T;
+        if (list && b > 0) tk.end(S_TEST);   // (the first list begins the scan)
         while (r0 >= T) {
             if (q0 >= nl) {
                 if (b >= ne) {
@@ -728,6 +760,7 @@ __device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLd
             r0 = 0;
             carry = 0;
         }
+        if (list) tk.end(S_LIST);
         constexpr int R = 2;
         int2 rr[R];
         int flag[R], pos[R], at[R], ng = 0, tot = 0;
@@ -799,7 +832,9 @@ __device__ __forceinline__ void scan_groups(CRep &C0, const Lds &L, const WaveLd
         if (done || g + ng > WL_GROUPS || A + tot > WL_ATOMS) {
             if (g > 0) {
                 wave_sync();
+                tk.end(S_TEST);
                 P.run(C, L, W, g, A);
+                tk.end(S_PAIRS);
                 wave_sync();
             }
             if (done) break;
@@ -851,10 +886,10 @@ __device__ __forceinline__ void order_pose(CRep &C, CSpecies &F, const WaveLds &
 // pose_near: the poses were generated from the species template or the
 // molecule's atoms (within the species' extent of the centre, the bound
 // Rep::nowrap rests on); poses given by a caller take the per-pair image shift.
-template <bool STAGED, int TM>
+template <bool STAGED, int TM, class TK>
 __device__ __forceinline__ void eval_poses_wave(CRep &C, const Lds &L, const WaveLds &W, int spi, int nf, int nset,
                                                 const float c0[3], const float c1[3], bool same_centre, int exclude,
-                                                bool pose_near, int part, int parts, PoseSums &out)
+                                                bool pose_near, int part, int parts, PoseSums &out, TK &tk)
 {
     EnergyPass<STAGED, TM> P;
     for (int i = 0; i < 2; ++i) P.acc[i] = 0.0;
@@ -871,7 +906,7 @@ __device__ __forceinline__ void eval_poses_wave(CRep &C, const Lds &L, const Wav
     for (int pass = 0; pass < (both ? 1 : 2); ++pass) {
         ScanSums q{};
         P.first = pass;
-        scan_groups(C, L, W, pass ? c1 : c0, c1, nset == 2 && both && !same_centre ? 2 : 1, exclude, part, parts, P, q);
+        scan_groups(C, L, W, pass ? c1 : c0, c1, nset == 2 && both && !same_centre ? 2 : 1, exclude, part, parts, P, q, tk);
         if (pass == 0) o = q;
         else {
             o.nin[1] = q.nin[0];
@@ -923,15 +958,12 @@ __device__ inline void count_add(T *p, T v)
 // statistics of a wave's evaluations (counters of the replica's State), added
 // up in registers and published once per claim
 struct ItemStats {
-    unsigned ticks[2];   // poses and adjacency, scan and pair passes
     unsigned nat, nin, neval, nfat;
 };
 
 template <bool LOCAL>
 __device__ inline void add_item_stats(State &W, const ItemStats &s, int nf)
 {
-    count_add<LOCAL>(&W.t_sub[0], (unsigned long long)s.ticks[0]);
-    count_add<LOCAL>(&W.t_sub[3], (unsigned long long)s.ticks[1]);
     count_add<LOCAL>(&W.n_eval, (unsigned long long)s.neval);
     count_add<LOCAL>(&W.n_pair, (unsigned long long)s.nat * nf);
     count_add<LOCAL>(&W.n_atom, (unsigned long long)s.nat);
@@ -1010,11 +1042,11 @@ __device__ __forceinline__ Move move_of(const State &S) { return make_move(S.kin
 // the energies.
 template <bool STAGED, int TM>
 __device__ __forceinline__ void trial_wave(CRep &C0, const Move &mv, int t, int part, int parts, const Lds &L,
-                                           const WaveLds &W, PoseSums &out, ItemStats &st)
+                                           const WaveLds &W, PoseSums &out)
 {
     CRep &C = fresh(C0);
     const int lane = fresh_lane();
-    const unsigned long long tq0 = wall_clock64();
+    Ticks tk(L.misc + M_TICKS, mv.step, t);
     const int kind = mv.kind, k = mv.k, step = mv.step;
     CSpecies &F = species_of(C, mv.spi);
     const int nf = F.nf;
@@ -1107,18 +1139,15 @@ __device__ __forceinline__ void trial_wave(CRep &C0, const Move &mv, int t, int 
             }
         }
     }
-    const unsigned long long tq1 = wall_clock64();
+    tk.end(S_POSE);
     // a rotation keeps the centre
-    eval_poses_wave<STAGED, TM>(C, L, W, mv.spi, nf, mv.nset, co, cn, kind != K_TRN, gid, true, part, parts, out);
+    eval_poses_wave<STAGED, TM>(C, L, W, mv.spi, nf, mv.nset, co, cn, kind != K_TRN, gid, true, part, parts, out, tk);
     if (TM == T_EWALD) {
         // the moving molecule (delete, translate, rotate) is in the PME grid
         const int base = kind == K_INS ? -1 : F.atomBase + slot * nf;
         out.e[0] += ewald_recip(C, F, W, 0, nf, base, part, parts);
         if (mv.nset == 2) out.e[1] += ewald_recip(C, F, W, 1, nf, base, part, parts);
     }
-    const unsigned long long tq2 = wall_clock64();
-    st.ticks[0] += (unsigned)(tq1 - tq0);
-    st.ticks[1] += (unsigned)(tq2 - tq1);
 }
 
 // energies of a trial to the replica's buffers, statistics, trace (one lane)
@@ -1200,7 +1229,7 @@ __device__ __forceinline__ void eval_items(CRep &C, const Move &mv, int item, in
         }
         const int t = item + min(j, cnt - 1), part = mv.coop ? wave % COOP : 0, parts = mv.coop ? COOP : 1;
         PoseSums r;
-        trial_wave<STAGED, TM>(C, mv, t, part, parts, L, W, r, st);
+        trial_wave<STAGED, TM>(C, mv, t, part, parts, L, W, r);
         if (mv.coop) team_sum<NT>(L, r);
         if (lane == 0 && part == 0 && j < cnt) finish_trial(C, mv, t, W, r, st);
         wave_sync();
@@ -2053,10 +2082,16 @@ __global__ __launch_bounds__(NT) void k_eval_plain(const Rep *reps, State *st, i
     const Lds L = carve(smem, lay);
     CRep &C = rep_of(reps, r);
     if (threadIdx.x == 0) L.misc[M_NEXT] = 0;
+    if (threadIdx.x < 4) L.misc[M_TICKS + threadIdx.x] = 0;
     stage_tables<NT, STAGED>(C, L, true, true);
     ItemStats ist{};
     eval_items<NT, STAGED, TM>(C, mv, item, min(per, mv.nitems - item), L, ist);
     if ((threadIdx.x & 63) == 0 && ist.neval) add_item_stats<false>(S, ist, species_of(C, mv.spi).nf);
+    __syncthreads();
+    if (threadIdx.x < 4) {
+        const int t = L.misc[M_TICKS + threadIdx.x];
+        if (t != 0) count_add<false>(&S.t_sub[threadIdx.x], (unsigned long long)t * TICKED);
+    }
 }
 
 template <int NT, bool STAGED, bool EW>
@@ -2133,6 +2168,7 @@ __global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, i
     // the trials this workgroup kept of a move it published (advance_and_publish)
     int kept = 0, kept_rep = -1;
     Move mv;
+    if (tid < 4) L.misc[M_TICKS + tid] = 0;   // (a claim's barriers come before the first use)
     while (true) {
         int found, item, cnt;
         if (kept > 0) {
@@ -2329,6 +2365,16 @@ __global__ __launch_bounds__(NT, 3) void k_batched(const Rep *reps, State *st, i
             }
             __builtin_amdgcn_s_setprio(0);
         }
+        // the phases of this replica's trials, complete since the barrier after them:
+        // when the workgroup leaves the replica (a kept move follows at once), and now
+        // and then
+        if ((kept == 0 || (mv.step & 255) == 0) && tid < 4) {
+            const int t = L.misc[M_TICKS + tid];
+            if (t != 0) {
+                count_add<true>(&S.t_sub[tid], (unsigned long long)t * TICKED);
+                L.misc[M_TICKS + tid] = 0;
+            }
+        }
         __syncthreads();
     }
 }
@@ -2410,7 +2456,8 @@ __global__ __launch_bounds__(NT) void k_eval_poses(const Rep *reps, int r, int s
         if (lane < nf) order_pose<TM>(C, F, W, 0, lane, make_float4(px, py, pz, F.kq[lane]), c);
         wave_sync();
         PoseSums s;
-        eval_poses_wave<STAGED, TM>(C, L, W, spi, nf, 1, c, c, true, x, false, part, PARTS, s);
+        NoTicks nt;
+        eval_poses_wave<STAGED, TM>(C, L, W, spi, nf, 1, c, c, true, x, false, part, PARTS, s, nt);
         if (TM == T_EWALD) {
             const bool own = x >= F.startRes && x < F.startRes + F.maxNum;
             s.e[0] += ewald_recip(C, F, W, 0, nf, own ? F.atomBase + (x - F.startRes) * nf : -1, part, PARTS);

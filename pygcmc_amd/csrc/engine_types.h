@@ -153,8 +153,8 @@ struct State {
     // 100 MHz time by which every write the current move's evaluations read
     // (prep, the previous move's commit) had reached L2; set when it is published
     unsigned long long t_data;
-    // sub-phases of evaluations (ticks, summed): pose+adjacency, stencil
-    // count+scan, candidate tests, pair passes
+    // sub-phases of evaluations (ticks, summed over waves): pose+adjacency, stencil
+    // cells and their counts, candidate tests, pair passes
     unsigned long long t_sub[4];
 };
 

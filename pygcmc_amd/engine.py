@@ -267,7 +267,9 @@ class Engine:
         return dict(zip(('eval', 'accept', 'prep', 'step'), (float(x) * 1e-8 for x in out)))
 
     def eval_sub_seconds(self, r=0):
-        """Time inside evaluations by sub-phase, seconds (summed over evaluations)."""
+        """Time inside evaluations by sub-phase, seconds, summed over the waves that
+        evaluate (one per trial, four where a move has at most 100 trials); one
+        trial in eight is timed and counts eight times."""
         out = np.zeros(4, np.uint64)
         _check(lib().gcmc_engine_sub_ticks(self._h, r, _p(out)))
         return dict(zip(('pose', 'stencil', 'candidates', 'pairs'), (float(x) * 1e-8 for x in out)))

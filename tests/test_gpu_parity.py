@@ -167,6 +167,25 @@ def test_lockstep_translation_steps(dx):
     assert trn > 50 and (gt['k'][s['moves'][:600] % 4 == 2] > 0).sum() > 20
 
 
+@pytest.mark.parametrize('mode', ['plain', 'batched', 'graph'])
+def test_evaluation_time_by_phase(mode):
+    """Every phase of the evaluations has its time, whether four waves share a
+    trial or one has it (fewer and more than 100 trials per move)."""
+    for conf in (4, 130):
+        s = systems.water(nsteps=300, conf=conf)
+        eng = Engine()
+        eng.add_system(s)
+        eng.upload()
+        assert not any(eng.eval_sub_seconds(0).values())
+        ms = eng.run(300, mode)
+        t = eng.eval_sub_seconds(0)
+        n = eng.counters(0)['evals']
+        print(mode, conf, n, {k: f'{1e9 * v / n:.0f} ns per evaluation' for k, v in t.items()})
+        assert all(v > 0.0 for v in t.values())
+        assert sum(t.values()) < 1e-3 * ms * 256 * 12   # all waves that fit on the GPU, all the time
+        eng.close()
+
+
 @pytest.mark.parametrize('wg_size', [256, 1024])
 def test_plain_batched_graph_identical(wg_size):
     s = systems.multi(nsteps=300, seed=11)
