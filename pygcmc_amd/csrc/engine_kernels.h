@@ -1512,6 +1512,7 @@ __device__ inline void select_groups(CRep &C, State &S, const Lds &L, int row, b
                     et += L.val[ap];
                     if (ins) am = decide();
                 }
+                wave_sync();   // other lanes' words of L.drop are read
                 // the first later group that loses a member
                 bool hit = false;
                 if (lane > g && lane < stand)
