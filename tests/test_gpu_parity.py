@@ -74,6 +74,49 @@ def test_eval_poses_by_number(n):
     eng.close()
 
 
+@pytest.mark.parametrize('terms', ['fp32', 'ewald'])
+def test_eval_poses_by_number_fp32_terms(terms):
+    """The same for FP32 pair terms, plain and Ewald: a pair's term is the same in
+    either form, so energies agree to the order of an FP64 sum."""
+    s = systems.populated_water()
+    eng = Engine(fp32_coulomb=1 if terms == 'fp32' else 0)
+    eng.add_system(s)
+    if terms == 'ewald':
+        eng.set_ewald(0, 0.34, 1.0)
+    eng.upload()
+    c, p = systems.random_poses(s, 0, 1500, seed=10)
+    E, N, H = eng.eval_poses(0, 0, c, p)
+    for i in range(0, 1500, 500):
+        e, n, h = eng.eval_poses(0, 0, c[i:i + 500], p[i:i + 500])
+        assert np.array_equal(N[i:i + 500], n) and np.array_equal(H[i:i + 500], h)
+        assert (np.abs(E[i:i + 500] - e) <= 1e-10 * np.maximum(np.abs(e), 1.0)).all()
+    eng.close()
+
+
+@pytest.mark.parametrize('excluding', [False, True])
+def test_eval_poses_in_chunks(excluding):
+    """More poses than go to the GPU at once (65,536), with and without excluded
+    molecules, then a small call in the same buffers."""
+    s = systems.populated_water()
+    eng = Engine()
+    eng.add_system(s)
+    eng.upload()
+    c, p = systems.random_poses(s, 0, 256, seed=12)
+    n = 65536 + 321
+    rng = np.random.default_rng(3)
+    q = rng.integers(0, 256, n)
+    first = int(s['frag'][0]['startRes'])
+    ex = np.where(np.arange(256) % 3 == 0, -1, first + np.arange(256) % int(s['frag'][0]['totalNum'])).astype(np.int32)
+    pick = (lambda i: ex[i]) if excluding else (lambda i: None)
+    parts = [eng.eval_poses(0, 0, c[i:i + 64], p[i:i + 64], pick(slice(i, i + 64))) for i in range(0, 256, 64)]
+    ref = [np.concatenate([x[k] for x in parts]) for k in range(3)]
+    for i in (q, q[-70:]):
+        E, N, H = eng.eval_poses(0, 0, c[i], p[i], pick(i))
+        assert np.array_equal(N, ref[1][i]) and np.array_equal(H, ref[2][i])
+        assert (np.abs(E - ref[0][i]) <= 1e-10 * np.maximum(np.abs(ref[0][i]), 1.0)).all()
+    eng.close()
+
+
 def test_water_fixture_on_gpu():
     """The reference's 3-water insertion (test/water/3water.pdb) on the GPU."""
     for ch, lj, key in ((True, False, 'expected_coulomb_kj'), (False, True, 'expected_lj_kj')):
