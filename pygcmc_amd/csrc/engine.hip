@@ -502,7 +502,6 @@ int upload_rep(gcmc_engine *E, HostRep &H)
             const Atom &A = F.atoms[a];
             S.tmpl[a] = make_float4(A.position[0], A.position[1], A.position[2], A.charge);
             S.kq[a] = (float)(KCOUL * (double)A.charge);
-            S.trow[a] = A.type * R.Y;
             S.ttype[a] = A.type;
             if (A.type < 0 || A.type >= R.X)
                 return fail(GCMC_E_ARG, "fragment atom type outside the pair table rows");
@@ -513,8 +512,8 @@ int upload_rep(gcmc_engine *E, HostRep &H)
         std::stable_sort(order, order + S.nf, [&](int a, int b) { return S.ttype[a] < S.ttype[b]; });
         for (int i = 0; i < S.nf; ++i) {
             S.slot[order[i]] = i;
-            S.srow[i] = S.trow[order[i]];
-            if (i == 0 || S.ttype[order[i]] != S.ttype[order[i - 1]]) S.run_row[S.nrun++] = S.trow[order[i]];
+            S.srow[i] = S.ttype[order[i]] * R.Y;
+            if (i == 0 || S.ttype[order[i]] != S.ttype[order[i - 1]]) S.run_row[S.nrun++] = S.srow[i];
             S.run_end[S.nrun - 1] = i + 1;
         }
     }
@@ -846,7 +845,6 @@ void launch_plain(gcmc_engine *E, int nsteps)
 // 115 us at 150 x 150 x 120 points (92 of them hipFFT's six passes), a move of a
 // 300,000-atom slab 50 us, and 46 % of its moves change nothing: 4,096 moves in
 // 462 ms, against 655 ms with the solve after every move.
-template <int NT, bool S>
 void launch_ewald_begin(gcmc_engine *E, int nsteps)
 {
     const int R = (int)E->reps.size();
@@ -886,10 +884,6 @@ struct RunPlain {
 template <int NT, bool S>
 struct RunBatched {
     static void run(gcmc_engine *E, int n) { launch_batched<NT, S>(E, n); }
-};
-template <int NT, bool S>
-struct RunEwaldBegin {
-    static void run(gcmc_engine *E, int n) { launch_ewald_begin<NT, S>(E, n); }
 };
 template <int NT, bool S>
 struct RunEwaldRounds {
@@ -1342,7 +1336,7 @@ int gcmc_engine_run(gcmc_engine *E, int nsteps, int mode)
         // moves this call runs: the most any system has left
         int n = 0;
         for (HostRep *H : E->reps) n = std::max(n, std::min(nsteps, std::max(H->rep.nmoves - H->host_step, 0)));
-        dispatch<RunEwaldBegin>(E, nsteps);
+        launch_ewald_begin(E, nsteps);
         // rounds in chunks, as many as the moves left will take at least at the
         // pace so far (one move per round at worst), then a look at the steps
         double pace = 2.0;   // moves per round

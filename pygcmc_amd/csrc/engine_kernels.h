@@ -312,10 +312,10 @@ __device__ __forceinline__ int wave_scan_max(int x)
 __device__ __forceinline__ int lane_up(int v, int src) { return __builtin_amdgcn_ds_bpermute(src * 4, v); }
 
 // ---- pair energies of a batch of included groups ----------------------------
-// One wave; lane <-> environment atom, two atoms per lane and round, the next
+// One wave; lane <-> environment atom, U atoms per lane and round, the next
 // round's atoms loaded while this one's terms are computed; loop over the
-// fragment atoms held in LDS, ordered by type so that the pair-table entry of
-// a lane's atom is fetched once per type, not once per fragment atom.  A batch's
+// fragment atoms held in LDS, ordered by type so that the pair-table entry of a
+// lane's atom is fetched once per type, not once per fragment atom.  A batch's
 // atoms serve one or two poses ("sets": the old and new pose of a translate or
 // rotate trial); bit s of a group's flags says that it is within the cutoff of
 // pose s's centre.  FP64 terms by default, FP32 terms (fp32_coulomb, Ewald)
@@ -328,7 +328,7 @@ struct EnergyPass {
     float x[2], y[2], z[2];   // centres of the poses (uniform)
     int first, nset;          // poses first .. first + nset - 1
     bool wrap;                // image shift per pair (else per environment atom)
-    int spi, nf;
+    int spi;
     double acc[2];            // this lane's sums
 
     template <class T>
@@ -491,7 +491,7 @@ struct EnergyPass {
     __device__ __forceinline__ void run(CRep &C0, const Lds &L, const WaveLds &W, int g, int A)
     {
         CRep &C = fresh(C0);
-        constexpr int U = 1;
+        constexpr int U = 1;   // (two: 56 vector registers spilled in k_batched instead of 17)
         const int lane = fresh_lane();
         const auto atom = gbl(C.atom);
         const auto atype = gbl(C.atype);
@@ -897,7 +897,6 @@ __device__ __forceinline__ void eval_poses_wave(CRep &C, const Lds &L, const Wav
     P.x[1] = c1[0]; P.y[1] = c1[1]; P.z[1] = c1[2];
     P.wrap = !(pose_near && C.nowrap != 0);
     P.spi = spi;
-    P.nf = nf;
     ScanSums o{};
     // two centres in one scan when the stencil is wide enough for both
     const bool both = nset == 1 || same_centre || C.nst_wide > 0;

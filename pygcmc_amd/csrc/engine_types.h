@@ -18,7 +18,6 @@
 
 namespace gcmc {
 
-constexpr int MAXWAVE = 16;          // waves of the largest workgroup (1024 threads)
 constexpr int MAXT = 32;             // species per system
 constexpr int MAXF = 20;             // atoms per fragment (AtomArray.atoms[20])
 constexpr int MAXK = 2048;           // trials per move (confBias)
@@ -47,7 +46,6 @@ struct Species {
     double B;              // beta*muex + ln(L0 L1 L2 conc 6.023e-4)
     float4 tmpl[MAXF];     // centred template (x, y, z, charge)
     float kq[MAXF];        // 1388.431112 * charge, rounded once
-    int trow[MAXF];        // type * Y: row of the pair table
     int ttype[MAXF];       // type
     // atoms ordered by type: place of each atom, row of the pair table per place,
     // and the runs of equal type (end place, row)

@@ -65,9 +65,9 @@ struct Spline3 {
 __device__ inline Spline3 splines(const float4 a, const Geo &g)
 {
     Spline3 s;
-    spline4(scaled(a.x, g.L[0], g.K[0]), g.K[0], s.f[0], s.w[0]);
-    spline4(scaled(a.y, g.L[1], g.K[1]), g.K[1], s.f[1], s.w[1]);
-    spline4(scaled(a.z, g.L[2], g.K[2]), g.K[2], s.f[2], s.w[2]);
+    spline4(scaled(a.x, g.L[0], g.K[0]), s.f[0], s.w[0]);
+    spline4(scaled(a.y, g.L[1], g.K[1]), s.f[1], s.w[1]);
+    spline4(scaled(a.z, g.L[2], g.K[2]), s.f[2], s.w[2]);
     return s;
 }
 

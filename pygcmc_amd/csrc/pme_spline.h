@@ -29,7 +29,7 @@ __device__ inline int base4(float u, float &t)
 }
 
 // weights of the 4 grid points f, f-1, f-2, f-3 of scaled coordinate u in [0, K)
-__device__ inline void spline4(float u, int, int &f, float w[4])
+__device__ inline void spline4(float u, int &f, float w[4])
 {
     float t;
     f = base4(u, t);
@@ -45,37 +45,6 @@ __device__ inline float scaled(float x, float L, int K)
     return u >= (float)K ? 0.0f : u;
 }
 
-// interpolated potential of grid Phi [K0][K1][K2] at (x, y, z)
-__device__ inline float gather(const float *Phi, const int K[3], const float L[3], float x, float y, float z)
-{
-    int f0, f1, f2;
-    float w0[4], w1[4], w2[4];
-    spline4(scaled(x, L[0], K[0]), K[0], f0, w0);
-    spline4(scaled(y, L[1], K[1]), K[1], f1, w1);
-    spline4(scaled(z, L[2], K[2]), K[2], f2, w2);
-    float s = 0.0f;
-#pragma unroll
-    for (int i0 = 0; i0 < 4; ++i0) {
-        int k0 = f0 - i0;
-        k0 += k0 < 0 ? K[0] : 0;
-#pragma unroll
-        for (int i1 = 0; i1 < 4; ++i1) {
-            int k1 = f1 - i1;
-            k1 += k1 < 0 ? K[1] : 0;
-            const float *row = Phi + ((size_t)k0 * K[1] + k1) * K[2];
-            float r = 0.0f;
-#pragma unroll
-            for (int i2 = 0; i2 < 4; ++i2) {
-                int k2 = f2 - i2;
-                k2 += k2 < 0 ? K[2] : 0;
-                r = fmaf(w2[i2], row[k2], r);
-            }
-            s = fmaf(w0[i0] * w1[i1], r, s);
-        }
-    }
-    return s;
-}
-
 // element i of a 4-vector held in registers (no indexed registers)
 __device__ inline float pick4(const float w[4], int i)
 {
@@ -83,15 +52,16 @@ __device__ inline float pick4(const float w[4], int i)
     return (i & 2) ? b : a;
 }
 
-// gather() by 16 lanes (sub = lane & 15), each one z row of the 4 x 4; the rows
-// are added in gather()'s order, so every lane has its value bit for bit
+// interpolated potential of grid Phi [K0][K1][K2] at (x, y, z) by 16 lanes (sub =
+// lane & 15), each one z row of the 4 x 4; the rows are added in order, so every
+// lane has the same value
 __device__ inline float gather16(const float *Phi, const int K[3], const float L[3], float x, float y, float z, int sub)
 {
     int f0, f1, f2;
     float w0[4], w1[4], w2[4];
-    spline4(scaled(x, L[0], K[0]), K[0], f0, w0);
-    spline4(scaled(y, L[1], K[1]), K[1], f1, w1);
-    spline4(scaled(z, L[2], K[2]), K[2], f2, w2);
+    spline4(scaled(x, L[0], K[0]), f0, w0);
+    spline4(scaled(y, L[1], K[1]), f1, w1);
+    spline4(scaled(z, L[2], K[2]), f2, w2);
     int k0 = f0 - (sub >> 2), k1 = f1 - (sub & 3);
     k0 += k0 < 0 ? K[0] : 0;
     k1 += k1 < 0 ? K[1] : 0;
@@ -132,8 +102,8 @@ __device__ inline float pair_kernel_slab(const float *Gk, const int K[3], const 
     for (int a = 0; a < 3; ++a) {
         int fx, fy;
         float wx[4], wy[4];
-        spline4(scaled(x[a], L[a], K[a]), K[a], fx, wx);
-        spline4(scaled(y[a], L[a], K[a]), K[a], fy, wy);
+        spline4(scaled(x[a], L[a], K[a]), fx, wx);
+        spline4(scaled(y[a], L[a], K[a]), fy, wy);
         df[a] = fx - fy;
 #pragma unroll
         for (int j = 0; j < 7; ++j) c[a][j] = 0.0f;
