@@ -199,10 +199,14 @@ int gcmc_engine_set_trace(gcmc_engine *e, int replica, int max_steps, int max_k)
 int gcmc_engine_get_trace(gcmc_engine *e, int replica, gcmc_trace *out);
 
 /* ---- single evaluations ---------------------------------------------------
- * Energies (kJ/mol, FP32 pair terms, compensated sums, FP64 result) of npose
- * poses of one species against the replica's current state, each tested
- * around centres[i] and excluding residue exclude[i] (-1: none).  The same
- * kernel path as the MC step (calcEnergy, gcmc/cpp/gcmc_energy.h:142-204). */
+ * Energies (kJ/mol; pair terms in FP64, or in FP32 with fp32_coulomb or Ewald;
+ * sums in FP64) of npose poses of one species against the replica's current
+ * state, each tested around centres[i] and excluding residue exclude[i] (-1:
+ * none).  The same kernel path as the MC step (calcEnergy,
+ * gcmc/cpp/gcmc_energy.h:142-204).  In calls of fewer than 1,024 poses four
+ * waves share a pose, in larger ones a pose is one wave's: the order of a
+ * pose's FP64 sum, and so the energy's last bits, depend on which it is, and on
+ * nothing else.  Groups and hashes are the same. */
 int gcmc_engine_eval_poses(gcmc_engine *e, int replica, int species, int npose,
                            const float *centres, const float *poses, const int *exclude,
                            double *energy, int *ninc, uint32_t *inchash);
@@ -227,8 +231,11 @@ int gcmc_engine_occupancy(gcmc_engine *e, int replica, int species, const double
  * pair by the rule of gcmc/python/simulation.py:63-72.  Writes energy[i]
  * (kJ/mol), dEdx[i][f][3] = dE_i/dx_f (kJ/mol/A) and partial[i][3][Y] =
  * dE_i/d(dq, eps_kcal, rmin_half).  All pointers are DEVICE pointers;
- * poses [npose][nf][3], centres [npose][3].  Work is queued on `stream`
- * (a hipStream_t; NULL = the default stream) and not waited for. */
+ * poses [npose][nf][3], centres [npose][3].  In calls of fewer than 2,048 poses
+ * four waves share a pose, in larger ones a pose is one wave's (when four poses'
+ * type sums fit in LDS): the order of the sums, and so a pose's last bits,
+ * depend on that.  Work is queued on `stream` (a hipStream_t; NULL = the default
+ * stream) and not waited for. */
 int gcmc_engine_adjoint(gcmc_engine *e, int replica, int species, int npose,
                         const float *centres, const float *poses, const float *eps_kcal,
                         const float *rmin_half, const float *dq, double *energy, float *dEdx,
@@ -267,11 +274,14 @@ int gcmc_adjoint_backward_noalloc(int npose, int per_pose, int ncol, const float
  * Its trial energies then use K q q' erfc(beta r)/r in the group-cutoff pair
  * terms plus the reciprocal interaction sum_f q_f phi(x_f) with the PME
  * potential phi of the current state (the moving molecule's own share
- * removed), and the potential is updated after every move.  In the batched
- * and graph forms an engine's systems are either all Ewald systems or none:
- * Ewald systems then run move by move (each move's trials in one launch,
- * accept, PME update), the graph form replaying a captured chunk of moves;
- * the chains equal the plain form's.  The reference ignores InfoStruct.PME, and so
+ * removed), and the potential is current for every move's evaluations.  In the
+ * batched and graph forms an engine's systems are either all Ewald systems or
+ * none.  Ewald systems then run in rounds: every system goes on to the end of a
+ * move that changed its charges, then the changes enter the grids and the
+ * potentials are solved anew; the host looks at the systems' steps between
+ * chunks of rounds (gcmc_engine_run waits for them), and the graph form replays
+ * a captured chunk of eight.  The chains equal the plain form's, which solves
+ * after every move.  The reference ignores InfoStruct.PME, and so
  * do runGCMC_hip and gcmc_engine_add_system.  eval_poses adds the same
  * reciprocal term; its exclude[i], when a molecule of the evaluated species,
  * must be one present in the state. */

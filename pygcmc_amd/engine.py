@@ -316,7 +316,9 @@ class Engine:
         return out
 
     def eval_poses(self, r, species, centres, poses, exclude=None):
-        """FP32/compensated energies of poses [n, nf, 3] around centres [n, 3]."""
+        """Energies (kJ/mol, float64), included groups and their hashes of poses
+        [n, nf, 3] around centres [n, 3].  The last bits of an energy depend on
+        whether the call has at least 1,024 poses (order of the FP64 sum)."""
         c = np.ascontiguousarray(centres, np.float32)
         p = np.ascontiguousarray(poses, np.float32)
         n = len(c)
