@@ -26,6 +26,9 @@
 // shorter sums had been 6e-7 off), the charge derivatives' from batch to batch in
 // FP64 (2,100 poses of nine species, five systems each: 1.30e-7 off 64 bits in the
 // geometric mean, 1.51e-7 with one FP32 sum per lane and pose; no time).
+// Bound by issue at low residency: the registers hold six sums per fragment atom,
+// 116 in all for up to 4 atoms (four waves per SIMD), 161 for 8 (three), 205 for 12
+// (two), 256 for 20 (one).
 #pragma once
 
 #include "engine_kernels.h"

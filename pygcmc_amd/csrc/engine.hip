@@ -143,7 +143,7 @@ int pme_spread_counted(gcmc_pme *p, int cap, const int *count, const float4 *xyz
 
 // Buffers of an engine for given poses (inputs, then results), kept from call to
 // call.  A few poses (POSE_DIRECT) stay in pinned memory, where the kernel itself
-// reads the inputs and writes the results: 201 methanol poses take 37 us, 118 with
+// reads the inputs and writes the results: 201 methanol poses take 32 us, 126 with
 // buffers allocated per call and six copies.  More go to device memory, at most
 // POSE_CHUNK at a time.
 constexpr int POSE_CHUNK = 65536;
@@ -359,7 +359,12 @@ std::vector<int> make_stencil(const float L[3], const int nc[3], float rc, float
 
 // Translations of at most this much (grid_dx, A) evaluate the old and the new
 // pose in one scan of a stencil wide enough for both centres; the wider ones
-// scan twice (the union of two distant neighbourhoods would be scanned for each).
+// scan twice.  The union of the neighbourhoods, each group tested against both
+// centres, grows with the distance: us per move of 64 systems' moves of up to 128
+// trials, one scan / two, 136 / 172 at 1 A, 139 / 171 at 2, 142 / 170 at 3, 146 / 169
+// at 4 (one system, one trial: 14.5 / 18.1, 14.0 / 17.4, 14.1 / 17.2, 14.2 / 17.1).
+// One scan would still be the faster at 4 A; the line lies above the steps in use
+// (a grid's edge, 1 A).
 constexpr float WIDE_DX = 2.0f;
 // The stencil reaches further towards positive offsets only: negative steps scan
 // twice.
@@ -893,7 +898,12 @@ struct RunEwaldRounds {
 // with benzene poses: 38 against 42 us at 700, 47 against 42 at 1,024, 70 against
 // 52 at 2,000).
 constexpr int POSE_WAVES = 1024;
-constexpr int ADJ_WAVES = 2048;   // the same for gradients
+// The same for gradients, us forward, shared / one wave: 64 poses 13 / 27 (water,
+// 3 atoms) and 25 / 54 (benzene, 12), 1,024 19 / 28 and 55 / 60, 1,536 33 / 31 and
+// 103 / 68, 2,048 33 / 30 and 102 / 67, 4,096 60 / 54 and 193 / 129.  The sides meet
+// a little above 1,024 poses, where the shared form's workgroups no longer run all at
+// once.
+constexpr int ADJ_WAVES = 2048;
 
 // The adjoint's backward: poses are summed in chunks of 64 to ADJ_CHUNKS chunks,
 // work holding ADJ_CHUNKS x ncol sums.

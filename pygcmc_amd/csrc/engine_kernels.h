@@ -54,7 +54,8 @@ using CSpecies = const Species;
 #endif
 // The same Rep behind an address the compiler cannot relate to C: fields read
 // through it are loaded where they are used (scalar loads), instead of all at
-// once ahead of the loops, which spilled a hundred scalars into vector registers.
+// once ahead of the loops: k_batched (256 threads, FP64 terms) then spills 323
+// scalar and 26 vector registers, 190 and 17 this way.
 __device__ __forceinline__ CRep &fresh(CRep &C)
 {
     CRep *p = &C;
@@ -572,8 +573,8 @@ __device__ inline void stage_tables(CRep &C, const Lds &L, bool rep, bool tab)
 
 // The FP32 group test (within, gcmc_math.h) of a wave's lanes at once: without
 // branches when no lane is past the shift table (one ballot), else literally.
-// Nested branches per axis kept a dozen execution masks alive and spilled the
-// scalar registers.
+// (3,000 moves of one system take 79.5 ms, 80.9 with branches per axis, of 64
+// systems 123-127 and 129; k_batched spills 190 scalar registers both ways.)
 struct GroupCut {
     AxisCut ax[3];
     float r2max;
@@ -1014,7 +1015,12 @@ __device__ inline double ewald_recip(CRep &C, CSpecies &F, const WaveLds &W, int
 // A move of at most COOP_TRIALS trials is on its replica's critical path: its
 // trials' cells are shared by four waves.  In larger moves every trial is one
 // wave's.  The rule depends on the move alone: every form sums a pose's energy in
-// the same order.
+// the same order.  Sharing pays where waves would idle and costs where none do, so
+// the line is a compromise between few systems and many.  us per move of a water
+// chain among 8,000 atoms, shared / not: one system 11.9 / 18.5 at one trial,
+// 40 / 48 at 64, 55 / 59 at 100, 75 / 79 at 200, 104 / 103 at 400; eight systems
+// 46 / 54, 66 / 64, 85 / 84 and 134 / 134 at 64, 100, 200 and 400; 64 systems
+// 15 / 21, 47 / 44, 60 / 57, 81 / 74 and 148 / 100 at 1, 32, 64, 100 and 200.
 constexpr int COOP_TRIALS = 100, COOP = 4;
 
 struct Move {
@@ -1361,7 +1367,9 @@ __device__ inline double key_value(unsigned long long k)
 // An accepted pick drops its neighbours from the later groups: the groups before
 // the first one that loses a member stand, the next batch starts there.  Batches
 // grow from 8 to SEL_GROUPS groups while all of them stand and shrink to the pace
-// at which they do not.
+// at which they do not (insertions of eight fragments, 10 to 400 trials each, into
+// 20,000 atoms: 34.0 us per move, 35.2 in batches of 8 throughout; 36.2 on another
+// machine, 37.4 in batches of 64).
 // (One wave taking the groups one after another, weights included, spent
 // 1.3 us on each.)
 template <int NT>
