@@ -4,9 +4,8 @@ Workload: 64 independent GCMC systems whose fixed-atom counts are
 log-uniform in 5,000-60,000 (box 40*(N/2000)^(1/3) A, fixed-atom density of the
 2,000-atom sphere system), each with its own seed and muex and the 8 rigid
 fragment types + TIP3P water (confBias 400/15/10/20/15/300/100/200/2), 10,000
-moves each, FP32 pair energies with compensated sums (Coulomb terms from the
-exactly formed FP32 displacement in FP64), FP64 totals and acceptance, all
-systems in one persistent kernel.  Synthetic data (seeded).
+moves each, FP64 pair terms from FP32 positions, FP64 totals and acceptance,
+all systems in one persistent kernel.  Synthetic data (seeded).
 
 One bench step is one whole pass of that workload: every system returned to
 its initial state on the device (device-to-device copies from a snapshot
@@ -351,8 +350,8 @@ def ewald_bench(moves, warm=32):
     """The 300,000-atom slab (150 x 150 x 120 A, 15 A pore, water +
     methylammonium / acetate, PME 1 A grid, beta 0.34 /A, 12 A cutoff) in
     Ewald mode: `moves` moves after `warm` untimed ones, in the plain form
-    (launches issued move by move) and the graph form (captured 32-move
-    chunks replayed); both compute the same chain."""
+    (launches issued move by move) and the graph form (captured chunks of
+    rounds replayed); both compute the same chain."""
     from pygcmc_amd import synth
     from pygcmc_amd.engine import Engine
     s = synth.slab(mcsteps=50000)
@@ -556,7 +555,7 @@ def main():
         'scaling': 'weak',
         'vs_baseline': None,
         'dtype': 'fp64 (pair terms from fp32 positions, 1/r an fp32 estimate refined by one fp64 Newton step; '
-                 'fp64 sums and acceptance)' if not args.fp32_coulomb else 'fp32 pair terms, compensated sums; '
+                 'fp64 sums and acceptance)' if not args.fp32_coulomb else 'fp32 pair terms; '
                                                                           'fp64 sums and acceptance',
         'data': 'synthetic (seeded)',
         'config': {'workload': f'{R} uneven GCMC replicas (5k-60k fixed atoms, 8 fragments + water), '
